@@ -163,12 +163,19 @@ def _slots_of(table, lo, hi):
 
 def _seed_weights(module, g):
     """N(0, 0.02) matrices, conv taps and an embedding on the scale of what they meet; norm gains and the Polar
-    priors as the module sets them."""
+    priors as the module sets them.  Each KV group's queries and key share a direction, so that a sequence's first
+    token, which reads only its own write, reads more than the rounding of a product near zero (the memory's
+    readout is normed: of a near-zero one the direction is undefined in any precision)."""
     with torch.no_grad():
         for name, p in module.named_parameters():
             if p.dim() > 1 or name.endswith("bias"):
                 std = 0.3 if "canon" in name or "conv." in name else 0.5 if name == "embed.weight" else 0.02
                 p.copy_(_randn(g, *p.shape, std=std))
+        for m in module.modules():
+            if isinstance(m, PolarAttention):
+                shared = _randn(g, m.num_kv_heads, 1, m.head_dim, std=0.5)
+                m.k.bias.copy_(shared.view(-1))
+                m.q.bias.view(m.num_kv_heads, -1, 2 * m.head_dim)[..., :m.head_dim] = shared
     return module
 
 
@@ -284,6 +291,14 @@ def prepare(case, seed):
 
 
 # ------------------------------------------------------------------ one pass
+def _gradients(grads):
+    """The large gradients as they are and the small ones (biases, gains, taps, the Polar parameters) in one flat
+    buffer, as an optimiser holds them: eight values that are small differences of large sums have no precision of
+    their own to compare."""
+    return dict(grads=[t for t in grads if t.numel() > 16384],
+                small=torch.cat([t.flatten() for t in grads if t.numel() <= 16384]))
+
+
 def run(s):
     case = s["case"]
     kind = case["kind"]
@@ -307,11 +322,11 @@ def run(s):
         c, mag = polar_attention(s["q"], s["k"], s["v"], s["n_keys"], window=window, **s["params"])
         wrt = [s["q"], s["k"], s["v"]] + [s["params"][n] for n in POLAR]
         grads = torch.autograd.grad([c, mag], wrt, [s["gc"], s["gm"]])
-        return dict(c=c.detach(), mag=mag.detach(), grads=grads)
+        return dict(c=c.detach(), mag=mag.detach(), **_gradients(grads))
     if kind == "train_block":
         y = s["layer"](s["x"])
         grads = torch.autograd.grad(y, [s["x"]] + list(s["layer"].parameters()), s["go"])
-        return dict(y=y.detach(), grads=grads)
+        return dict(y=y.detach(), **_gradients(grads))
     with torch.no_grad():
         if kind in ("forward", "block"):
             return s["layer"](s["x"])
@@ -391,11 +406,10 @@ def work(case):
 
 def tolerance(case):
     # three to four times the distance from ``exact`` measured for each kind (the 16-bit ops 0.2-0.4%, a layer
-    # 0.75%, the fp32 block 7e-7), no more than 3%: a block's gradients, the attention's length-gain gradient
-    # (a small difference of large sums) and the four-block model measure 1.5 to 2%
+    # 0.85%, the fp32 block 7e-7), no more than 3%: a block's gradients and the four-block model measure 1.2 to 1.7%
     return {"decode": {"rel": 1e-2}, "memory": {"rel": 1.5e-2}, "forward": {"rel": 2.5e-2},
             "prefill": {"rel": 2.5e-2}, "continue": {"rel": 2.5e-2}, "block": {"rel": 1e-5},
-            "train_polar": {"rel": 3e-2}, "train_memory": {"rel": 1.5e-2}, "train_block": {"rel": 3e-2},
+            "train_polar": {"rel": 1.5e-2}, "train_memory": {"rel": 1.5e-2}, "train_block": {"rel": 3e-2},
             "serve_prefill": {"rel": 3e-2}, "serve_decode": {"rel": 3e-2}}[case["kind"]]
 
 
@@ -576,7 +590,7 @@ def exact(case, seed):
             ps = {n: s["params"][n].detach().double().requires_grad_(True) for n in POLAR}
             c, mag = _attend64(*ins, ps, case["window"])
             grads = torch.autograd.grad([c, mag], ins + [ps[n] for n in POLAR], [s["gc"].double(), s["gm"].double()])
-            return dict(c=c.detach(), mag=mag.detach(), grads=grads)
+            return dict(c=c.detach(), mag=mag.detach(), **_gradients(grads))
         if kind in ("block", "train_block"):
             w = _weights64(s["layer"])
             x = s["x"].detach().double()
@@ -585,7 +599,7 @@ def exact(case, seed):
             for t in (x, *w.values()):
                 t.requires_grad_(True)
             y = _block64(w, x, case)
-            return dict(y=y.detach(), grads=torch.autograd.grad(y, [x, *w.values()], s["go"].double()))
+            return dict(y=y.detach(), **_gradients(torch.autograd.grad(y, [x, *w.values()], s["go"].double())))
         if kind == "forward":
             return _mixer64(_weights64(s["layer"]), s["x"].double(), case)[0]
         if kind in ("prefill", "continue"):

@@ -84,6 +84,9 @@ SIGNATURES = {
                                 _p, _i64, _i64, _i64, _i64, _f32, _i32, _p]),
     "atma_lfm2_conv_packed": (_i32, [_p, _i64, _p, _i64, _p, _i64, _p, _i64, _i64, _p, _p, _p, _i64, _i64,
                                      _i32, _p]),
+    "atma_canon_qkv": (_i32, [_p] * 10 + [_i64] * 3 + [_p] * 4 + [_i64, _i32, _p, _i64, _i64, _i64, _f32, _i32, _i32, _p]),
+    "atma_canon_bwd_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64]),
+    "atma_canon_bwd": (_i32, [_p] * 6 + [_i64] * 4 + [_i32, _i32, _p, _sz, _p]),
     "atma_packed_causal_conv1d": (_i32, [
         _p, _i64, _i64, _p, _i64, _i64, _p, _p, _i64, _i64, _i64, _i64, _p, _p, _p, _i64, _i64, _i64,
         _i32, _i32, _p]),

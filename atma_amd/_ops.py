@@ -769,3 +769,70 @@ def store_kvcache_op(key: Tensor, value: Tensor, k_cache: Tensor, v_cache: Tenso
 @store_kvcache_op.register_fake
 def _(key, value, k_cache, v_cache, slot_mapping):
     return None
+
+
+# --------------------------------------------------------------------------- Canon convs (training)
+def _canon_check(xs, ws):
+    _need_cuda(*xs, *ws)
+    B, T, _ = xs[0].shape
+    for x, w in zip(xs, ws):
+        if x.dim() != 3 or x.shape[:2] != (B, T) or x.dtype != xs[0].dtype or not x.is_contiguous() \
+                or w.dim() != 3 or w.shape[0] != x.shape[2] or w.shape[1] != 1 or w.shape[2] != ws[0].shape[2]:
+            raise ValueError("canon_conv: contiguous rows (B, T, C) in one dtype and conv weights (C, 1, K)")
+
+
+@torch.library.custom_op("atma_hip::canon_conv", mutates_args=())
+def canon_conv_op(xs: List[Tensor], ws: List[Tensor]) -> List[Tensor]:
+    from .kernel.canon import _L3, _I3, _P3, _taps
+    _canon_check(xs, ws)
+    xs = [_rows16(x) for x in xs]
+    taps, wdt = _taps(ws, xs[0].dtype)
+    B, T, _ = xs[0].shape
+    K, C = taps[0].shape[-1], [x.shape[2] for x in xs]
+    d = 128 if all(c % 128 == 0 for c in C) else 64
+    outs = [torch.empty_like(x) for x in xs]
+    if B * T == 0:
+        return outs
+    rc = _lib.load().atma_canon_qkv(
+        _P3(*[x.data_ptr() for x in xs]), _L3(*C), _L3(d, d, d), _L3(*[c // d for c in C]), _I3(0, 0, 0),
+        _P3(*[w.data_ptr() for w in taps]), _P3(*[o.data_ptr() for o in outs]), None, None, None, len(xs), B * T, T,
+        None, None, None, None, 0, 0, None, 0, K, d, 0.0, _lib.dtype_code(wdt), _lib.dtype_code(xs[0].dtype),
+        _lib.stream_handle(xs[0].device))
+    _lib.check(rc, "canon_conv")
+    return outs
+
+
+@canon_conv_op.register_fake
+def _(xs, ws):
+    return [torch.empty_like(x) for x in xs]
+
+
+@torch.library.custom_op("atma_hip::canon_conv_bwd", mutates_args=())
+def canon_conv_bwd_op(gs: List[Tensor], xs: List[Tensor], ws: List[Tensor]) -> List[Tensor]:
+    """dx of every stream, then every weight's gradient (its weight's dtype)."""
+    from .kernel.canon import _L3, _P3, _taps
+    _canon_check(xs, ws)
+    _canon_check(gs, ws)
+    gs, xs = [_rows16(g) for g in gs], [_rows16(x) for x in xs]
+    taps, wdt = _taps(ws, xs[0].dtype)
+    B, T, _ = xs[0].shape
+    K, C = taps[0].shape[-1], [x.shape[2] for x in xs]
+    dev = xs[0].device
+    dx = [torch.empty_like(x) for x in xs]
+    dw = [torch.empty(w.shape, device=dev, dtype=wdt) for w in ws]
+    if B * T == 0:
+        return dx + [torch.zeros_like(w) for w in ws]
+    lib = _lib.load()
+    ws_bytes = lib.atma_canon_bwd_workspace_bytes(B * T, T, sum(C), K)
+    buf = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
+    rc = lib.atma_canon_bwd(
+        _P3(*[g.data_ptr() for g in gs]), _P3(*[x.data_ptr() for x in xs]), _P3(*[w.data_ptr() for w in taps]),
+        _P3(*[t.data_ptr() for t in dx]), _P3(*[t.data_ptr() for t in dw]), _L3(*C), len(xs), B * T, T, K,
+        _lib.dtype_code(wdt), _lib.dtype_code(xs[0].dtype), buf.data_ptr(), ws_bytes, _lib.stream_handle(dev))
+    _lib.check(rc, "canon_conv_bwd")
+    return dx + [g.to(w.dtype) for g, w in zip(dw, ws)]
+
+
+@canon_conv_bwd_op.register_fake
+def _(gs, xs, ws):
+    return [torch.empty_like(x) for x in xs] + [torch.empty_like(w) for w in ws]

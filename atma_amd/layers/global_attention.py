@@ -41,6 +41,7 @@ from ..kernel import (StartSignal, causal_conv1d_decode_step, chunk_gated_delta_
                       gated_delta_decode_step, gated_delta_gates, global_decode_step, polar_attention,
                       polar_attention_decode, polar_attention_fwd, polar_attention_packed_fwd,
                       recurrence_pays_to_overlap)
+from ..kernel.canon import canon_conv, canon_qkv, canon_supported
 from ..kernel.decode_fusions import (PartialSums, chunk_width, global_decode_gate, global_decode_prep,
                                      linear_tokens_chunks, linear_tokens_gated, linear_tokens_multi,
                                      linear_tokens_multi_supported,
@@ -246,6 +247,42 @@ class PolarAttention(nn.Module):
             return head_rms_norm(q, F32_EPS), gate, head_rms_norm(k, F32_EPS), v
         return F.rms_norm(q, (dk,)), gate, F.rms_norm(k, (dk,)), v
 
+    def _project_canon(self, x, B, T, cache=None, slots=None, slot_mapping=None, continuing=False, token_maps=None):
+        """The projections, per-head norms and residual Canon convs of B sequences of T rows (or of the rows
+        ``token_maps`` packs), x flattening to (B T, dim): q (B T, H, dk), gate (a view of the q|gate projection), k, v
+        (B T, Hkv, dk).  With ``cache`` the conv tails of the sequences' table rows are stored (and read first when
+        ``continuing``) and k / v written to the pages.  Inference at the shapes ``canon_qkv`` serves makes one launch
+        of everything after the projections; training makes the convs one differentiable call (``canon_conv``)."""
+        H, Hkv, dk, rows = self.num_heads, self.num_kv_heads, self.head_dim, B * T
+        convs = (self.canon_q, self.canon_k, self.canon_v)
+        served = canon_supported(x, dk, self.kernel_size)
+        tables = None if cache is None else (cache.conv_q, cache.conv_k, cache.conv_v)
+        if cache is not None:
+            served = served and all(t.dtype == x.dtype and t.is_contiguous()
+                                    for t in (*tables, cache.k_cache, cache.v_cache))
+        if served and not torch.is_grad_enabled():
+            qg = self.q(x).view(rows, H, 2 * dk)
+            q, k, v = canon_qkv(qg[..., :dk], self.k(x).view(rows, Hkv, dk), self.v(x).view(rows, Hkv, dk),
+                                [c.weight for c in convs], F32_EPS, seq_len=T, token_maps=token_maps, tails=tables,
+                                slots=slots, continuing=continuing, slot_mapping=slot_mapping,
+                                caches=None if cache is None else (cache.k_cache, cache.v_cache))
+            return q, qg[..., dk:], k, v
+        q, gate, k, v = self._project(x)
+        if served and cache is None:
+            q, k, v = canon_conv(q.reshape(B, T, H * dk), k.reshape(B, T, Hkv * dk), v.reshape(B, T, Hkv * dk),
+                                 *[c.weight for c in convs])
+        elif cache is None or continuing:
+            q, k, v = (self._conv_prefill(t.reshape(B, T, h * dk), c, t_, slots, continuing) for t, h, c, t_ in
+                       zip((q, k, v), (H, Hkv, Hkv), convs, tables or (None,) * 3))
+        else:
+            maps = token_maps if token_maps is not None else self.dense_token_maps(B, T, slots)
+            q, k, v = (self._conv_packed(t.reshape(rows, h * dk), c, t_, maps) for t, h, c, t_ in
+                       zip((q, k, v), (H, Hkv, Hkv), convs, tables))
+        q, k, v = q.reshape(rows, H, dk), k.reshape(rows, Hkv, dk), v.reshape(rows, Hkv, dk)
+        if cache is not None:
+            store_kvcache(k, v, cache.k_cache, cache.v_cache, slot_mapping)
+        return q, gate.reshape(rows, H, dk), k, v
+
     @staticmethod
     def _conv_prefill(t, conv, tails=None, slots=None, continuing=False):
         """Residual causal depthwise conv over (B, T, C); optionally stores the last K-1
@@ -357,11 +394,7 @@ class PolarAttention(nn.Module):
     def forward(self, x):
         """Causal full-sequence mixer (``model/reference.py:127-195``): x (B, T, dim)."""
         B, T, _ = x.shape
-        H, Hkv, dk = self.num_heads, self.num_kv_heads, self.head_dim
-        q, gate, k, v = self._project(x)
-        q = self._conv_prefill(q.reshape(B, T, H * dk), self.canon_q).view(B, T, H, dk)
-        k = self._conv_prefill(k.reshape(B, T, Hkv * dk), self.canon_k).view(B, T, Hkv, dk)
-        v = self._conv_prefill(v.reshape(B, T, Hkv * dk), self.canon_v).view(B, T, Hkv, dk)
+        q, gate, k, v = (t.unflatten(0, (B, T)) for t in self._project_canon(x, B, T))
         return self._attend_prefill(x, q, gate, k, v, None, None)
 
     def _attend_prefill(self, x, q, gate, k, v, S0, final_sink, defer=False):
@@ -405,13 +438,8 @@ class PolarAttention(nn.Module):
         slot_mapping: (B*T,) int32 cache slots of every token (-1 = skip)."""
         B, T, _ = x.shape
         H, Hkv, dk = self.num_heads, self.num_kv_heads, self.head_dim
-        q, gate, k, v = self._project(x)
-        maps = self.dense_token_maps(B, T, slots)
-        q = self._conv_packed(q.reshape(B * T, H * dk), self.canon_q, cache.conv_q, maps).view(B, T, H, dk)
-        k = self._conv_packed(k.reshape(B * T, Hkv * dk), self.canon_k, cache.conv_k, maps).view(B, T, Hkv, dk)
-        v = self._conv_packed(v.reshape(B * T, Hkv * dk), self.canon_v, cache.conv_v, maps).view(B, T, Hkv, dk)
-        store_kvcache(k.reshape(B * T, Hkv, dk), v.reshape(B * T, Hkv, dk), cache.k_cache, cache.v_cache,
-                      slot_mapping)
+        q, gate, k, v = (t.unflatten(0, (B, T)) for t in
+                         self._project_canon(x, B, T, cache, slots, slot_mapping))
         S0 = cache.mem_table[slots] if self.mem is not None else None
 
         def sink(S):
@@ -433,13 +461,7 @@ class PolarAttention(nn.Module):
         (token_seq_starts, token_seq_ends, token_seq_slots) int32 (one entry per token)."""
         total = x.shape[0]
         H, Hkv, dk = self.num_heads, self.num_kv_heads, self.head_dim
-        q, gate, k, v = self._project(x)
-        q = self._conv_packed(q.reshape(total, H * dk), self.canon_q, cache.conv_q, token_maps).view(total, H, dk)
-        k = self._conv_packed(k.reshape(total, Hkv * dk), self.canon_k, cache.conv_k, token_maps).view(
-            total, Hkv, dk)
-        v = self._conv_packed(v.reshape(total, Hkv * dk), self.canon_v, cache.conv_v, token_maps).view(
-            total, Hkv, dk)
-        store_kvcache(k, v, cache.k_cache, cache.v_cache, slot_mapping)
+        q, gate, k, v = self._project_canon(x, 1, total, cache, slots, slot_mapping, token_maps=token_maps)
         c, mag = polar_attention_packed_fwd(q, k, v, *tile_maps, window=self.window, **self.polar_params())
         if self._glue_fusable(x):
             rs, start = [], 0
@@ -480,14 +502,8 @@ class PolarAttention(nn.Module):
         B, T, _ = x.shape
         H, Hkv, dk = self.num_heads, self.num_kv_heads, self.head_dim
         cached = [int(c) for c in cached]
-        q, gate, k, v = self._project(x)
-        q = self._conv_prefill(q.reshape(B, T, H * dk), self.canon_q, cache.conv_q, slots, True).view(B, T, H, dk)
-        k = self._conv_prefill(k.reshape(B, T, Hkv * dk), self.canon_k, cache.conv_k, slots, True).view(
-            B, T, Hkv, dk)
-        v = self._conv_prefill(v.reshape(B, T, Hkv * dk), self.canon_v, cache.conv_v, slots, True).view(
-            B, T, Hkv, dk)
-        store_kvcache(k.reshape(B * T, Hkv, dk), v.reshape(B * T, Hkv, dk), cache.k_cache, cache.v_cache,
-                      slot_mapping)
+        q, gate, k, v = (t.unflatten(0, (B, T)) for t in
+                         self._project_canon(x, B, T, cache, slots, slot_mapping, continuing=True))
         page = cache.k_cache.shape[1]
         cs, ms = [], []
         for b in range(B):

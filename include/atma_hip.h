@@ -649,6 +649,36 @@ int atma_lfm2_conv_packed(const void* bcx, int64_t ld, const void* weight, int64
                           const int32_t* token_seq_ends, const int32_t* token_seq_slots, int64_t total, int64_t D,
                           int dtype, void* stream);
 
+/*
+ * The Canon step of the global layer over whole rows (model/reference.py:136-155; the engine's tails
+ * inference/models/atma.py:102-162), no reference counterpart as one call.  n streams (1..3; arrays of n): stream i
+ * has rows of heads[i] heads, element (row, h, e) of x[i] at row ldr[i] + h ldh[i] + e; with xn = norm[i] ?
+ * rms_norm(x) per head (eps) rounded to dtype : x,
+ *   out[i][row] = xn[row] + sum_j w[i][c, j] xn[row - (K - 1) + j]     ((rows, heads d) contiguous; w (heads d, K))
+ * within the row's sequence.  T > 0: rows / T sequences of T rows; T 0: packed rows with the token maps of
+ * atma_packed_causal_conv1d.  tails (or tails[i]) non-NULL: (num_slots, heads d, K - 1), row stride tails_ss[i]; the
+ * sequence's last K - 1 xn go to row slots[b] (T > 0) or the map's; continuing (T > 0): that row is read first as
+ * the left context instead of zeros.  cache[i] non-NULL: out row r is also stored to row slot_mapping[r] of the
+ * contiguous (total_slots, heads d) cache, negative and out-of-range slots skipped.  K 2..4, d 64 or 128, head-rows
+ * 16-byte aligned; w_dtype is dtype or ATMA_F32.
+ */
+int atma_canon_qkv(const void* const* x, const int64_t* ldr, const int64_t* ldh, const int64_t* heads, const int* norm,
+                   const void* const* w, void* const* out, void* const* tails, const int64_t* tails_ss,
+                   void* const* cache, int64_t n, int64_t rows, int64_t T, const int32_t* seq_starts,
+                   const int32_t* seq_ends, const int32_t* seq_slots, const int64_t* slots, int64_t num_slots,
+                   int continuing, const int32_t* slot_mapping, int64_t total_slots, int64_t K, int64_t d, float eps,
+                   int w_dtype, int dtype, void* stream);
+
+/*
+ * The backward of out = x + conv(x) for n streams (1..3) of (rows, channels[i]) contiguous rows, rows / T sequences of
+ * T rows: dx[i] (rows' dtype) and dw[i] (channels[i], K) in w_dtype, summed in fp32 in a fixed order.  channels a
+ * multiple of 8; workspace of atma_canon_bwd_workspace_bytes(rows, T, the channels' sum, K).
+ */
+size_t atma_canon_bwd_workspace_bytes(int64_t rows, int64_t T, int64_t channels, int64_t K);
+int atma_canon_bwd(const void* const* dy, const void* const* x, const void* const* w, void* const* dx, void* const* dw,
+                   const int64_t* channels, int64_t n, int64_t rows, int64_t T, int64_t K, int w_dtype, int dtype,
+                   void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -31,6 +31,14 @@ def _rows16(t: Tensor) -> Tensor:
 
 
 # --------------------------------------------------------------------------- Polar fwd
+def _polar_fwd_scratch(lib, q, Hkv, Tk, is_causal, window):
+    """Workspace of a forward launch whose tiles are split along the keys (None: whole tiles)."""
+    B, Hq, Tq, d = q.shape
+    n = lib.atma_polar_attention_fwd_workspace_bytes(B, Hq, Hkv, Tq, Tk, d, _lib.dtype_code(q.dtype),
+                                                     1 if is_causal else 0, window)
+    return torch.empty(n, device=q.device, dtype=torch.uint8) if n else None, n
+
+
 @torch.library.custom_op("atma_hip::polar_attention_fwd", mutates_args=())
 def polar_attention_fwd_op(q: Tensor, k: Tensor, v: Tensor, n_keys: Tensor, v_null: Tensor,
                            null_base: Tensor, null_slope_raw: Tensor, len_gain_raw: Tensor,
@@ -43,14 +51,15 @@ def polar_attention_fwd_op(q: Tensor, k: Tensor, v: Tensor, n_keys: Tensor, v_nu
     Hkv, Tk = k.shape[1], k.shape[2]
     c = torch.empty((B, Hq, Tq, d), device=q.device, dtype=q.dtype)
     mag = torch.empty((B, Hq, Tq), device=q.device, dtype=q.dtype)
-    rc = lib.atma_polar_attention_fwd(
+    ws, ws_bytes = _polar_fwd_scratch(lib, q, Hkv, Tk, is_causal, window)
+    rc = lib.atma_polar_attention_fwd_ws(
         q.data_ptr(), q.stride(0), q.stride(1), q.stride(2),
         k.data_ptr(), k.stride(0), k.stride(1), k.stride(2),
         v.data_ptr(), v.stride(0), v.stride(1), v.stride(2),
         n_keys.data_ptr(), v_null.data_ptr(), null_base.data_ptr(), null_slope_raw.data_ptr(),
         len_gain_raw.data_ptr(), mag_beta_raw.data_ptr(), c.data_ptr(), mag.data_ptr(),
         None, None, None, None, B, Hq, Hkv, Tq, Tk, d, _lib.dtype_code(q.dtype),
-        1 if is_causal else 0, window, 0, eps, _lib.stream_handle(q.device))
+        1 if is_causal else 0, window, 0, eps, _lib.ptr(ws), ws_bytes, _lib.stream_handle(q.device))
     _lib.check(rc, "polar_attention_fwd")
     return [c, mag]
 
@@ -78,7 +87,8 @@ def polar_attention_fwd_train_op(q: Tensor, k: Tensor, v: Tensor, n_keys: Tensor
     mag = torch.empty((B, Hq, Tq), device=q.device, dtype=q.dtype)
     M, L, Q2 = (torch.empty((B, Hq, Tq), device=q.device, dtype=torch.float32) for _ in range(3))
     S = torch.empty((B, Hq, Tq, d), device=q.device, dtype=torch.float32)
-    rc = lib.atma_polar_attention_fwd(
+    ws, ws_bytes = _polar_fwd_scratch(lib, q, Hkv, Tk, is_causal, window)
+    rc = lib.atma_polar_attention_fwd_ws(
         q.data_ptr(), q.stride(0), q.stride(1), q.stride(2),
         k.data_ptr(), k.stride(0), k.stride(1), k.stride(2),
         v.data_ptr(), v.stride(0), v.stride(1), v.stride(2),
@@ -86,7 +96,7 @@ def polar_attention_fwd_train_op(q: Tensor, k: Tensor, v: Tensor, n_keys: Tensor
         len_gain_raw.data_ptr(), mag_beta_raw.data_ptr(), c.data_ptr(), mag.data_ptr(),
         M.data_ptr(), L.data_ptr(), Q2.data_ptr(), S.data_ptr(), B, Hq, Hkv, Tq, Tk, d,
         _lib.dtype_code(q.dtype), 1 if is_causal else 0, window, 1 if preserve_length else 0, eps,
-        _lib.stream_handle(q.device))
+        _lib.ptr(ws), ws_bytes, _lib.stream_handle(q.device))
     _lib.check(rc, "polar_attention_fwd")
     return [c, mag, M, L, Q2, S]
 

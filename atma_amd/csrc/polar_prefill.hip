@@ -30,6 +30,7 @@
 //    leaves the safe range -- the first block, or a new maximum far above the old.
 //  * bf16/fp16 use v_mfma_f32_32x32x16_{bf16,f16}; fp32 inputs use
 //    v_mfma_f32_32x32x2f32 (full fp32 products: the 1e-4 mode).
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -72,7 +73,32 @@ struct PolarFwdArgs {
   const int* tile_q_start;
   const int* tile_seq_len;
   int total_tokens;
+  // split launches (kSplit kernels; see fwd_split_plan): a workgroup takes split_blocks key blocks of its tile, and
+  // nsplit workgroups stand ready for each tile
+  int split_blocks, nsplit;
+  f32x4* part;      // [nsplit][B Hq Tq] (m, L, Q2, key blocks of the tile)
+  float* part_acc;  // [nsplit][B Hq Tq][d]
+  f32x2* part_null; // [B Hq Tq] (null logit in the log2 domain, softplus(mag_beta_raw)), from the first chunk
 };
+
+// The unnormalised state of one chunk of a tile's keys, for polar_fwd_merge_kernel.  Lane pair (l, l ^ 32) holds query
+// row `row` (h = l / 32) and the accumulators in the O^T layout.
+template <int D>
+__device__ __forceinline__ void store_partial(const PolarFwdArgs& a, int chunk, int tile_blocks, int64_t row, bool ok,
+                                              int h, float m, float L, float Q2, float an2, float mbeta,
+                                              const f32x16* oacc) {
+  const int64_t at = (int64_t)chunk * a.B * a.Hq * a.Tq + row;
+  if (!ok) return;
+  if (h == 0) a.part[at] = f32x4{m, L, Q2, __builtin_bit_cast(float, tile_blocks)};
+  if (h == 0 && chunk == 0) a.part_null[row] = f32x2{an2, mbeta};
+  float* p = a.part_acc + at * D;
+#pragma unroll
+  for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *(f32x4*)(p + 32 * t + 8 * g + 4 * h) = f32x4{oacc[t][4 * g], oacc[t][4 * g + 1], oacc[t][4 * g + 2],
+                                                    oacc[t][4 * g + 3]};
+}
 
 template <typename T, int D>
 struct FwdCfg {
@@ -112,7 +138,7 @@ __device__ __forceinline__ f32x16 mfma32(const u32x4& a, const u32x4& b, const f
   }
 }
 
-template <typename T, int D>
+template <typename T, int D, bool kSplit>
 __global__ void __launch_bounds__(256, 2) polar_fwd_kernel(PolarFwdArgs args) {
   using Cfg = FwdCfg<T, D>;
   constexpr int BM = Cfg::BM, BN = Cfg::BN, VE = Cfg::VE, CPR = Cfg::CPR;
@@ -127,7 +153,13 @@ __global__ void __launch_bounds__(256, 2) polar_fwd_kernel(PolarFwdArgs args) {
 
   // ---- workgroup -> (b, q head, query tile), XCD-aware, longest tile first
   const int G = args.Hq / args.Hkv;
-  int bid = blockIdx.x;
+  int bid = blockIdx.x, rank = 0, chunk = 0;
+  if constexpr (kSplit) {  // one chunk of one tile: every tile's first chunk, the longest tile first, then the second ...
+    const int per_rank = args.B * args.Hq, rc = bid / per_rank;
+    bid %= per_rank;
+    chunk = rc / args.n_qtiles;
+    rank = rc % args.n_qtiles;
+  }
   if (args.xcd_remap) {
     const int x = bid & 7, p = bid >> 3;
     bid = (x + 8 * (p / G)) * G + p % G;
@@ -137,15 +169,16 @@ __global__ void __launch_bounds__(256, 2) polar_fwd_kernel(PolarFwdArgs args) {
   // A workgroup takes a pair of query tiles, the i-th longest and the i-th shortest
   // of its head, so under a causal mask every pair costs the same number of key
   // blocks: the grid has no long tail.
-  const int npairs = (args.n_qtiles + 1) / 2;
-  const int pair = unit % npairs;
+  const int npairs = kSplit ? 1 : (args.n_qtiles + 1) / 2;
+  const int pair = kSplit ? rank : unit % npairs;
   const int grp = unit / npairs;  // b * Hkv + kv head
   const int b = grp / args.Hkv, hk = grp % args.Hkv;
   const int hq = hk * G + g;
-  const int npass = pair < args.n_qtiles - 1 - pair ? 2 : 1;
+  const int npass = !kSplit && pair < args.n_qtiles - 1 - pair ? 2 : 1;
   for (int pass = 0; pass < npass; ++pass) {
   const int qt = pass == 0 ? args.n_qtiles - 1 - pair : pair;
   const int q0 = qt * BM;
+  if (kSplit && args.is_causal && chunk > 0 && chunk * args.split_blocks * BN >= min(q0 + BM, args.Tk)) return;
 
   const T* qp = (const T*)args.q + b * args.q_sb + hq * args.q_sh;
   const T* kp = (const T*)args.k + b * args.k_sb + hk * args.k_sh;
@@ -192,7 +225,14 @@ __global__ void __launch_bounds__(256, 2) polar_fwd_kernel(PolarFwdArgs args) {
     if (args.window > 0) kbeg = max((int)floorf(g_nlo) - args.window, 0);
     kbeg = (kbeg / BN) * BN;
   }
-  const int nblk_beg = kbeg / BN, nblk_end = (kend + BN - 1) / BN;
+  int nblk_beg = kbeg / BN, nblk_end = (kend + BN - 1) / BN;
+  const int tile_blocks = max(nblk_end - nblk_beg, 0);
+  if constexpr (kSplit) {
+    if (chunk > 0 && chunk * args.split_blocks >= tile_blocks) return;  // the same for every wave
+    nblk_beg += chunk * args.split_blocks;
+    // the last chunk takes whatever remains: counts that are not row + 1 may need more blocks than the plan's estimate
+    if (chunk + 1 < args.nsplit) nblk_end = min(nblk_end, nblk_beg + args.split_blocks);
+  }
 
   // ---- query operand (B of S^T) in registers
   u32x4 qreg16[Cfg::kHalf ? Cfg::QSTEPS : 1];
@@ -484,6 +524,14 @@ __global__ void __launch_bounds__(256, 2) polar_fwd_kernel(PolarFwdArgs args) {
   // ---- fold the null sink, normalise, magnitude
   float L = l_part + __shfl_xor(l_part, 32, 64);
   float Q2 = q2_part + __shfl_xor(q2_part, 32, 64);
+  if constexpr (kSplit) {
+    const int64_t prow = ((int64_t)b * args.Hq + hq) * args.Tq + qi;
+    if (tile_blocks > args.split_blocks) {
+      store_partial<D>(args, chunk, tile_blocks, prow, q_ok, h, m_run, L, Q2, temp * nullv * kLog2e, mbeta, oacc);
+      return;
+    }
+    if (q_ok && h == 0) args.part[prow] = f32x4{0.f, 0.f, 0.f, __builtin_bit_cast(float, tile_blocks)};
+  }
   const float an2 = temp * nullv * kLog2e;
   const float mn = fmaxf(m_run, an2);
   const float al = exp2f(m_run - mn);
@@ -976,7 +1024,7 @@ __global__ void __launch_bounds__(256, 2) polar_fwd16_kernel(PolarFwdArgs args) 
 // 2m + 1.  The two heads share every K / V tile, so a tile is copied once for 256 query
 // rows.  Each wave's arithmetic is polar_fwd16_kernel's, in the same order: the two
 // kernels give the same bits.
-template <typename T, int D>
+template <typename T, int D, bool kSplit>
 __global__ void __launch_bounds__(512, 1) polar_fwd16_pp_kernel(PolarFwdArgs args) {
   constexpr int BM = 128, BN = 64, CPR = D / 8, NT = D / 32, QSTEPS = D / 16;
   constexpr int RPI = 64 / CPR;  // rows per wave copy instruction (1 KB)
@@ -997,8 +1045,15 @@ __global__ void __launch_bounds__(512, 1) polar_fwd16_pp_kernel(PolarFwdArgs arg
   // pairs of one KV group adjacent (and on one XCD when the remap applies)
   const int G = args.Hq / args.Hkv, G2 = G / 2;
   const int per_rank = args.B * args.Hkv * G2;
-  const int rank = blockIdx.x / per_rank;
+  int rank = blockIdx.x / per_rank, chunk = 0;
   int u = blockIdx.x % per_rank;
+  if constexpr (kSplit) {
+    // every tile's first chunk, the longest tile first, then the second ...: consecutive workgroups go to the XCDs in
+    // turn, and with a tile's chunks adjacent the chunks that short tiles do not have would all miss the same XCDs.
+    // (Kept scalar: the copies' offsets derive from them.)
+    chunk = __builtin_amdgcn_readfirstlane(rank / args.n_qtiles);
+    rank = __builtin_amdgcn_readfirstlane(rank % args.n_qtiles);
+  }
   if (args.xcd_remap) {
     const int x = u & 7, p = u >> 3;
     u = (x + 8 * (p / G2)) * G2 + p % G2;
@@ -1008,6 +1063,7 @@ __global__ void __launch_bounds__(512, 1) polar_fwd16_pp_kernel(PolarFwdArgs arg
   const int hq = hk * G + 2 * (u % G2) + grp;
   const int q0 = (args.n_qtiles - 1 - rank) * BM;
   const int Tq = args.Tq, Tk = args.Tk;
+  if (kSplit && args.is_causal && chunk > 0 && chunk * args.split_blocks * BN >= min(q0 + BM, Tk)) return;
 
   const int hq_u = __builtin_amdgcn_readfirstlane(hq);
   const float lg_raw = args.len_gain_raw[hq_u], ns_raw = args.null_slope_raw[hq_u];
@@ -1112,8 +1168,18 @@ __global__ void __launch_bounds__(512, 1) polar_fwd16_pp_kernel(PolarFwdArgs arg
   // the bounds are uniform (read from LDS by every lane): made scalar here, so every copy's
   // block offset is scalar arithmetic -- a vector-computed scalar offset would reach the
   // inline-asm copies through v_readfirstlane, whose SGPR write the copy may read stale
-  const int nblk_beg = __builtin_amdgcn_readfirstlane(kbeg / BN);
-  const int nblk_end = __builtin_amdgcn_readfirstlane((kend + BN - 1) / BN);
+  int nblk_beg = __builtin_amdgcn_readfirstlane(kbeg / BN);
+  int nblk_end = __builtin_amdgcn_readfirstlane((kend + BN - 1) / BN);
+  const int tile_blocks = max(nblk_end - nblk_beg, 0);
+  if constexpr (kSplit) {
+    if (chunk > 0 && chunk * args.split_blocks >= tile_blocks) {  // the same for every wave
+      wait_vmcnt<0>();
+      return;
+    }
+    nblk_beg += chunk * args.split_blocks;
+    // the last chunk takes whatever remains: counts that are not row + 1 may need more blocks than the plan's estimate
+    if (chunk + 1 < args.nsplit) nblk_end = min(nblk_end, nblk_beg + args.split_blocks);
+  }
   const int nblk = nblk_end > nblk_beg ? nblk_end - nblk_beg : 0;
   if (nblk > 0 && grp == 1) copy_tile(krs, kst2, nblk_beg, Ks);  // K(0) into K buffer 0
 
@@ -1325,6 +1391,14 @@ __global__ void __launch_bounds__(512, 1) polar_fwd16_pp_kernel(PolarFwdArgs arg
   // ---- fold the null sink, normalise, magnitude (as polar_fwd16_kernel)
   float L = l_part + __shfl_xor(l_part, 32, 64);
   float Q2 = q2_part + __shfl_xor(q2_part, 32, 64);
+  if constexpr (kSplit) {
+    const int64_t prow = ((int64_t)b * args.Hq + hq) * args.Tq + qi;
+    if (tile_blocks > args.split_blocks) {
+      store_partial<D>(args, chunk, tile_blocks, prow, q_ok, h, m_run, L, Q2, temp * nullv * kLog2e, mbeta, oacc);
+      return;
+    }
+    if (q_ok && h == 0) args.part[prow] = f32x4{0.f, 0.f, 0.f, __builtin_bit_cast(float, tile_blocks)};
+  }
   const float an2 = temp * nullv * kLog2e;
   const float mn = fmaxf(m_run, an2);
   const float al = exp2f(m_run - mn);
@@ -1382,33 +1456,209 @@ __global__ void __launch_bounds__(512, 1) polar_fwd16_pp_kernel(PolarFwdArgs arg
   }
 }
 
+// Rows whose tile was split: the chunks' states merged against their common maximum, then the unsplit kernels'
+// epilogue.  A row is D / 8 lanes of eight dims; every lane reads the row's (m, L, Q2) itself.  Its arithmetic is per
+// row and repeated in every lane, so the logarithms of the row's calibration come from the first chunk's workgroup
+// (with D / 4 lanes a row computing them again the launch was bound by it: 15.7 us for 24,000 rows).
+template <typename T, int D>
+__global__ void __launch_bounds__(256) polar_fwd_merge_kernel(PolarFwdArgs a) {
+  constexpr int LPR = D / 8;
+  const int64_t rows = a.B * a.Hq * a.Tq;  // a split launch has under 512 workgroups' rows: 32-bit indexes
+  const int row = (int)(blockIdx.x * (256 / LPR) + threadIdx.x / LPR);
+  if (row >= rows) return;
+  const float blocks_bits = a.part[row][3];  // (a bit cast of the subscripted vector itself reads element 0)
+  const int blocks = __builtin_bit_cast(int, blocks_bits);
+  const int ns = min((blocks + a.split_blocks - 1) / a.split_blocks, a.nsplit);
+  if (ns <= 1) return;  // written by its only chunk
+  const int e0 = 8 * (threadIdx.x % LPR);
+  const int qi = row % a.Tq, bh = row / a.Tq, hq = bh % a.Hq;
+  const int64_t b = bh / a.Hq;
+  const f32x4* vp = (const f32x4*)(a.v_null + (int64_t)hq * D + e0);
+  const f32x4 vn[2] = {vp[0], vp[1]};
+  const f32x2 nul = a.part_null[row];
+  // four chunks at a time: their loads are issued together, then merged against the running maximum
+  float m = kSentinel, L = 0.f, Q2 = 0.f;
+  f32x4 s[2] = {};
+  for (int c0 = 0; c0 < ns; c0 += 4) {
+    f32x4 st[4], acc[4][2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int64_t at = min(c0 + i, ns - 1) * rows + row;
+      st[i] = a.part[at];
+      const f32x4* p = (const f32x4*)(a.part_acc + at * D + e0);
+      acc[i][0] = p[0];
+      acc[i][1] = p[1];
+    }
+    float mx = m;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) mx = fmaxf(mx, st[i][0]);
+    const float old = exp2f(m - mx);
+    L *= old;
+    Q2 *= old * old;
+    s[0] *= old;
+    s[1] *= old;
+    m = mx;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float al = c0 + i < ns ? exp2f(st[i][0] - mx) : 0.f;
+      L += st[i][1] * al;
+      Q2 += st[i][2] * al * al;
+      s[0] += acc[i][0] * al;
+      s[1] += acc[i][1] * al;
+    }
+  }
+  const float mn = fmaxf(m, nul[0]);
+  const float al = exp2f(m - mn), pn = exp2f(nul[0] - mn);
+  L *= al;
+  Q2 *= al * al;
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    s[i] = s[i] * al + vn[i] * pn;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss += s[i][e] * s[i][e];
+  }
+#pragma unroll
+  for (int x = 1; x < LPR; x *= 2) ss += __shfl_xor(ss, x, 64);
+  const float inv = 1.f / fmaxf(sqrtf(ss), a.eps);
+  T* cp = (T*)a.c + b * a.c_sb + hq * a.c_sh + qi * a.c_st + e0;
+  if constexpr (sizeof(T) == 2) {
+    *(u32x4*)cp = u32x4{pack2<T>(s[0][0] * inv, s[0][1] * inv), pack2<T>(s[0][2] * inv, s[0][3] * inv),
+                        pack2<T>(s[1][0] * inv, s[1][1] * inv), pack2<T>(s[1][2] * inv, s[1][3] * inv)};
+  } else {
+    ((f32x4*)cp)[0] = s[0] * inv;
+    ((f32x4*)cp)[1] = s[1] * inv;
+  }
+  if (e0 == 0) {
+    const float m_eff = L * L / fmaxf(Q2, 1e-30f) * (L / fmaxf(L + pn, a.eps));
+    ((T*)a.mag)[b * a.m_sb + hq * a.m_sh + qi * a.m_st] = (T)tanhf(nul[1] * log1pf(m_eff));
+    if (a.stat_m) a.stat_m[row] = mn * kLn2;
+    if (a.stat_l) a.stat_l[row] = L;
+    if (a.stat_q2) a.stat_q2[row] = Q2;
+  }
+  if (a.stat_s) {
+    f32x4* sp = (f32x4*)(a.stat_s + (int64_t)row * D + e0);
+    sp[0] = s[0];
+    sp[1] = s[1];
+  }
+}
+
+// Whether a launch's tiles are split along the keys, and how.  A grid of a few tiles (one prompt, a chunk behind a long
+// prefix) leaves CUs idle or waits for its longest tile: up to about T = 16,000 at 8 heads.  Its tiles are cut into
+// chunks of `blocks` 64-key blocks, each a workgroup, and a second launch merges them.  Chosen by estimated time in
+// units of one block's: the smallest chunk that keeps the grid within one, two or three rounds of the device against
+// the whole tiles, counting a workgroup's prologue and epilogue (about 8 us) and the merge launch with its traffic.
+// Tiles of 8 blocks or fewer (fp32: 4) stay whole, as do grids that fill two rounds and 16-bit launches of odd GQA groups (the
+// one-head kernel, whose two workgroups per CU leave half as many slots idle).  The plan depends on sizes only (256 CUs
+// assumed).  Measured (8 / 2 heads, d = 128): 2,048 bf16 queries behind 12,000 keys 325 -> 115 + 9 us (merge); one
+// prompt of 2,999 tokens beside the recurrence 79 -> 41 + 8.5 us; fp32, 2,048 tokens 344 -> 209 + 14 us.
+struct SplitPlan {
+  int blocks = 0, nsplit = 0;  // 0: whole tiles
+};
+
+static SplitPlan fwd_split_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Tq, int64_t Tk, bool f32, bool causal,
+                                int64_t window) {
+  // causal 16-bit: 224 of 256 CUs, since the memory's recurrence runs beside a single prompt's attention on 32 of them
+  const int64_t kSlots = f32 || !causal ? 256 : 224, kMinBlocks = f32 ? 4 : 8;
+  const int64_t nt = (Tq + 127) / 128;
+  const int64_t per = f32 ? B * Hq : B * Hq / 2;  // workgroups of a rank: a tile of one head, or of two
+  if (nt * per >= 2 * 256 || nt == 0 || (!f32 && Hq / Hkv % 2)) return {};
+  auto len = [&](int64_t r) {
+    int64_t n = causal ? (r + 1 < nt ? 128 * (r + 1) : Tk) : Tk;
+    if (window > 0 && n > window + 192) n = window + 192;
+    return (n + 63) / 64;
+  };
+  double total = 0;
+  int64_t longest = 0;
+  for (int64_t r = 0; r < nt; ++r) total += (double)len(r), longest = len(r) > longest ? len(r) : longest;
+  if (longest <= kMinBlocks) return {};
+  // a 16-bit block (two heads) takes about 1.65 us, an fp32 one 10 us; a merged workgroup's rows cost 270 / 135 KB
+  const double over = f32 ? 1.5 : 5, merge = f32 ? 0.5 : 3.5, merge_unit = f32 ? 0.0035 : 0.04;
+  auto rounds = [&](double longest_unit, double units) {
+    const double even = 1.1 * (total * (double)per + over * units) / kSlots;
+    return longest_unit + over > even ? longest_unit + over : even;
+  };
+  // fp32 whole tiles run in pairs, longest with shortest
+  const double whole = rounds(f32 && nt > 1 ? (double)(longest + len(0)) : (double)longest, (double)(nt * per));
+  SplitPlan best;
+  double best_time = 0.9 * whole;
+  for (int w = 1; w <= 3; ++w) {
+    int64_t lo = kMinBlocks, hi = longest;  // the smallest chunk within w rounds
+    auto units = [&](int64_t c) {
+      int64_t u = 0;
+      for (int64_t r = 0; r < nt; ++r) u += (len(r) + c - 1) / c;
+      return u * per;
+    };
+    while (lo < hi) {
+      const int64_t c = (lo + hi) / 2;
+      if (units(c) <= w * kSlots) hi = c;
+      else lo = c + 1;
+    }
+    if (lo >= longest) continue;
+    const double u = (double)units(lo);
+    const double stepped = (w == 1 ? 1 : w - 0.5) * ((double)lo + over);
+    const double time = (w == 1 ? stepped : std::max(stepped, rounds((double)lo, u))) + merge + merge_unit * u;
+    if (time < best_time) {
+      best_time = time;
+      best = SplitPlan{(int)lo, (int)((longest + lo - 1) / lo)};
+    }
+  }
+  return best;
+}
+
+static size_t fwd_split_bytes(const SplitPlan& p, int64_t rows, int64_t d) {
+  return p.nsplit ? (size_t)p.nsplit * (size_t)rows * (size_t)(16 + 4 * d) + (size_t)rows * 8 : 0;
+}
+
 template <typename T, int D>
 static int launch_fwd(PolarFwdArgs a, hipStream_t stream) {
   const int G = a.Hq / a.Hkv;
+  const bool split = a.nsplit > 0;
+  const int64_t tiles = (int64_t)a.n_qtiles * (split ? a.nsplit : 1);
   if constexpr (sizeof(T) == 2) {
     // the ping-pong kernel addresses a (b, KV head) slice of k / v through one 32-bit buffer range
     const bool slices32 = (int64_t)a.Tk * a.k_st * 2 < (1ll << 32) && (int64_t)a.Tk * a.v_st * 2 < (1ll << 32);
-    if (G % 2 == 0 && !a.tile_seq_start && slices32) {
+    if (G % 2 == 0 && slices32) {
       // two query heads of a KV group per workgroup, the ping-pong schedule
       const int64_t per_rank = (int64_t)a.B * a.Hkv * (G / 2);
       a.xcd_remap = (per_rank % (8 * (G / 2)) == 0) ? 1 : 0;
-      polar_fwd16_pp_kernel<T, D><<<dim3((unsigned)(a.n_qtiles * per_rank)), dim3(512), 0, stream>>>(a);
+      const dim3 grid((unsigned)(tiles * per_rank));
+      if (split) polar_fwd16_pp_kernel<T, D, true><<<grid, dim3(512), 0, stream>>>(a);
+      else polar_fwd16_pp_kernel<T, D, false><<<grid, dim3(512), 0, stream>>>(a);
+    } else {
+      // one query tile per workgroup
+      const int64_t per_rank = (int64_t)a.B * a.Hq;
+      a.xcd_remap = (per_rank % (8 * G) == 0) ? 1 : 0;
+      polar_fwd16_kernel<T, D><<<dim3((unsigned)(a.n_qtiles * per_rank)), dim3(256), 0, stream>>>(a);
       return check_launch("polar_attention_fwd");
     }
-    // one query tile per workgroup
+  } else if (split) {
     const int64_t per_rank = (int64_t)a.B * a.Hq;
     a.xcd_remap = (per_rank % (8 * G) == 0) ? 1 : 0;
-    polar_fwd16_kernel<T, D><<<dim3((unsigned)(a.n_qtiles * per_rank)), dim3(256), 0, stream>>>(a);
+    polar_fwd_kernel<T, D, true><<<dim3((unsigned)(tiles * per_rank)), dim3(256), 0, stream>>>(a);
   } else {
     // a pair of query tiles (the i-th longest and the i-th shortest) per workgroup
     const int64_t units = (int64_t)((a.n_qtiles + 1) / 2) * a.B * a.Hq;
     a.xcd_remap = (units % (8 * G) == 0) ? 1 : 0;
-    polar_fwd_kernel<T, D><<<dim3((unsigned)units), dim3(256), 0, stream>>>(a);
+    polar_fwd_kernel<T, D, false><<<dim3((unsigned)units), dim3(256), 0, stream>>>(a);
+  }
+  if (split) {
+    constexpr int kRows = 256 / (D / 8);
+    const int64_t rows = (int64_t)a.B * a.Hq * a.Tq;
+    polar_fwd_merge_kernel<T, D><<<dim3((unsigned)((rows + kRows - 1) / kRows)), dim3(256), 0, stream>>>(a);
   }
   return check_launch("polar_attention_fwd");
 }
 
 }  // namespace atma
+
+extern "C" size_t atma_polar_attention_fwd_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t Tq, int64_t Tk,
+                                                           int64_t d, int dtype, int is_causal, int64_t window) {
+  using namespace atma;
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || Tq <= 0 || Tk <= 0 || Tq > (1 << 30) || Tk > (1 << 30) || B * Hq > (1 << 24))
+    return 0;
+  return fwd_split_bytes(fwd_split_plan(B, Hq, Hkv, Tq, Tk, dtype == ATMA_F32, is_causal != 0, window), B * Hq * Tq, d);
+}
 
 extern "C" int atma_polar_attention_fwd(
     const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void* k, int64_t k_sb,
@@ -1418,6 +1668,20 @@ extern "C" int atma_polar_attention_fwd(
     float* stat_l, float* stat_q2, float* stat_s, int64_t B, int64_t Hq, int64_t Hkv, int64_t Tq,
     int64_t Tk, int64_t d, int dtype, int is_causal, int64_t window, int preserve_length, float eps,
     void* stream) {
+  return atma_polar_attention_fwd_ws(q, q_sb, q_sh, q_st, k, k_sb, k_sh, k_st, v, v_sb, v_sh, v_st, n_keys, v_null,
+                                     null_base, null_slope_raw, len_gain_raw, mag_beta_raw, c, mag, stat_m, stat_l,
+                                     stat_q2, stat_s, B, Hq, Hkv, Tq, Tk, d, dtype, is_causal, window, preserve_length,
+                                     eps, nullptr, 0, stream);
+}
+
+extern "C" int atma_polar_attention_fwd_ws(
+    const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void* k, int64_t k_sb,
+    int64_t k_sh, int64_t k_st, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_st,
+    const float* n_keys, const float* v_null, const float* null_base, const float* null_slope_raw,
+    const float* len_gain_raw, const float* mag_beta_raw, void* c, void* mag, float* stat_m,
+    float* stat_l, float* stat_q2, float* stat_s, int64_t B, int64_t Hq, int64_t Hkv, int64_t Tq,
+    int64_t Tk, int64_t d, int dtype, int is_causal, int64_t window, int preserve_length, float eps,
+    void* workspace, size_t workspace_bytes, void* stream) {
   using namespace atma;
   if (B < 0 || Hq <= 0 || Hkv <= 0 || Tq < 0 || Tk < 0)
     return set_error(ATMA_ERR_INVALID, "polar_attention_fwd: bad sizes");
@@ -1461,6 +1725,23 @@ extern "C" int atma_polar_attention_fwd(
   a.n_qtiles = (int)((Tq + 127) / 128);
   a.c_st = d; a.c_sh = Tq * d; a.c_sb = Hq * Tq * d;  // c, mag contiguous (B, Hq, Tq[, d])
   a.m_st = 1; a.m_sh = Tq; a.m_sb = Hq * Tq;
+  if (workspace) {
+    const SplitPlan p = fwd_split_plan(B, Hq, Hkv, Tq, Tk, dtype == ATMA_F32, is_causal != 0, window);
+    const int64_t rows = B * Hq * Tq;
+    if (workspace_bytes < fwd_split_bytes(p, rows, d) || (uintptr_t)workspace % 16)
+      return set_error(ATMA_ERR_WORKSPACE, "polar_attention_fwd: workspace too small or unaligned");
+    if (p.nsplit * (int64_t)a.n_qtiles * B * Hq > 0x7fffffff)
+      return set_error(ATMA_ERR_INVALID, "polar_attention_fwd: sizes too large");
+    // the one-head kernel also serves K / V slices beyond a 32-bit buffer range, whole
+    const bool wide = dtype != ATMA_F32 && (Tk * k_st * 2 >= (1ll << 32) || Tk * v_st * 2 >= (1ll << 32));
+    if (p.nsplit && !wide) {
+      a.split_blocks = p.blocks;
+      a.nsplit = p.nsplit;
+      a.part = (f32x4*)workspace;
+      a.part_acc = (float*)(a.part + p.nsplit * rows);
+      a.part_null = (f32x2*)(a.part_acc + p.nsplit * rows * d);
+    }
+  }
   hipStream_t s = (hipStream_t)stream;
   switch (dtype) {
     case ATMA_BF16: return d == 128 ? launch_fwd<bf16, 128>(a, s) : launch_fwd<bf16, 64>(a, s);

@@ -91,6 +91,26 @@ int atma_polar_attention_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t 
                              float eps, void* stream);
 
 /*
+ * The same call with scratch for launches whose few tiles would leave CUs idle: their tiles are split along the keys
+ * into chunks whose fp32 states go through `workspace` (16-byte aligned) and a merge launch (outputs equal to
+ * rounding).  atma_polar_attention_fwd_workspace_bytes gives its size, 0 where whole tiles fill the device; a NULL
+ * workspace runs whole tiles, a smaller one is ATMA_ERR_WORKSPACE.
+ */
+size_t atma_polar_attention_fwd_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t Tq, int64_t Tk,
+                                                int64_t d, int dtype, int is_causal, int64_t window);
+int atma_polar_attention_fwd_ws(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st,
+                             const void* k, int64_t k_sb, int64_t k_sh, int64_t k_st,
+                             const void* v, int64_t v_sb, int64_t v_sh, int64_t v_st,
+                             const float* n_keys, const float* v_null, const float* null_base,
+                             const float* null_slope_raw, const float* len_gain_raw,
+                             const float* mag_beta_raw, void* c, void* mag, float* stat_m,
+                             float* stat_l, float* stat_q2, float* stat_s, int64_t B,
+                             int64_t Hq, int64_t Hkv, int64_t Tq, int64_t Tk, int64_t d,
+                             int dtype, int is_causal, int64_t window, int preserve_length,
+                             float eps, void* workspace,
+                             size_t workspace_bytes, void* stream);
+
+/*
  * Grouped fresh-prefill Polar attention over packed ragged requests.  Replaces
  * polar_attention_packed_fwd / _polar_packed_fwd_kernel (kernel/polar_triton.py:194-309,
  * 613-669).  q: (total_tokens, Hq, d) strides (q_st, q_sh, 1); k, v: (total_tokens, Hkv, d)

@@ -79,6 +79,10 @@ SIGNATURES = {
     "atma_linear_tokens_chunks": (_i32, [_p, _i64, _i64, _i64, _i64, _p, _p, _i64, _p, _i32, _p]),
     "atma_residual_rms_norm": (_i32, [_p, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64,
                                       _p, _p, _i64, _i64, _i64, _f32, _i32, _p]),
+    "atma_partial_sums": (_i32, [_p, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _i64, _i64, _i32, _p]),
+    "atma_memory_gate_logits": (_i32, [_p, _i64, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i32, _p]),
+    "atma_polar_params_f32": (_i32, [_p] * 6 + [_i64, _i64, _i32, _p]),
+    "atma_paged_kv_concat": (_i32, [_p, _p, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _i64, _p, _p, _i64, _i32, _p]),
     "atma_lfm2_conv_step": (_i32, [_p, _i64, _p, _i64, _p, _p, _i64, _i64, _p, _i64, _i64, _i64, _i32, _p]),
     "atma_global_decode_prep": (_i32, [_p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p, _i64, _p, _i64, _p, _i64,
                                        _p, _i64, _i64, _p, _p, _p, _p, _p, _p, _f32, _f32, _f32, _i64, _i64,

@@ -7,6 +7,8 @@
 //    and the norm read and write the row once together.  The branch is a 16-bit tensor or
 //    fp32 partial sums (linear_tokens' chunks form) plus biases and a low-rank term (the
 //    global layer's mu_proj(mag), 4, 8 or 16 inputs), added in fp32 and rounded once.
+//    atma_partial_sums is the same sum without the norm: a layer called on its own writes its output in one launch where
+//    torch makes about nine (65,536 x 1,024: see the layer's forward).
 //  * lfm2_conv_step: the LFM2 block's gated conv for one token, c * conv(b * x)
 //    (model/reference.py:31-48, inference/models/atma.py:625-673) from the rows of its
 //    in_proj output, state table advanced in place.
@@ -52,7 +54,7 @@ struct ResNormArgs {
   void* res_out;  // new stream (may be null when res is null)
   int64_t ldro;
   const void* w;  // (D,) T RMSNorm gain
-  void* out;      // (M, D) T
+  void* out;      // (M, D) T; null: no norm, the stream alone
   int64_t ldo;
   float eps;
   int M, D;
@@ -85,7 +87,7 @@ __global__ void __launch_bounds__(256) residual_rms_norm_kernel(ResNormArgs a) {
   for (int p = 0; p < P; ++p) {
     const int c = (p * 64 + lane) * 8;
     const int cc = c < a.D ? c : 0;  // lanes past the row read column 0 and drop it
-    wv[p] = *(const u32x4*)((const T*)a.w + cc);
+    if (a.out) wv[p] = *(const u32x4*)((const T*)a.w + cc);
     if constexpr (MU > 0) {
       // rows cc .. cc + 7 of mu_w (D, MU): 8 MU contiguous values, MU 16-byte vectors
 #pragma unroll
@@ -185,6 +187,7 @@ __global__ void __launch_bounds__(256) residual_rms_norm_kernel(ResNormArgs a) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) sq += s[p][e] * s[p][e];
     }
+    if (!a.out) continue;  // the sum alone (atma_partial_sums)
     const float rstd = rsqrtf(wave_sum(sq) / (float)a.D + a.eps);
 #pragma unroll
     for (int p = 0; p < P; ++p) {
@@ -354,30 +357,27 @@ __global__ void __launch_bounds__(64) global_decode_prep_kernel(GlobalPrepArgs a
 // ---------------------------------------------------------------------------- C ABI
 using namespace atma;
 
-extern "C" int atma_residual_rms_norm(const void* y, int64_t ldy, const float* parts, int64_t n_parts,
-                                      const void* const* bias, int64_t n_bias, const void* mu_x, int64_t ldmu,
-                                      const void* mu_w, int64_t mu_k, const void* res, int64_t ldr,
-                                      void* res_out, int64_t ldro, const void* weight, void* out, int64_t ldo,
-                                      int64_t M, int64_t D, float eps, int dtype, void* stream) {
+// atma_residual_rms_norm (weight and out given) and atma_partial_sums (neither).
+static int res_norm(const char* what, const void* y, int64_t ldy, const float* parts, int64_t n_parts,
+                    const void* const* bias, int64_t n_bias, const void* mu_x, int64_t ldmu, const void* mu_w,
+                    int64_t mu_k, const void* res, int64_t ldr, void* res_out, int64_t ldro, const void* weight,
+                    void* out, int64_t ldo, int64_t M, int64_t D, float eps, int dtype, void* stream) {
   if (dtype != ATMA_BF16 && dtype != ATMA_F16)
-    return set_error(ATMA_ERR_UNSUPPORTED, "residual_rms_norm: 16-bit only (dtype %d)", dtype);
+    return set_error(ATMA_ERR_UNSUPPORTED, "%s: 16-bit only (dtype %d)", what, dtype);
   if (M < 0 || D < 8 || D % 8 || D > 4096 || M > 0x7fffffff)
-    return set_error(ATMA_ERR_INVALID, "residual_rms_norm: D must be a multiple of 8 in [8, 4096] (got %lld)",
-                     (long long)D);
+    return set_error(ATMA_ERR_INVALID, "%s: D must be a multiple of 8 in [8, 4096] (got %lld)", what, (long long)D);
   if (M == 0) return ATMA_OK;
-  if (!weight || !out || (!y && !parts) || (y && parts))
-    return set_error(ATMA_ERR_INVALID, "residual_rms_norm: need weight, out and exactly one of y / parts");
+  if ((!y && !parts) || (y && parts))
+    return set_error(ATMA_ERR_INVALID, "%s: need weight, out and exactly one of y / parts", what);
   if ((parts && (n_parts < 1 || n_parts > kResMaxParts)) || n_bias < 0 || n_bias > kResMaxBias || (n_bias && !bias))
-    return set_error(ATMA_ERR_INVALID, "residual_rms_norm: 1 to %d parts and at most %d biases", kResMaxParts,
-                     kResMaxBias);
+    return set_error(ATMA_ERR_INVALID, "%s: 1 to %d parts and at most %d biases", what, kResMaxParts, kResMaxBias);
   if (mu_x && (!mu_w || (mu_k != 4 && mu_k != 8 && mu_k != 16) || ldmu < mu_k || ldmu % 2 || ((uintptr_t)mu_x & 3) ||
                ((uintptr_t)mu_w & 15)))
-    return set_error(ATMA_ERR_INVALID, "residual_rms_norm: the low-rank term needs a 16-byte aligned mu_w of width 4, 8 "
-                     "or 16");
+    return set_error(ATMA_ERR_INVALID, "%s: the low-rank term needs a 16-byte aligned mu_w of width 4, 8 or 16", what);
   auto al16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
   if ((y && (!al16(y) || ldy % 8 || ldy < D)) || (parts && !al16(parts)) || (res && (!al16(res) || ldr % 8 || ldr < D)) ||
-      (res_out && (!al16(res_out) || ldro % 8 || ldro < D)) || !al16(weight) || !al16(out) || ldo % 8 || ldo < D)
-    return set_error(ATMA_ERR_INVALID, "residual_rms_norm: rows must be 16-byte aligned and at least D long");
+      (res_out && (!al16(res_out) || ldro % 8 || ldro < D)) || !al16(weight) || !al16(out) || ldo % 8 || (out && ldo < D))
+    return set_error(ATMA_ERR_INVALID, "%s: rows must be 16-byte aligned and at least D long", what);
   ResNormArgs a{};
   a.y = y;
   a.ldy = ldy;
@@ -385,7 +385,7 @@ extern "C" int atma_residual_rms_norm(const void* y, int64_t ldy, const float* p
   a.n_parts = parts ? (int)n_parts : 0;
   a.n_bias = (int)n_bias;
   for (int i = 0; i < a.n_bias; ++i) {
-    if (!bias[i] || !al16(bias[i])) return set_error(ATMA_ERR_INVALID, "residual_rms_norm: bias %d null or unaligned", i);
+    if (!bias[i] || !al16(bias[i])) return set_error(ATMA_ERR_INVALID, "%s: bias %d null or unaligned", what, i);
     a.bias[i] = bias[i];
   }
   a.mu_x = mu_x;
@@ -405,7 +405,27 @@ extern "C" int atma_residual_rms_norm(const void* y, int64_t ldy, const float* p
   hipStream_t s = (hipStream_t)stream;
   if (dtype == ATMA_BF16) launch_res_norm<bf16>(a, s);
   else launch_res_norm<f16>(a, s);
-  return check_launch("residual_rms_norm");
+  return check_launch(what);
+}
+
+extern "C" int atma_residual_rms_norm(const void* y, int64_t ldy, const float* parts, int64_t n_parts,
+                                      const void* const* bias, int64_t n_bias, const void* mu_x, int64_t ldmu,
+                                      const void* mu_w, int64_t mu_k, const void* res, int64_t ldr,
+                                      void* res_out, int64_t ldro, const void* weight, void* out, int64_t ldo,
+                                      int64_t M, int64_t D, float eps, int dtype, void* stream) {
+  if (M > 0 && (dtype == ATMA_BF16 || dtype == ATMA_F16) && (!weight || !out))
+    return set_error(ATMA_ERR_INVALID, "residual_rms_norm: need weight, out and exactly one of y / parts");
+  return res_norm("residual_rms_norm", y, ldy, parts, n_parts, bias, n_bias, mu_x, ldmu, mu_w, mu_k, res, ldr, res_out,
+                  ldro, weight, out, ldo, M, D, eps, dtype, stream);
+}
+
+extern "C" int atma_partial_sums(const void* y, int64_t ldy, const float* parts, int64_t n_parts,
+                                 const void* const* bias, int64_t n_bias, const void* mu_x, int64_t ldmu,
+                                 const void* mu_w, int64_t mu_k, void* out, int64_t ldo, int64_t M, int64_t D, int dtype,
+                                 void* stream) {
+  if (M > 0 && !out) return set_error(ATMA_ERR_INVALID, "partial_sums: null output");
+  return res_norm("partial_sums", y, ldy, parts, n_parts, bias, n_bias, mu_x, ldmu, mu_w, mu_k, nullptr, 0, out, ldo,
+                  nullptr, nullptr, 0, M, D, 0.f, dtype, stream);
 }
 
 extern "C" int atma_lfm2_conv_step(const void* bcx, int64_t ld, const void* weight, int64_t K, const int64_t* slots,

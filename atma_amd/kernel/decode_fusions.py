@@ -47,7 +47,7 @@ class PartialSums:
     (P, M, N) from ``linear_tokens_chunks``, plus ``biases`` (each (N,)) and an optional
     low-rank term ``mu_x @ mu_w.T`` (mu_x (M, k), mu_w (N, k), k 4, 8 or 16).
     ``residual_rms_norm`` adds it to the residual stream in the same launch (fp32, one
-    rounding); ``materialize`` is the same sum in torch."""
+    rounding); ``materialize`` is the sum alone, one launch for the rows that serves."""
 
     __slots__ = ("parts", "base", "biases", "mu_x", "mu_w", "dtype")
 
@@ -61,7 +61,31 @@ class PartialSums:
     def shape(self):
         return self.parts.shape[1:] if self.parts is not None else self.base.shape
 
+    def _summable(self):
+        t = self.parts if self.base is None else self.base
+        return (not torch.is_grad_enabled() and t.is_cuda and self.dtype in _DT and t.shape[-1] % 8 == 0
+                and 8 <= t.shape[-1] <= 4096 and len(self.biases) <= 3
+                and (t.dtype == torch.float32 and t.is_contiguous() and t.shape[0] <= 8 if self.base is None
+                     else t.dtype == self.dtype and t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0)
+                and all(b.dtype == self.dtype and b.data_ptr() % 16 == 0 for b in self.biases)
+                and (self.mu_x is None or (self.mu_x.shape[1] in (4, 8, 16) and self.mu_x.dtype == self.dtype
+                                           and self.mu_w.dtype == self.dtype and self.mu_x.stride(1) == 1)))
+
     def materialize(self):
+        if self._summable():
+            M, D = self.shape
+            out = torch.empty((M, D), device=(self.parts if self.base is None else self.base).device, dtype=self.dtype)
+            biases = [b.contiguous() for b in self.biases]
+            _b, pb = _addr(ctypes.c_void_p, [b.data_ptr() for b in biases] or [None])
+            mu_w = None if self.mu_x is None else self.mu_w.contiguous()
+            rc = _lib.load().atma_partial_sums(
+                _lib.ptr(self.base), 0 if self.base is None else self.base.stride(0), _lib.ptr(self.parts),
+                0 if self.parts is None else self.parts.shape[0], pb, len(biases), _lib.ptr(self.mu_x),
+                0 if self.mu_x is None else self.mu_x.stride(0), _lib.ptr(mu_w),
+                0 if self.mu_x is None else self.mu_x.shape[1], out.data_ptr(), out.stride(0), M, D,
+                _lib.dtype_code(self.dtype), _lib.stream_handle(out.device))
+            _lib.check(rc, "partial_sums")
+            return out
         s = self.parts.sum(0) if self.parts is not None else self.base.float()
         for b in self.biases:
             s = s + b.float()

@@ -1,6 +1,7 @@
 """Per-head glue of the global layer, the LFM2 prefill conv and the MLP's gated first
 projection over many rows, backed by libatma_hip.so (C ABI ``atma_head_rms_norm``,
-``atma_global_gate``, ``atma_lfm2_conv_packed``, ``atma_linear_gated``).
+``atma_global_gate``, ``atma_lfm2_conv_packed``, ``atma_linear_gated``), and the small launches around the layer's
+prefill (``atma_memory_gate_logits``, ``atma_paged_kv_concat``).
 
 No reference counterparts: each is one launch for a chain of the reference's eager ops on
 the served path (``model/reference.py:31-48,131-139``, ``model/blocks.py:470-490``,
@@ -125,3 +126,48 @@ def linear_gated(x, weight, bias=None):
                                        _lib.stream_handle(x.device))
     _lib.check(rc, "linear_gated")
     return y
+
+
+def memory_gate_logits_supported(x, wg, wb):
+    """Rows ``memory_gate_logits`` serves: contiguous 16-bit (..., K) with K a multiple of 128, at most 16 heads."""
+    return (x.is_cuda and x.dtype in _DT and x.is_contiguous() and x.data_ptr() % 16 == 0 and x.shape[-1] % 128 == 0
+            and x.shape[-1] > 0 and wg.shape == wb.shape and wg.shape[0] <= 16 and wg.shape[1] == x.shape[-1]
+            and wg.dtype == wb.dtype == x.dtype and wg.is_contiguous() and wb.is_contiguous()
+            and wg.data_ptr() % 16 == 0 and wb.data_ptr() % 16 == 0)
+
+
+@torch.no_grad()
+def memory_gate_logits(x, wg, bg, wb, bb):
+    """``(x @ wg.T + bg, x @ wb.T + bb)`` in fp32 (never rounded to the rows' dtype), one launch: x (..., K) contiguous
+    16-bit, weights (H, K), biases (H,) or None.  Returns two (..., H) fp32 tensors."""
+    _gpu16(x, wg, wb)
+    K, H = x.shape[-1], wg.shape[0]
+    zg, zb = (torch.empty((*x.shape[:-1], H), device=x.device, dtype=torch.float32) for _ in range(2))
+    bg, bb = (None if b is None else b.to(x.dtype).contiguous() for b in (bg, bb))
+    rc = _lib.load().atma_memory_gate_logits(x.data_ptr(), K, wg.data_ptr(), _lib.ptr(bg), wb.data_ptr(), _lib.ptr(bb),
+                                             zg.data_ptr(), zb.data_ptr(), x.numel() // K, K, H,
+                                             _lib.dtype_code(x.dtype), _lib.stream_handle(x.device))
+    _lib.check(rc, "memory_gate_logits")
+    return zg, zb
+
+
+@torch.no_grad()
+def paged_kv_concat(k_cache, v_cache, pages, cached, k_new, v_new):
+    """A continued sequence's keys and values, contiguous: its first ``cached`` rows from the paged caches (num_pages,
+    page_size, Hkv, d), ``pages`` (1-D int32) naming the page of each page_size rows, then the chunk's k_new, v_new
+    (T, Hkv, d).  Returns two (cached + T, Hkv, d) tensors, one launch."""
+    num_pages, page, Hkv, d = k_cache.shape
+    T = k_new.shape[0]
+    if k_cache.shape != v_cache.shape or not (k_cache.is_contiguous() and v_cache.is_contiguous()) \
+            or k_new.shape != (T, Hkv, d) or v_new.shape != k_new.shape or pages.numel() * page < cached \
+            or any(t.dtype != k_cache.dtype for t in (v_cache, k_new, v_new)) \
+            or any(t.stride(2) != 1 or t.stride(1) != d for t in (k_new, v_new)):
+        raise ValueError("paged_kv_concat: contiguous caches, chunk rows (T, Hkv, d) and pages for every cached row")
+    pages = pages.to(device=k_cache.device, dtype=torch.int32).contiguous()
+    kb, vb = (torch.empty((cached + T, Hkv, d), device=k_cache.device, dtype=k_cache.dtype) for _ in range(2))
+    rc = _lib.load().atma_paged_kv_concat(k_cache.data_ptr(), v_cache.data_ptr(), num_pages, page, pages.data_ptr(), cached,
+                                          k_new.data_ptr(), k_new.stride(0), v_new.data_ptr(), v_new.stride(0), T,
+                                          kb.data_ptr(), vb.data_ptr(), Hkv * d, _lib.dtype_code(k_cache.dtype),
+                                          _lib.stream_handle(k_cache.device))
+    _lib.check(rc, "paged_kv_concat")
+    return kb, vb

@@ -12,6 +12,18 @@ from .. import _lib, _ops  # noqa: F401  (_ops registers torch.ops.atma_hip.*)
 
 
 def _params(device, v_null, null_base, null_slope_raw, len_gain_raw, mag_beta_raw):
+    """The five parameters in fp32 on ``device``; those of a 16-bit layer widened in one launch."""
+    ps = (v_null, null_base, null_slope_raw, len_gain_raw, mag_beta_raw)
+    if v_null.dtype in (torch.bfloat16, torch.float16) and not torch.compiler.is_compiling() and v_null.dim() == 2 \
+            and all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.device == device
+                    and t.dtype == v_null.dtype and t.is_contiguous() for t in ps) \
+            and all(t.numel() == v_null.shape[0] for t in ps[1:]):
+        H, d = v_null.shape
+        buf = torch.empty(H * (d + 4), device=device, dtype=torch.float32)
+        rc = _lib.load().atma_polar_params_f32(*[t.data_ptr() for t in ps], buf.data_ptr(), H, d,
+                                               _lib.dtype_code(v_null.dtype), _lib.stream_handle(device))
+        _lib.check(rc, "polar_params_f32")
+        return (buf[:H * d].view(H, d), *buf[H * d:].view(4, H).unbind())
     f = lambda t: t.detach().to(device=device, dtype=torch.float32).contiguous()  # noqa: E731
     return (f(v_null), f(null_base), f(null_slope_raw), f(len_gain_raw), f(mag_beta_raw))
 

@@ -21,8 +21,8 @@ latency-bound with one workgroup per CU, so this pays only when its grid is smal
 quarter of the CUs or less: long sequences, small batches), and only if its workgroups
 start before Polar's fill the GPU; Polar's launch therefore waits on the recurrence's
 start signal (``StartSignal``).  ``overlap="auto"`` (default) takes the overlapped
-schedule exactly when ``recurrence_pays_to_overlap`` says so, ``True`` always, ``False``
-never.  Results are bitwise the same in every schedule.
+schedule for sequences of ``OVERLAP_TOKENS`` or more when ``recurrence_pays_to_overlap``
+says so, ``True`` always, ``False`` never.  Results are bitwise the same in every schedule.
 Training: when autograd must see the call (grad mode on and an input or parameter
 requiring grad), the full-sequence route runs the differentiable ops -- ``polar_attention``
 (HIP forward with saved statistics + HIP backward) and the autograd form of
@@ -48,7 +48,8 @@ from ..kernel.decode_fusions import (PartialSums, chunk_width, global_decode_gat
                                      residual_rms_norm, residual_rms_norm_supported)
 from ..kernel.inference_ops import (linear_tokens, linear_tokens_supported, packed_causal_conv1d,
                                      squared_relu_gate)
-from ..kernel.layer_fusions import global_gate, head_rms_norm, linear_gated, linear_gated_supported
+from ..kernel.layer_fusions import (global_gate, head_rms_norm, linear_gated, linear_gated_supported,
+                                    memory_gate_logits, memory_gate_logits_supported, paged_kv_concat)
 from ..kernel.polar import global_decode_step_supported_shape
 from .attention import store_kvcache
 
@@ -63,6 +64,9 @@ def decode_rows(x):
     return (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and x.dim() == 2 and x.shape[0] <= 32
             and x.is_contiguous() and not torch.is_grad_enabled())
 
+
+# overlap="auto": sequences from this length on run the memory branch beside Polar (PolarAttention._overlapped)
+OVERLAP_TOKENS = 8192
 
 # Polar structural priors (model/reference.py:17-20)
 LEN_GAIN_INIT = -1.0
@@ -107,8 +111,11 @@ class TitansMemory(nn.Module):
         nn.init.zeros_(self.proj.bias)
 
     def raw_logits(self, x):
-        """Gate logits before the biases (fp32); the biases are added by the fused
-        gate kernel together with the activations."""
+        """Gate logits before the retention and write biases (fp32), which the fused gate kernel adds together with
+        the activations.  16-bit inference rows: both projections in one launch (``memory_gate_logits``)."""
+        wg, wb = self.w_gamma, self.w_beta
+        if not torch.is_grad_enabled() and x.dim() > 2 and memory_gate_logits_supported(x, wg.weight, wb.weight):
+            return memory_gate_logits(x, wg.weight, wg.bias, wb.weight, wb.bias)
         return self.w_gamma(x).float(), self.w_beta(x).float()
 
     def _out(self, x, r):
@@ -358,12 +365,15 @@ class PolarAttention(nn.Module):
         return torch.is_grad_enabled() and (any(t.requires_grad for t in inputs)
                                             or any(p.requires_grad for p in self.parameters()))
 
-    def _overlapped(self, B, dtype, device, training=False):
+    def _overlapped(self, B, T, dtype, device, training=False):
+        """Whether the memory branch runs beside Polar.  Short sequences do not (``OVERLAP_TOKENS``): their layer is
+        bound by its launches, and the second stream's events cost the host about 190 us, more than the recurrence
+        it hides (2,999 tokens: 0.69 ms overlapped, 0.51 ms on one stream; 2,048 behind 12,000: 0.71 and 0.53 ms)."""
         if self.mem is None or self.overlap is False or device.type != "cuda" or training \
                 or torch.cuda.is_current_stream_capturing():
             return False
-        return self.overlap is True or recurrence_pays_to_overlap(B, self.num_heads, self.head_dim,
-                                                                  dtype, device)
+        return self.overlap is True or (T >= OVERLAP_TOKENS and recurrence_pays_to_overlap(
+            B, self.num_heads, self.head_dim, dtype, device))
 
     def _with_memory(self, polar_fn, mem_fn, inputs):
         """Run the Polar part on the current stream and the memory branch (``mem_fn(signal)``)
@@ -371,7 +381,7 @@ class PolarAttention(nn.Module):
         if self.mem is None:
             return polar_fn(), None
         x = inputs[0]
-        if not self._overlapped(x.shape[0], x.dtype, x.device, self._training(*inputs)):
+        if not self._overlapped(x.shape[0], x.shape[1], x.dtype, x.device, self._training(*inputs)):
             return polar_fn(), mem_fn(None)
         main = torch.cuda.current_stream(x.device)
         side = self._side_stream(x.device)
@@ -505,28 +515,42 @@ class PolarAttention(nn.Module):
         q, gate, k, v = (t.unflatten(0, (B, T)) for t in
                          self._project_canon(x, B, T, cache, slots, slot_mapping, continuing=True))
         page = cache.k_cache.shape[1]
-        cs, ms = [], []
+        kvs = []
         for b in range(B):
             n = cached[b]
             if n > 0:
-                pages = block_tables[b, :(n + page - 1) // page].long()
-                kp = cache.k_cache[pages].reshape(-1, Hkv, dk)[:n]
-                vp = cache.v_cache[pages].reshape(-1, Hkv, dk)[:n]
-                kb, vb = torch.cat([kp, k[b]], 0), torch.cat([vp, v[b]], 0)
+                kb, vb = paged_kv_concat(cache.k_cache, cache.v_cache, block_tables[b, :(n + page - 1) // page], n,
+                                         k[b], v[b])
             else:
                 kb, vb = k[b], v[b]
-            n_keys = torch.arange(n + 1, n + T + 1, device=x.device, dtype=torch.float32)
-            c, mag = polar_attention_fwd(q[b].transpose(0, 1).unsqueeze(0), kb.transpose(0, 1).unsqueeze(0),
-                                         vb.transpose(0, 1).unsqueeze(0), n_keys, is_causal=n == 0,
-                                         window=self.window, **self.polar_params())
-            cs.append(c[0].transpose(0, 1))
-            ms.append(mag[0].transpose(0, 1))
-        out = self._combine(torch.stack(cs), torch.stack(ms), gate)
-        if self.mem is not None:
-            r, S = self.mem(x, q, k, v, initial_state=cache.mem_table[slots], output_final_state=True)
-            cache.mem_table[slots] = S
-            out = out + r
-        return out
+            kvs.append((kb, vb, n))
+
+        def attend():
+            cs, ms = [], []
+            for b, (kb, vb, n) in enumerate(kvs):
+                n_keys = torch.arange(n + 1, n + T + 1, device=x.device, dtype=torch.float32)
+                c, mag = polar_attention_fwd(q[b].transpose(0, 1).unsqueeze(0), kb.transpose(0, 1).unsqueeze(0),
+                                             vb.transpose(0, 1).unsqueeze(0), n_keys, is_causal=n == 0,
+                                             window=self.window, **self.polar_params())
+                cs.append(c.transpose(1, 2))
+                ms.append(mag.transpose(1, 2))
+            return (cs[0], ms[0]) if B == 1 else (torch.cat(cs), torch.cat(ms))
+
+        fused = self._glue_fusable(x)
+        S0 = cache.mem_table[slots] if self.mem is not None else None
+
+        def memory(signal):
+            return (self.mem.readout if fused else self.mem)(x, q, k, v, initial_state=S0, output_final_state=True,
+                                                             start_signal=signal)
+
+        (c, mag), m = self._with_memory(attend, memory, (x, q, k, v))
+        if m is not None:
+            cache.mem_table[slots] = m[1]
+        if fused:
+            return self._fused_out(x.reshape(B * T, -1), c, mag.reshape(B * T, H), gate.reshape(B * T, H, dk),
+                                   m[0].reshape(B * T, H, dk)).materialize().view(B, T, -1)
+        out = self._combine(c, mag, gate)
+        return out if m is None else out + m[0]
 
     def _decode_fusable(self, x, cache, block_tables):
         H, Hkv, dk = self.num_heads, self.num_kv_heads, self.head_dim

@@ -699,6 +699,41 @@ int atma_canon_bwd(const void* const* dy, const void* const* x, const void* cons
                    const int64_t* channels, int64_t n, int64_t rows, int64_t T, int64_t K, int w_dtype, int dtype,
                    void* workspace, size_t workspace_bytes, void* stream);
 
+/*
+ * The sum atma_residual_rms_norm adds to its stream, alone (no reference counterpart as one call; the global layer's
+ * output, inference/models/atma.py:246-252): out = round(y or the parts' sum + biases + mu_x mu_w^T), in fp32 with one
+ * rounding.  Arguments as there.
+ */
+int atma_partial_sums(const void* y, int64_t ldy, const float* parts, int64_t n_parts, const void* const* bias,
+                      int64_t n_bias, const void* mu_x, int64_t ldmu, const void* mu_w, int64_t mu_k, void* out,
+                      int64_t ldo, int64_t M, int64_t D, int dtype, void* stream);
+
+/*
+ * The memory branch's raw gate logits (model/blocks.py:466-467) in fp32: zg = x wg^T + bg, zb = x wb^T + bb, (M, H)
+ * contiguous, one pass over the 16-bit rows x (M, K).  wg, wb (H, K) contiguous, bg, bb (H,) or NULL in the rows'
+ * dtype; H at most 16, K a multiple of 128.
+ */
+int atma_memory_gate_logits(const void* x, int64_t ldx, const void* wg, const void* bg, const void* wb, const void* bb,
+                            float* zg, float* zb, int64_t M, int64_t K, int64_t H, int dtype, void* stream);
+
+/*
+ * The Polar parameters of a 16-bit layer in fp32, as the attention entry points read them: out = v_null (H, d), then
+ * null_base, null_slope_raw, len_gain_raw and mag_beta_raw (H,) each, in one fp32 buffer of H (d + 4).
+ */
+int atma_polar_params_f32(const void* v_null, const void* null_base, const void* null_slope_raw,
+                          const void* len_gain_raw, const void* mag_beta_raw, float* out, int64_t H, int64_t d,
+                          int dtype, void* stream);
+
+/*
+ * A sequence's keys and values for a continued prefill (inference/models/atma.py:509-544): rows 0 .. cached - 1 from
+ * its pages (row r in page pages[r / page_size]; a page outside the cache reads as zeros), then the n_new rows of the
+ * chunk (row strides k_st, v_st), into contiguous (cached + n_new, row_elems) k_out and v_out.
+ */
+int atma_paged_kv_concat(const void* k_cache, const void* v_cache, int64_t num_pages, int64_t page_size,
+                         const int32_t* pages, int64_t cached, const void* k_new, int64_t k_st, const void* v_new,
+                         int64_t v_st, int64_t n_new, void* k_out, void* v_out, int64_t row_elems, int dtype,
+                         void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -970,40 +970,73 @@ __global__ void __launch_bounds__(256, 1) gdn_scan16_pair_kernel(GdnArgs a) {
 
 // Entry states of the segments from their summaries (fp32): seg_in[0] = s0 (or 0) and
 // seg_in[s] = M_{s-1} seg_in[s-1] + B_{s-1}, where summary s - 1 holds [B | M] row by row.
-// One workgroup per (sequence-head, 16 state columns); M is staged in LDS (rows padded
-// against bank conflicts) and thread t owns row t % D and D / 16 of the columns.
+// One workgroup of four waves per (sequence-head, 16 state columns), a wave D / 4 rows of the product on
+// v_mfma_f32_16x16x4f32 with the k index permuted (step i contracts k = D/4 g + i), so that a lane's operand of M is
+// D / 4 consecutive floats.  The chain is one product per segment: M and B of the next one are loaded under it, and the
+// state passes between the waves through LDS.  Bound by latency, one load and one chain of D / 8 dependent
+// products a segment: 20,000 tokens of 4 heads 13.8 us, 85 us with the products on VALU and M staged through LDS.
 template <int D>
 __global__ void __launch_bounds__(256) gdn_seg_combine_kernel(GdnArgs a) {
-  constexpr int NCOL = D / 16, MP = D + 1;
-  __shared__ float Ms[D * MP];
-  __shared__ float cur[D][16];
-  const int bh = blockIdx.x, j0 = 16 * blockIdx.y, tid = threadIdx.x;
-  const int k = tid % D, jc = NCOL * (tid / D);
-  for (int e = tid; e < D * 16; e += 256) {
-    const int r = e / 16, jj = e % 16;
-    const float x = a.s0 ? a.s0[((int64_t)bh * D + r) * D + j0 + jj] : 0.f;
-    cur[r][jj] = x;
-    a.seg_in[((int64_t)bh * a.nseg * D + r) * D + j0 + jj] = x;
-  }
-  for (int sg = 1; sg < a.nseg; ++sg) {
-    const float* sum = a.seg_sum + ((int64_t)bh * a.nseg + sg - 1) * D * 2 * D;
-    __syncthreads();  // the previous step's reads of Ms and cur are done
-    for (int e = tid; e < D * D; e += 256) Ms[(e / D) * MP + e % D] = sum[(e / D) * 2 * D + D + e % D];
-    __syncthreads();
-    float acc[NCOL];
+  constexpr int RT = D / 64, KL = D / 4;  // 16-row tiles per wave; k values per lane
+  __shared__ __attribute__((aligned(16))) float cur[2][16][D + 4];  // the entry state's columns, [column][row]
+  const int bh = blockIdx.x, j0 = 16 * blockIdx.y;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
+  const float* s0 = a.s0 ? a.s0 + (int64_t)bh * D * D : nullptr;
+  f32x4 S[RT];
 #pragma unroll
-    for (int c = 0; c < NCOL; ++c) acc[c] = sum[k * 2 * D + j0 + jc + c];
-    for (int m = 0; m < D; ++m) {
-      const float mk = Ms[k * MP + m];
+  for (int t = 0; t < RT; ++t)
 #pragma unroll
-      for (int c = 0; c < NCOL; ++c) acc[c] = fmaf(mk, cur[m][jc + c], acc[c]);
+    for (int i = 0; i < 4; ++i) {
+      const int row = 16 * (RT * wave + t) + 4 * g + i;
+      S[t][i] = s0 ? s0[row * D + j0 + c] : 0.f;
     }
-    __syncthreads();  // every thread has read cur
+  f32x4 m[RT][KL / 4], B[RT];
+  auto load = [&](int sg) {
+    const float* sum = a.seg_sum + ((int64_t)bh * a.nseg + sg) * D * 2 * D;
 #pragma unroll
-    for (int c = 0; c < NCOL; ++c) {
-      cur[k][jc + c] = acc[c];
-      a.seg_in[(((int64_t)bh * a.nseg + sg) * D + k) * D + j0 + jc + c] = acc[c];
+    for (int t = 0; t < RT; ++t) {
+      const float* mr = sum + (16 * (RT * wave + t) + c) * 2 * D + D + KL * g;
+#pragma unroll
+      for (int i = 0; i < KL / 4; ++i) m[t][i] = *(const f32x4*)(mr + 4 * i);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) B[t][i] = sum[(16 * (RT * wave + t) + 4 * g + i) * 2 * D + j0 + c];
     }
+  };
+  load(0);
+  for (int sg = 0; sg < a.nseg; ++sg) {
+    float* in = a.seg_in + ((int64_t)bh * a.nseg + sg) * D * D + j0 + c;
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      const int r0 = 16 * (RT * wave + t) + 4 * g;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) in[(r0 + i) * D] = S[t][i];
+      *(f32x4*)&cur[sg & 1][c][r0] = S[t];
+    }
+    if (sg + 1 == a.nseg) break;
+    __syncthreads();  // (the other buffer's readers are past the previous step's barrier)
+    f32x4 acc[RT][2];
+    float mm[RT][KL], bb[KL];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      acc[t][0] = B[t];
+      acc[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < KL; ++i) mm[t][i] = m[t][i >> 2][i & 3];
+    }
+    if (sg + 2 < a.nseg) load(sg + 1);
+#pragma unroll
+    for (int i = 0; i < KL / 4; ++i) {
+      const f32x4 v = *(const f32x4*)&cur[sg & 1][c][KL * g + 4 * i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bb[4 * i + e] = v[e];
+    }
+#pragma unroll
+    for (int i = 0; i < KL; ++i)
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+        acc[t][i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(mm[t][i], bb[i], acc[t][i & 1], 0, 0, 0);
+#pragma unroll
+    for (int t = 0; t < RT; ++t) S[t] = acc[t][0] + acc[t][1];
   }
 }
 

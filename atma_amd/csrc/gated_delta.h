@@ -33,23 +33,30 @@ struct GdnArgs {
   // seg runs chunks [seg * seg_len, min(NC, (seg + 1) * seg_len)).  seg_mode 0: one segment,
   // the plain scan.  1: segment summaries -- no output; state columns >= D start from the
   // identity with v = 0, so a segment's exit state holds its affine map [B | M] (exit = M
-  // entry + B), written to seg_sum.  2: replay -- each segment starts from seg_in and
-  // writes its output; the last one writes s_out.
+  // entry + B), written to seg_sum.  2: replay -- each segment starts from its entry state
+  // and writes its output; the last one writes s_out.
   int seg_len, nseg, seg_mode;
-  float* seg_sum;  // [B*H][nseg][D][2D] fp32
-  float* seg_in;   // [B*H][nseg][D][D] fp32
+  float* seg_sum;  // [B*H][nseg - 1][D][2D] fp32: the summaries; then segment s + 1's entry state over the B half of s
+  float* seg_in;   // [B*H][D][D] fp32: segment 0's entry state (s0 may be s_out)
 };
 
-// Segments of the 16-bit recurrence for B*H sequence-heads of NC chunks at head dim D on a
-// device with `cus` compute units: enough that the summary pass (B*H*(2D/32) workgroups
-// per segment, one per CU) fills the device, each segment at least 8 chunks; 1 (the plain
-// scan) when the heads alone fill half of it.
-inline int gdn16_segments(int64_t BH, int64_t NC, int D, int cus) {
-  const int64_t per = BH * (2 * D / 32);  // summary workgroups of one segment
-  if (NC < 16 || 2 * per > cus) return 1;
-  int64_t n = 1 + cus / per;
+// Segments of the 16-bit recurrence for B*H sequence-heads of NC chunks at head dim D on a device with `cus` compute
+// units; `states` = the D x D states of scratch per sequence-head.  The summaries and the replays cost the same per chunk
+// (1.4 and 1.2 us at D = 128), so a split into n takes 2 / n of the plain scan, and n is as large as keeps both on one workgroup
+// per CU, with at least 8 chunks a segment; 1 (the plain scan) below 3 segments, where nothing is gained, or when the
+// heads alone fill half of the device.  One summary of n - 1 takes two states, the first entry state one.
+inline int gdn16_segments(int64_t BH, int64_t NC, int D, int cus, int64_t& states) {
+  const int64_t per = BH * (D / 32);  // workgroups of one segment: summaries (64 of 2D columns each), replays (32 of D)
+  states = 0;
+  if (NC < 16 || 4 * per > cus) return 1;
+  const int64_t room = 1 + cus / (2 * per);
+  states = 3 * (room < NC / 8 ? room : NC / 8);
+  int64_t n = cus / per;
   n = n < NC / 8 ? n : NC / 8;
-  return n < 2 ? 1 : (int)n;
+  n = n < (states + 1) / 2 ? n : (states + 1) / 2;
+  if (n >= 3) return (int)n;
+  states = 0;
+  return 1;
 }
 
 // Start signal of the recurrence kernel.  The scan is latency-bound and needs a whole CU

@@ -24,7 +24,7 @@
 //    over in LDS, and issues the copies: the k, q rows, the v slab and the record of chunk
 //    c + 2 stream into a third LDS slot (direct buffer copies) while chunk c computes.  Two
 //    workgroup barriers per chunk order the slots and the hand-over.  Segment summaries (no
-//    output) run the two-wave gdn_scan16 with the chain and the copies on the same waves.
+//    output) run four such chain waves per workgroup, which issue the copies as well.
 //
 // Fragment layouts (v_mfma_f32_16x16x32: A lane (g, r) holds row r, k = 8g + [0, 8); B lane
 // (g, c) holds column c, same k; accumulator lane (g, c) register i holds row 4g + i,
@@ -323,37 +323,38 @@ __device__ __forceinline__ int rec_swizzle(int r) {
   return CPR == 16 ? (r & 15) : ((r >> 1) & 7);
 }
 
-// OUT: the plain scan and segment replays (seg_mode 0, 2) produce the output; segment
-// summaries (seg_mode 1) skip the q rows and every output product.
-template <typename T, int D, bool OUT>
-__global__ void __launch_bounds__(128, 1) gdn_scan16_kernel(GdnArgs a) {
+// Segment summaries (seg_mode 1) of the split recurrence: the state a segment leaves from a zero entry state (columns
+// below D) and its transition matrix (columns from D, from the identity with v = 0).  Four waves of one workgroup, 16
+// of its 64 columns each, one per SIMD; LDS holds one workgroup per CU, so the workgroup's columns set how many segments
+// fill the device.  Bound by a wave's chain of products per chunk (its reads of the k rows and T fragments share the LDS
+// with the other waves'): 1.4 us a chunk at D = 128 where two waves of 32 columns took 1.2, and twice the segments, so
+// 20,000 tokens of 8 heads take summary + combine + replay 127 us, 157 with 32 columns.
+template <typename T, int D>
+__global__ void __launch_bounds__(256, 1) gdn_summary16_kernel(GdnArgs a) {
   constexpr int C = kChunk, KS = D / 32, ST = D / 16;
-  constexpr int CPR = D / 8;                    // 16-byte chunks per k / q row
-  constexpr int KB = C * D, VB = C * 32;        // elements of one slot's k (q) rows, v slab
+  constexpr int CPR = D / 8;                    // 16-byte chunks per k row
+  constexpr int KB = C * D, VB = C * 64;        // elements of one slot's k rows, v slab
   constexpr int RB = kGdn16RecBytes;            // bytes of one slot's record
-  constexpr int RPI = 64 / CPR;                 // k / q rows per copy instruction
-  constexpr int NKQ = 32 / RPI;                 // copy instructions per wave for its 32 k (q) rows
-  constexpr int NREC = (RB / 1024 + 1) / 2;     // record blocks per wave (wave 1 repeats its last)
-  constexpr int NDMA = 2 * NKQ + 2 + NREC;      // copies per wave per chunk
+  constexpr int RPI = 64 / CPR;                 // k rows per copy instruction
+  constexpr int NK = 16 / RPI;                  // copy instructions per wave for its 16 k rows
+  constexpr int NREC = (RB / 1024 + 3) / 4;     // record blocks per wave (wave 3 repeats the last)
+  constexpr int NDMA = NK + 2 + NREC;           // copies per wave per chunk
   static_assert(RB % 1024 == 0, "record of whole 1 KiB blocks");
   // three slots per array: chunk c lives in slot c % 3, so within the three-times unrolled
   // loop every slot offset is an instruction immediate
   __shared__ __attribute__((aligned(16))) T Ks[3 * KB];
-  __shared__ __attribute__((aligned(16))) T Qs[3 * KB];
   __shared__ __attribute__((aligned(16))) T Vs[3 * VB];
   __shared__ __attribute__((aligned(16))) char Rs[3 * RB];
 
-  if (a.seg_mode != 2) gdn_signal_start(a);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, c16 = lane & 15;
-  const int bh = blockIdx.x, b = bh / a.H, h = bh % a.H, hk = h / a.G;
-  const int vw = 32 * blockIdx.y;    // the workgroup's 32 state columns (>= D: a summary's transition)
+  const int bh = blockIdx.x, b = bh / a.H, hk = bh % a.H / a.G;
+  const int vw = 64 * blockIdx.y;    // the workgroup's 64 state columns (>= D: the transition)
   const int v0 = vw + 16 * wave;     // this wave's 16
   const int seg = blockIdx.z;
   const int c_begin = seg * a.seg_len, c_end = min(a.NC, c_begin + a.seg_len);
-  const bool summary = !OUT;             // no output; columns >= D carry the transition
-  const bool trans = summary && vw >= D;
+  const bool trans = vw >= D;
 
   // ---- state: tile t, register i <-> row k = 32 (t/2) + 8g + 4 (t%2) + i, column v0 + c16
   f32x4 S[ST];
@@ -362,71 +363,63 @@ __global__ void __launch_bounds__(128, 1) gdn_scan16_kernel(GdnArgs a) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int kx = 32 * (t >> 1) + 8 * g + 4 * (t & 1) + i;
-      float x;
-      if (a.seg_mode == 0) x = a.s0 ? a.s0[((int64_t)bh * D + kx) * D + v0 + c16] : 0.f;
-      else if (a.seg_mode == 2) x = a.seg_in[(((int64_t)bh * a.nseg + seg) * D + kx) * D + v0 + c16];
-      else x = (trans && kx == v0 + c16 - D) ? 1.f : 0.f;
-      S[t][i] = x;
+      S[t][i] = (trans && kx == v0 + c16 - D) ? 1.f : 0.f;
     }
 
   // ---- lane parts of the LDS addresses (elements; tile and slot offsets are immediates).
   // k rows use lds_swizzle, whose value for the rows a lane touches is fixed: A fragments
   // read row 16p + c16 (swizzle of c16), transposing reads row 32j + 4g + c16/4 (+16)
-  // (swizzle 4 (c16/4) + g); q rows use rec_swizzle (c16 for 256-byte rows).
+  // (swizzle 4 (c16/4) + g).
   const int ksw = lds_swizzle<CPR>(c16);
-  int kAo[KS], qBo[KS], kTo[KS];
+  int kAo[KS], kTo[KS];
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
     kAo[s] = c16 * D + 8 * ((4 * s + g) ^ ksw);
-    qBo[s] = c16 * D + 8 * ((4 * s + g) ^ rec_swizzle<CPR>(c16));
     // tile t = 2s (+1): lane supplies columns 32 s + 8 (c16 % 4) + 4 (t % 2) of row
     // 4g + c16/4 (+ 32j, + 16): chunk 4s + c16 % 4
     const int r0 = 4 * g + (c16 >> 2);
     kTo[s] = r0 * D + 8 * ((4 * s + (c16 & 3)) ^ lds_swizzle<CPR>(r0));
   }
-  const int vo = (4 * g + (c16 >> 2)) * 32 + 16 * wave + 4 * (c16 & 3);
+  // v slab rows of 128 bytes, 16-byte chunk c of row r at c ^ (r / 2 mod 8): the 16 rows a transposing read touches fall
+  // in distinct banks
+  const int vr0 = 4 * g + (c16 >> 2);
+  const int vo = vr0 * 64 + 8 * ((2 * wave + ((c16 & 3) >> 1)) ^ ((vr0 >> 1) & 7)) + 4 * (c16 & 1);
 
-  // ---- copies of chunk j into slot sl: wave w copies k and q rows 32w .. 32w + 31 (k with
-  // lds_swizzle, q with rec_swizzle), v slab rows 32w .. 32w + 31 (64 bytes each) and half
-  // of the record's 1 KiB blocks (with an odd count, wave 1 copies its last block twice so
-  // both waves issue the same number of copies).  Rows past T read as zeros.
-  const uint32_t kst2 = (uint32_t)a.k_st * 2u, qst2 = (uint32_t)a.q_st * 2u, vst2 = (uint32_t)a.v_st * 2u;
-  uint32_t kvo[NKQ], qvo[NKQ], vvo[2];
+  // ---- copies of chunk j into slot sl: wave w copies k and v slab rows 16w .. 16w + 15 (with their swizzles) and a
+  // quarter of the record's 1 KiB blocks (wave 3 copies the last one again, so that every wave issues the same number of
+  // copies).  Rows past T read as zeros.
+  const uint32_t kst2 = (uint32_t)a.k_st * 2u, vst2 = (uint32_t)a.v_st * 2u;
+  uint32_t kvo[NK], vvo[2];
 #pragma unroll
-  for (int r = 0; r < NKQ; ++r) {
-    const int row = 32 * wave + RPI * r + lane / CPR, pc = lane % CPR;
+  for (int r = 0; r < NK; ++r) {
+    const int row = 16 * wave + RPI * r + lane / CPR, pc = lane % CPR;
     kvo[r] = row * kst2 + 16u * (pc ^ lds_swizzle<CPR>(row));
-    qvo[r] = row * qst2 + 16u * (pc ^ rec_swizzle<CPR>(row));
   }
 #pragma unroll
-  for (int r = 0; r < 2; ++r) vvo[r] = (32 * wave + 16 * r + lane / 4) * vst2 + 16u * (lane % 4);
+  for (int r = 0; r < 2; ++r) {
+    const int row = 16 * wave + 8 * r + lane / 8;
+    vvo[r] = row * vst2 + 16u * ((lane % 8) ^ ((row >> 1) & 7));
+  }
   const uint32_t rvo = 16u * lane;  // record blocks: the block offset is a scalar (always in range)
   const T* kb = (const T*)a.k + b * a.k_sb + hk * a.k_sh;
-  const T* qb = (const T*)a.q + b * a.q_sb + h * a.q_sh;
   const T* vb = (const T*)a.v + b * a.v_sb + hk * a.v_sh + (trans ? 0 : vw);
   const char* rb0 = (const char*)a.ws + (int64_t)bh * a.NC * RB;
   const int last = c_end - 1;
   // LDS byte offsets of this wave's copy destinations, in scalar registers
-  const uint32_t mk = __builtin_amdgcn_readfirstlane(lds_offset(Ks + 32 * wave * D));
-  const uint32_t mq = __builtin_amdgcn_readfirstlane(lds_offset(Qs + 32 * wave * D));
-  const uint32_t mv = __builtin_amdgcn_readfirstlane(lds_offset(Vs + 32 * wave * 32));
+  const uint32_t mk = __builtin_amdgcn_readfirstlane(lds_offset(Ks + 16 * wave * D));
+  const uint32_t mv = __builtin_amdgcn_readfirstlane(lds_offset(Vs + 16 * wave * 64));
   const uint32_t mr = __builtin_amdgcn_readfirstlane(lds_offset(Rs));
   auto copy_chunk = [&](int j, auto slot_c) {
     constexpr int sl = decltype(slot_c)::value;
     const int rows = min(a.T - j * C, C);
     const auto krs = buffer_rsrc(kb + (int64_t)j * C * a.k_st, (uint32_t)((rows - 1) * a.k_st + D) * 2u);
-    // (a summary reads no q rows, and its transition columns take v = 0: empty ranges, so
-    // the copies only write zeros)
-    const auto qrs = buffer_rsrc(qb + (int64_t)j * C * a.q_st, summary ? 0u : (uint32_t)((rows - 1) * a.q_st + D) * 2u);
-    const auto vrs = buffer_rsrc(vb + (int64_t)j * C * a.v_st, trans ? 0u : (uint32_t)((rows - 1) * a.v_st + 32) * 2u);
+    // (transition columns take v = 0: an empty range, so that the copies only write zeros)
+    const auto vrs = buffer_rsrc(vb + (int64_t)j * C * a.v_st, trans ? 0u : (uint32_t)((rows - 1) * a.v_st + 64) * 2u);
     const auto rrs = buffer_rsrc(rb0 + (int64_t)j * RB, RB);
 #pragma unroll
-    for (int r = 0; r < NKQ; ++r) {
-      dma_buf16_at(krs, kvo[r], 0, mk + (sl * KB + RPI * r * D) * 2);
-      dma_buf16_at(qrs, qvo[r], 0, mq + (sl * KB + RPI * r * D) * 2);
-    }
+    for (int r = 0; r < NK; ++r) dma_buf16_at(krs, kvo[r], 0, mk + (sl * KB + RPI * r * D) * 2);
 #pragma unroll
-    for (int r = 0; r < 2; ++r) dma_buf16_at(vrs, vvo[r], 0, mv + (sl * VB + 16 * r * 32) * 2);
+    for (int r = 0; r < 2; ++r) dma_buf16_at(vrs, vvo[r], 0, mv + (sl * VB + 8 * r * 64) * 2);
 #pragma unroll
     for (int r = 0; r < NREC; ++r) {
       const uint32_t blk = (uint32_t)min(NREC * wave + r, RB / 1024 - 1) * 1024u;
@@ -434,25 +427,18 @@ __global__ void __launch_bounds__(128, 1) gdn_scan16_kernel(GdnArgs a) {
     }
   };
 
-  // this sequence's output rows as one buffer: rows past T are dropped
-  const auto orsrc = buffer_rsrc((const T*)a.o + (int64_t)b * a.T * a.H * D, (uint32_t)((int64_t)a.T * a.H * D * 2));
-  const uint32_t oo = (uint32_t)((c16 * a.H + h) * D + v0 + 4 * g) * 2u;  // lane part of the output offset
-  const uint32_t otok = (uint32_t)a.H * D * 2u;                          // bytes per token
-
   auto body = [&](int c, auto slot_c) {
     constexpr int sl = decltype(slot_c)::value;
     // this wave's copies of chunk c have landed (only those of chunk c + 1 may be in
-    // flight: loads complete in order, and stores are not counted), then the other's
+    // flight: loads complete in order), then the others'
     wait_vmcnt<NDMA>();
     __syncthreads();
 
     const T* Kl = Ks + sl * KB;
-    const T* Ql = Qs + sl * KB;
     const T* Vl = Vs + sl * VB;
     const char* Rl = Rs + sl * RB;
     const float* Fp = (const float*)(Rl + kGdn16F);
     const u32x4* Tb = (const u32x4*)(Rl + kGdn16Tb);
-    const u32x4* Rb = (const u32x4*)(Rl + kGdn16Rb);
 
     // The LDS reads of each phase are issued before its first product and the scheduling
     // barriers keep that order (one wave per SIMD: no other wave hides a read's latency).
@@ -488,31 +474,20 @@ __global__ void __launch_bounds__(128, 1) gdn_scan16_kernel(GdnArgs a) {
       __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
-    // chunk c + 2 goes to the slot chunk c - 1 used (both waves are past the barrier above);
+    // chunk c + 2 goes to the slot chunk c - 1 used (every wave is past the barrier above);
     // issued here, behind the products, so the copies' issue does not delay them.  Past the
     // last chunk the copies repeat it, so every step issues the same count.
     copy_chunk(min(c + 2, last), std::integral_constant<int, (sl + 2) % 3>{});
 
-    // (3) reads: q rows as B fragments of S^T Q^T (tile p': row 16p' + c16) and geqs of the
-    // lane's tokens; for X and U, v by transposing reads of the slab (lane c16 supplies row
-    // r0 + c16 / 4, columns 16 wave + 4 (c16 % 4)) in the token slot order
-    // 32j + 4g + [0,4), 32j + 16 + 4g + [0,4), geik of the same tokens, T diag(beta)
-    u32x4 qB[4][KS];
-    float wq[4];
-    if constexpr (OUT) {
-#pragma unroll
-      for (int p = 0; p < 4; ++p) {
-#pragma unroll
-        for (int s = 0; s < KS; ++s) qB[p][s] = lds16(Ql + 16 * p * D + qBo[s]);
-        wq[p] = Fp[128 + 16 * p + c16];
-      }
-    }
+    // (3) reads for X and U: v by transposing reads of the slab (lane c16 supplies row r0 + c16 / 4, columns
+    // 16 wave + 4 (c16 % 4)) in the token slot order 32j + 4g + [0,4), 32j + 16 + 4g + [0,4), geik of the same tokens,
+    // T diag(beta)
     u32x2 vlo[2], vhi[2];
     f32x4 wl[2], wh[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      vlo[j] = lds_read_tr16(Vl + 32 * j * 32 + vo);
-      vhi[j] = lds_read_tr16(Vl + (32 * j + 16) * 32 + vo);
+      vlo[j] = lds_read_tr16(Vl + 32 * j * 64 + vo);
+      vhi[j] = lds_read_tr16(Vl + (32 * j + 16) * 64 + vo);
       wl[j] = *(const f32x4*)(Fp + 64 + 32 * j + 4 * g);
       wh[j] = *(const f32x4*)(Fp + 64 + 32 * j + 16 + 4 * g);
     }
@@ -521,18 +496,7 @@ __global__ void __launch_bounds__(128, 1) gdn_scan16_kernel(GdnArgs a) {
     for (int f = 0; f < 6; ++f) tb[f] = Tb[f * 64 + lane];
     __builtin_amdgcn_sched_barrier(0);
 
-    // (4) output, first term: O^T tile p' (rows = columns v0 + 4g + i, cols = tokens
-    // 16p' + c16) = S^T Q^T, scaled by geqs of the token; with it X = V - geik K S as B
-    // fragments over token steps j
-    f32x4 o[4];
-    if constexpr (OUT) {
-#pragma unroll
-      for (int pp = 0; pp < 4; ++pp) o[pp] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s = 0; s < KS; ++s)
-#pragma unroll
-        for (int pp = 0; pp < 4; ++pp) o[pp] = mfma16x16x32<T>(sf[s], qB[pp][s], o[pp]);
-    }
+    // (4) X = V - geik K S as B fragments over token steps j
     u32x4 xf[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -544,17 +508,12 @@ __global__ void __launch_bounds__(128, 1) gdn_scan16_kernel(GdnArgs a) {
       }
       xf[j] = pack8<T>(xl, xh);
     }
-#pragma unroll
-    for (int i = 0; i < 4 * KS; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);
-      __builtin_amdgcn_sched_group_barrier(0x002, 3, 1);
-    }
     __builtin_amdgcn_sched_barrier(0);
 
-    // (5) reads for the state update and the output's second term: A fragments of K^T by
+    // (5) reads for the state update: A fragments of K^T by
     // transposing reads (for tile t, lane c16 supplies row r0 + c16 / 4 and the 4 columns
     // 32 (t/2) + 8 (c16 % 4) + 4 (t%2) .., so lane r receives column 32 (t/2) + 8 (r/4) +
-    // 4 (t%2) + r % 4, the state row of tile t); Rq fragments; kf of the token slots
+    // 4 (t%2) + r % 4, the state row of tile t); kf of the token slots
     u32x4 kT[2][ST];
 #pragma unroll
     for (int j = 0; j < 2; ++j)
@@ -565,11 +524,6 @@ __global__ void __launch_bounds__(128, 1) gdn_scan16_kernel(GdnArgs a) {
         const u32x2 hi = lds_read_tr16(pl + 16 * D);
         kT[j][t] = u32x4{lo[0], lo[1], hi[0], hi[1]};
       }
-    u32x4 rq[6];
-    if constexpr (OUT) {
-#pragma unroll
-      for (int f = 0; f < 6; ++f) rq[f] = Rb[f * 64 + lane];
-    }
     f32x4 kl[2], kh[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -578,9 +532,8 @@ __global__ void __launch_bounds__(128, 1) gdn_scan16_kernel(GdnArgs a) {
     }
     __builtin_amdgcn_sched_barrier(0);
 
-    // (6) U = T diag(beta) X: tile P = tokens 16P + 4g + i (T is lower triangular); U as
-    // fragments in the token slot order, plain (U^T A fragments of the output) and weighted
-    // by kf (B fragments of the update)
+    // (6) U = T diag(beta) X: tile P = tokens 16P + 4g + i (T is lower triangular); U as B fragments of the update in
+    // the token slot order, weighted by kf
     const f32x4 z = {0.f, 0.f, 0.f, 0.f};
     f32x4 U[4];
     U[0] = mfma16x16x32<T>(tb[0], xf[0], z);
@@ -589,31 +542,13 @@ __global__ void __launch_bounds__(128, 1) gdn_scan16_kernel(GdnArgs a) {
     U[3] = mfma16x16x32<T>(tb[4], xf[0], z);
     U[2] = mfma16x16x32<T>(tb[3], xf[1], U[2]);
     U[3] = mfma16x16x32<T>(tb[5], xf[1], U[3]);
-    u32x4 uf[2], ukf[2];
+    u32x4 ukf[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      uf[j] = pack8<T>(U[2 * j], U[2 * j + 1]);
       ukf[j] = pack8<T>(U[2 * j] * kl[j], U[2 * j + 1] * kh[j]);
     }
 
-    // (7) output second term + U^T Rq^T and the 8-byte row pieces O[token][v0 + 4g ..] (stored
-    // before the update's products, so they complete before the next chunk's copy wait), then
-    // S += K^T diag(kf) U
-    if constexpr (OUT) {
-#pragma unroll
-      for (int pp = 0; pp < 4; ++pp) {
-        f32x4 x = o[pp] * wq[pp];
-        if (pp < 2) {
-          x = mfma16x16x32<T>(uf[0], rq[pp], x);
-        } else {
-          x = mfma16x16x32<T>(uf[0], rq[2 * pp - 2], x);
-          x = mfma16x16x32<T>(uf[1], rq[2 * pp - 1], x);
-        }
-        const u32x2 pk = {pack2<T>(x[0], x[1]), pack2<T>(x[2], x[3])};
-        // (the whole offset in the lane's voffset: only that part is range-checked)
-        __builtin_amdgcn_raw_buffer_store_b64(pk, orsrc, oo + (uint32_t)(c * C + 16 * pp) * otok, 0, 0);
-      }
-    }
+    // (7) S += K^T diag(kf) U
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -631,23 +566,14 @@ __global__ void __launch_bounds__(128, 1) gdn_scan16_kernel(GdnArgs a) {
     if (c + 2 < c_end) body(c + 2, S2{});
   }
 
-  float* sdst = nullptr;  // the exit state: [k][col] rows of D (2D for a summary) floats
-  int64_t sld = D;
-  if (a.seg_mode == 1) {
-    sdst = a.seg_sum + ((int64_t)bh * a.nseg + seg) * D * 2 * D;
-    sld = 2 * D;
-  } else if (seg == a.nseg - 1 && a.s_out) {
-    sdst = a.s_out + (int64_t)bh * D * D;
-  }
-  if (sdst) {
+  float* sdst = a.seg_sum + ((int64_t)bh * (a.nseg - 1) + seg) * D * 2 * D;  // the exit state: [k][2D columns]
 #pragma unroll
-    for (int t = 0; t < ST; ++t)
+  for (int t = 0; t < ST; ++t)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int kx = 32 * (t >> 1) + 8 * g + 4 * (t & 1) + i;
-        sdst[kx * sld + v0 + c16] = S[t][i];
-      }
-  }
+    for (int i = 0; i < 4; ++i) {
+      const int kx = 32 * (t >> 1) + 8 * g + 4 * (t & 1) + i;
+      sdst[kx * 2 * D + v0 + c16] = S[t][i];
+    }
   // the copies issued past the last chunk land before the workgroup's LDS is released
   wait_vmcnt<0>();
 }
@@ -692,6 +618,10 @@ __global__ void __launch_bounds__(256, 1) gdn_scan16_pair_kernel(GdnArgs a) {
   const int seg = blockIdx.z;
   const int c_begin = seg * a.seg_len, c_end = min(a.NC, c_begin + a.seg_len);
 
+  // a replay's entry state: segment 0's, or the one over the previous segment's summary
+  const float* seg_in = seg ? a.seg_sum + ((int64_t)bh * (a.nseg - 1) + seg - 1) * D * 2 * D : a.seg_in + (int64_t)bh * D * D;
+  const int sld = seg ? 2 * D : D;
+
   // ---- chain: state tile t, register i <-> row k = 32 (t/2) + 8g + 4 (t%2) + i, column v0 + c16
   f32x4 S[ST];
   u32x4 sf[KS];
@@ -703,7 +633,7 @@ __global__ void __launch_bounds__(256, 1) gdn_scan16_pair_kernel(GdnArgs a) {
         const int kx = 32 * (t >> 1) + 8 * g + 4 * (t & 1) + i;
         float x;
         if (a.seg_mode == 0) x = a.s0 ? a.s0[((int64_t)bh * D + kx) * D + v0 + c16] : 0.f;
-        else x = a.seg_in[(((int64_t)bh * a.nseg + seg) * D + kx) * D + v0 + c16];
+        else x = seg_in[kx * sld + v0 + c16];
         S[t][i] = x;
       }
 #pragma unroll
@@ -714,7 +644,7 @@ __global__ void __launch_bounds__(256, 1) gdn_scan16_pair_kernel(GdnArgs a) {
   }
 
   // ---- lane parts of the LDS addresses (elements; tile and slot offsets are immediates),
-  // as in gdn_scan16_kernel
+  // as in gdn_summary16_kernel
   const int ksw = lds_swizzle<CPR>(c16);
   int kAo[KS], qBo[KS], kTo[KS];
 #pragma unroll
@@ -968,13 +898,13 @@ __global__ void __launch_bounds__(256, 1) gdn_scan16_pair_kernel(GdnArgs a) {
   wait_vmcnt<0>();
 }
 
-// Entry states of the segments from their summaries (fp32): seg_in[0] = s0 (or 0) and
-// seg_in[s] = M_{s-1} seg_in[s-1] + B_{s-1}, where summary s - 1 holds [B | M] row by row.
+// Entry states of the segments from their summaries (fp32): E_0 = s0 (or 0) and E_s = M_{s-1} E_{s-1} + B_{s-1}, where
+// summary s - 1 holds [B | M] row by row.  E_s goes over B_{s-1}, whose columns only this workgroup reads.
 // One workgroup of four waves per (sequence-head, 16 state columns), a wave D / 4 rows of the product on
-// v_mfma_f32_16x16x4f32 with the k index permuted (step i contracts k = D/4 g + i), so that a lane's operand of M is
-// D / 4 consecutive floats.  The chain is one product per segment: M and B of the next one are loaded under it, and the
-// state passes between the waves through LDS.  Bound by latency, one load and one chain of D / 8 dependent
-// products a segment: 20,000 tokens of 4 heads 13.8 us, 85 us with the products on VALU and M staged through LDS.
+// v_mfma_f32_16x16x4f32 with the k index permuted (step 4 j + e contracts k = 16 j + 4 g + e), so that the four lanes
+// of a row load 64 consecutive bytes of M.  The chain is one product per segment: M and B are loaded two segments ahead, and the state
+// passes between the waves through LDS.  Bound by latency, about 2.8 us a segment (its D / 8 dependent products take 1):
+// 20,000 tokens of 8 heads in 5 segments 13.8 us, 85 us with the products on VALU and M staged through LDS.
 template <int D>
 __global__ void __launch_bounds__(256) gdn_seg_combine_kernel(GdnArgs a) {
   constexpr int RT = D / 64, KL = D / 4;  // 16-row tiles per wave; k values per lane
@@ -990,53 +920,58 @@ __global__ void __launch_bounds__(256) gdn_seg_combine_kernel(GdnArgs a) {
       const int row = 16 * (RT * wave + t) + 4 * g + i;
       S[t][i] = s0 ? s0[row * D + j0 + c] : 0.f;
     }
-  f32x4 m[RT][KL / 4], B[RT];
-  auto load = [&](int sg) {
-    const float* sum = a.seg_sum + ((int64_t)bh * a.nseg + sg) * D * 2 * D;
+  f32x4 m[2][RT][KL / 4], B[2][RT];  // of summary sg in slot sg % 2, loaded two steps ahead
+  auto load = [&](int sg, auto slot_c) {
+    constexpr int sl = decltype(slot_c)::value;
+    const float* sum = a.seg_sum + ((int64_t)bh * (a.nseg - 1) + sg) * D * 2 * D;
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
-      const float* mr = sum + (16 * (RT * wave + t) + c) * 2 * D + D + KL * g;
+      const float* mr = sum + (16 * (RT * wave + t) + c) * 2 * D + D + 4 * g;
 #pragma unroll
-      for (int i = 0; i < KL / 4; ++i) m[t][i] = *(const f32x4*)(mr + 4 * i);
+      for (int i = 0; i < KL / 4; ++i) m[sl][t][i] = *(const f32x4*)(mr + 16 * i);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) B[t][i] = sum[(16 * (RT * wave + t) + 4 * g + i) * 2 * D + j0 + c];
+      for (int i = 0; i < 4; ++i) B[sl][t][i] = sum[(16 * (RT * wave + t) + 4 * g + i) * 2 * D + j0 + c];
     }
   };
-  load(0);
-  for (int sg = 0; sg < a.nseg; ++sg) {
-    float* in = a.seg_in + ((int64_t)bh * a.nseg + sg) * D * D + j0 + c;
+  auto step = [&](int sg, auto slot_c) {
+    constexpr int sl = decltype(slot_c)::value;
+    float* in = j0 + c + (sg ? a.seg_sum + ((int64_t)bh * (a.nseg - 1) + sg - 1) * D * 2 * D : a.seg_in + (int64_t)bh * D * D);
+    const int ld = sg ? 2 * D : D;
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
       const int r0 = 16 * (RT * wave + t) + 4 * g;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) in[(r0 + i) * D] = S[t][i];
-      *(f32x4*)&cur[sg & 1][c][r0] = S[t];
+      for (int i = 0; i < 4; ++i) in[(r0 + i) * ld] = S[t][i];
+      *(f32x4*)&cur[sl][c][r0] = S[t];
     }
-    if (sg + 1 == a.nseg) break;
+    if (sg + 1 == a.nseg) return;
     __syncthreads();  // (the other buffer's readers are past the previous step's barrier)
     f32x4 acc[RT][2];
-    float mm[RT][KL], bb[KL];
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
-      acc[t][0] = B[t];
+      acc[t][0] = B[sl][t];
       acc[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int i = 0; i < KL; ++i) mm[t][i] = m[t][i >> 2][i & 3];
     }
-    if (sg + 2 < a.nseg) load(sg + 1);
 #pragma unroll
     for (int i = 0; i < KL / 4; ++i) {
-      const f32x4 v = *(const f32x4*)&cur[sg & 1][c][KL * g + 4 * i];
+      const f32x4 v = *(const f32x4*)&cur[sl][c][16 * i + 4 * g];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) bb[4 * i + e] = v[e];
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+          acc[t][e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(m[sl][t][i][e], v[e], acc[t][e & 1], 0, 0, 0);
     }
-#pragma unroll
-    for (int i = 0; i < KL; ++i)
-#pragma unroll
-      for (int t = 0; t < RT; ++t)
-        acc[t][i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(mm[t][i], bb[i], acc[t][i & 1], 0, 0, 0);
+    if (sg + 3 < a.nseg) load(sg + 2, slot_c);
 #pragma unroll
     for (int t = 0; t < RT; ++t) S[t] = acc[t][0] + acc[t][1];
+  };
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, 1>;
+  load(0, S0{});
+  if (a.nseg > 2) load(1, S1{});
+  for (int sg = 0; sg < a.nseg; sg += 2) {
+    step(sg, S0{});
+    if (sg + 1 < a.nseg) step(sg + 1, S1{});
   }
 }
 
@@ -1047,17 +982,18 @@ __global__ void __launch_bounds__(256) gdn_seg_combine_kernel(GdnArgs a) {
 // from the device's CU count and never under graph capture or autograd) takes the plain
 // scan, and the plain and segmented scans differ in rounding only (the segment entry
 // states are combined in fp32; agreement at 1e-2 of the output is tested at T = 65,536).
-static void gdn16_plan(int64_t BH, int NC, int D, int& nseg, int& seg_len) {
-  nseg = gdn16_segments(BH, NC, D, 256);
+static int64_t gdn16_plan(int64_t BH, int NC, int D, int& nseg, int& seg_len) {
+  int64_t states;  // of scratch per sequence-head
+  nseg = gdn16_segments(BH, NC, D, 256, states);
   seg_len = (NC + nseg - 1) / nseg;
   nseg = (NC + seg_len - 1) / seg_len;
+  return states;
 }
 
 size_t gdn16_workspace_bytes(int64_t BH, int64_t NC, int D) {
   int nseg, seg_len;
-  gdn16_plan(BH, (int)NC, D, nseg, seg_len);
-  const size_t recs = (size_t)(BH * NC) * (size_t)kGdn16RecBytes;
-  return nseg == 1 ? recs : recs + (size_t)BH * nseg * D * 3 * D * sizeof(float);
+  const int64_t states = gdn16_plan(BH, (int)NC, D, nseg, seg_len);
+  return (size_t)(BH * NC) * (size_t)kGdn16RecBytes + (size_t)(BH * states * D * D) * sizeof(float);
 }
 
 template <typename T, int D>
@@ -1082,9 +1018,9 @@ static int launch16(const GdnArgs& a0, hipStream_t s) {
   }
   // long sequences with few heads: segment summaries, their entry states, then the replays
   a.seg_sum = (float*)((char*)a.ws + (size_t)items * kGdn16RecBytes);
-  a.seg_in = a.seg_sum + BH * a.nseg * D * 2 * D;
+  a.seg_in = a.seg_sum + BH * (a.nseg - 1) * D * 2 * D;
   a.seg_mode = 1;
-  gdn_scan16_kernel<T, D, false><<<dim3((unsigned)BH, 2 * D / 32, a.nseg - 1), dim3(128), 0, s>>>(a);
+  gdn_summary16_kernel<T, D><<<dim3((unsigned)BH, 2 * D / 64, a.nseg - 1), dim3(256), 0, s>>>(a);
   rc = check_launch("chunk_gated_delta_rule(summary16)");
   if (rc) return rc;
   gdn_seg_combine_kernel<D><<<dim3((unsigned)BH, D / 16), dim3(256), 0, s>>>(a);

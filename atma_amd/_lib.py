@@ -108,6 +108,10 @@ SIGNATURES = {
         _p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64,
         _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i32, _f32, _i32, _i32, _f32, _f32,
         _i64, _p, _sz, _p, _i32, _p]),
+    "atma_gated_delta_prefill_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _p]),
+    "atma_gated_delta_prefill": (_i32, [
+        _p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _p, _p, _p, _i64, _p, _i64, _i64, _p,
+        _i64, _i64, _i64, _i32, _f32, _i32, _i32, _f32, _f32, _p, _sz, _p, _i32, _p]),
     "atma_wait_start_flag": (_i32, [_p, _i32, _i64, _p]),
 }
 

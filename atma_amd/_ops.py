@@ -10,6 +10,8 @@ implementation: a CPU tensor raises, and a missing library raises
 
 from typing import List, Optional
 
+import ctypes
+
 import torch
 from torch import Tensor
 
@@ -744,6 +746,33 @@ def _(q, k, v, g, beta, initial_state, scale, use_qk_l2norm, want_final, start_f
     dv = v.shape[3]
     o = q.new_empty((B, T, H, dv))
     return [o, q.new_empty((B, H, dk, dv), dtype=torch.float32)] if want_final else [o]
+
+
+@torch.library.custom_op("atma_hip::gated_delta_prefill", mutates_args=("state_table", "o", "start_flag"))
+def gated_delta_prefill_op(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, state_table: Tensor,
+                           slots: Tensor, o: Tensor, seq_lens: Optional[List[int]], g_bias: float, b_bias: float,
+                           start_flag: Optional[Tensor], start_epoch: int) -> None:
+    """Prefill recurrence from and to rows of a state table, ragged with ``seq_lens``."""
+    _need_cuda(q, k, v, g, beta, state_table, slots, o)
+    lib = _lib.load()
+    q, k, v = _rows16(q), _rows16(k), _rows16(v)
+    B, T, H, d = q.shape
+    lens = None if seq_lens is None else (ctypes.c_int64 * len(seq_lens))(*seq_lens)
+    n = B if lens is None else len(lens)
+    lp = None if lens is None else ctypes.addressof(lens)
+    ws_bytes = lib.atma_gated_delta_prefill_workspace_bytes(n, T, H, d, lp)
+    ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8)
+    rc = lib.atma_gated_delta_prefill(
+        q.data_ptr(), *q.stride()[:3], k.data_ptr(), *k.stride()[:3], v.data_ptr(), *v.stride()[:3], g.data_ptr(),
+        beta.data_ptr(), state_table.data_ptr(), slots.data_ptr(), state_table.shape[0], o.data_ptr(), n, T, lp, H,
+        k.shape[2], d, _lib.dtype_code(q.dtype), 1.0, 1, 1, g_bias, b_bias, ws.data_ptr(), ws_bytes,
+        _lib.ptr(start_flag), start_epoch, _lib.stream_handle(q.device))
+    _lib.check(rc, "gated_delta_prefill")
+
+
+@gated_delta_prefill_op.register_fake
+def _(q, k, v, g, beta, state_table, slots, o, seq_lens, g_bias, b_bias, start_flag, start_epoch):
+    return None
 
 
 @torch.library.custom_op("atma_hip::wait_start_flag", mutates_args=("flag",))

@@ -38,7 +38,48 @@ struct GdnArgs {
   int seg_len, nseg, seg_mode;
   float* seg_sum;  // [B*H][nseg - 1][D][2D] fp32: the summaries; then segment s + 1's entry state over the B half of s
   float* seg_in;   // [B*H][D][D] fp32: segment 0's entry state (s0 may be s_out)
+  // 16-bit path: s0 and s_out are rows of a state table, sequence b's at row slots[b] (negative: from the end;
+  // a row outside the table reads as zeros and is not written); null: one state per sequence in order
+  const int64_t* slots;
+  int64_t num_slots;
 };
+
+// The state of sequence b, head h under `base` (s0 or s_out); null: none.
+__device__ __forceinline__ float* gdn_state(const GdnArgs& a, const float* base, int b, int h, int D) {
+  if (!base) return nullptr;
+  int row = b;
+  if (a.slots) {
+    int64_t i = a.slots[b];
+    if (i < 0) i += a.num_slots;
+    if (i < 0 || i >= a.num_slots) return nullptr;
+    row = __builtin_amdgcn_readfirstlane((int)i);
+  }
+  return const_cast<float*>(base) + ((int64_t)row * a.H + h) * D * D;
+}
+
+// Which tokens a sequence of the launch has.  Dense: B sequences of T tokens.  Packed: up to kVarSeqs ragged sequences of
+// one packed token axis (batch stride unused), passed by value in the kernel arguments (no upload, graph capturable),
+// the longest first so that the recurrence's workgroups start in that order.
+constexpr int kVarSeqs = 64;
+struct DenseSeqs {};
+struct VarSeqs {
+  int n;
+  int start[kVarSeqs], len[kVarSeqs];  // tokens
+  int chunk0[kVarSeqs];                // chunks of the sequences before
+  int row[kVarSeqs];                   // index into slots
+};
+struct SeqView {
+  int64_t tok0, qo, ko, vo;  // first token (g, beta, o); element offsets of its q, k, v
+  int T, NC, row;
+  int64_t chunk0;  // records of one head before this sequence's
+};
+__device__ __forceinline__ SeqView gdn_seq(const GdnArgs& a, const DenseSeqs&, int b) {
+  return SeqView{(int64_t)b * a.T, b * a.q_sb, b * a.k_sb, b * a.v_sb, a.T, a.NC, b, (int64_t)b * a.NC};
+}
+__device__ __forceinline__ SeqView gdn_seq(const GdnArgs& a, const VarSeqs& v, int b) {
+  const int64_t t = v.start[b];
+  return SeqView{t, t * a.q_st, t * a.k_st, t * a.v_st, v.len[b], (v.len[b] + 63) / 64, v.row[b], v.chunk0[b]};
+}
 
 // Segments of the 16-bit recurrence for B*H sequence-heads of NC chunks at head dim D on a device with `cus` compute
 // units; `states` = the D x D states of scratch per sequence-head.  The summaries and the replays cost the same per chunk
@@ -89,7 +130,7 @@ __device__ __forceinline__ float gdn_load_beta(const GdnArgs& a, int64_t i) {
 }
 
 // Workspace of the 16-bit path: one record of kGdn16RecBytes per (sequence, head, chunk)
-// item, item = (b * H + h) * NC + chunk, written by the prep kernel and copied whole into
+// item, item = (chunks before b) * H + h * NC + chunk, written by the prep kernel and copied whole into
 // LDS by the scan.  With C = 64 tokens, T = (I + A)^-1, A[p,s] = beta_p exp(lg_p - lg_s)
 // kn_p . kn_s (s < p) and Rq[p,s] = exp(lg_p - lg_s) qn_p . kn_s (s <= p):
 //   Tb  [6][64 lanes][8]  T diag(beta), lower 16 x 32 blocks as MFMA A fragments: fragment
@@ -105,7 +146,7 @@ __device__ __forceinline__ float gdn_load_beta(const GdnArgs& a, int64_t i) {
 // inclusive log-decays (13 KiB in all).
 constexpr int kGdn16Tb = 0, kGdn16Rb = 6144, kGdn16F = 12288, kGdn16RecBytes = 13312;
 
-int launch_gdn16(const GdnArgs& a, int dtype, int D, hipStream_t stream);
+int launch_gdn16(const GdnArgs& a, const VarSeqs* seqs, int dtype, int D, hipStream_t stream);
 // Workspace of the 16-bit path: the records, plus the segment summaries and entry states
 // when the launch splits the recurrence into segments.
 size_t gdn16_workspace_bytes(int64_t BH, int64_t NC, int D);

@@ -19,6 +19,8 @@
 // chunks in order, parallel over (sequence, head) x 16-column slabs of S (the
 // state columns are independent), with the slab resident in LDS for the whole
 // sequence.  All arithmetic is fp32.
+#include <algorithm>
+
 #include "gated_delta.h"
 
 namespace atma {
@@ -388,8 +390,137 @@ extern "C" int atma_chunk_gated_delta_rule(
   a.gate_logits = gate_logits ? 1 : 0; a.g_bias = g_bias; a.b_bias = b_bias;
   a.start_flag = start_flag; a.start_epoch = start_epoch;
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == ATMA_BF16 || dtype == ATMA_F16) return launch_gdn16(a, dtype, (int)dk, s);
+  if (dtype == ATMA_BF16 || dtype == ATMA_F16) return launch_gdn16(a, nullptr, dtype, (int)dk, s);
   return dk == 128 ? launch_gdn<float, 128>(a, s) : launch_gdn<float, 64>(a, s);
+}
+
+namespace atma {
+// A ragged launch scans every sequence plainly, so its longest one sets the time.  Sequences long enough to split (64
+// chunks; one of 4,096 tokens and 8 heads then takes about half the time, two of them in turn already as long as one
+// plain launch of both) are split one after another where that takes less: all their halves against the longest.
+static bool gdn_long(int64_t H, int64_t d, int64_t T) {
+  const int64_t chunks = (T + kChunk - 1) / kChunk;
+  int64_t states;
+  return chunks >= 64 && gdn16_segments(H, chunks, (int)d, 256, states) >= 4;
+}
+static bool gdn_split_long(int64_t B, int64_t H, int64_t d, const int64_t* seq_lens) {
+  int64_t longest = 0, sum = 0;
+  for (int64_t b = 0; b < B; ++b)
+    if (gdn_long(H, d, seq_lens[b])) {
+      longest = std::max(longest, seq_lens[b]);
+      sum += seq_lens[b];
+    }
+  return sum > 0 && sum < 2 * longest;
+}
+}  // namespace atma
+
+extern "C" size_t atma_gated_delta_prefill_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t d,
+                                                           const int64_t* seq_lens) {
+  using namespace atma;
+  if (B <= 0 || H <= 0 || (d != 64 && d != 128)) return 0;
+  if (!seq_lens) return T > 0 ? gdn16_workspace_bytes(B * H, (T + kChunk - 1) / kChunk, (int)d) : 0;
+  int64_t most = 0;  // the launches of kVarSeqs sequences follow each other in the same workspace
+  for (int64_t b0 = 0; b0 < B; b0 += kVarSeqs) {
+    int64_t chunks = 0;
+    for (int64_t b = b0; b < B && b < b0 + kVarSeqs; ++b) chunks += seq_lens[b] > 0 ? (seq_lens[b] + kChunk - 1) / kChunk : 0;
+    most = std::max(most, chunks);
+  }
+  size_t bytes = (size_t)(most * H) * (size_t)kGdn16RecBytes;
+  if (gdn_split_long(B, H, d, seq_lens))
+    for (int64_t b = 0; b < B; ++b)
+      if (gdn_long(H, d, seq_lens[b]))
+        bytes = std::max(bytes, gdn16_workspace_bytes(H, (seq_lens[b] + kChunk - 1) / kChunk, (int)d));
+  return bytes;
+}
+
+extern "C" int atma_gated_delta_prefill(
+    const void* q, int64_t q_sb, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sb, int64_t k_st, int64_t k_sh,
+    const void* v, int64_t v_sb, int64_t v_st, int64_t v_sh, const float* g, const float* beta, float* state_table,
+    const int64_t* slots, int64_t num_slots, void* o, int64_t B, int64_t T, const int64_t* seq_lens, int64_t H,
+    int64_t Hkv, int64_t d, int dtype, float scale, int use_qk_l2norm, int gate_logits, float g_bias, float b_bias,
+    void* workspace, size_t workspace_bytes, int32_t* start_flag, int32_t start_epoch, void* stream) {
+  using namespace atma;
+  if (dtype != ATMA_BF16 && dtype != ATMA_F16)
+    return set_error(ATMA_ERR_UNSUPPORTED, "gated_delta_prefill: 16-bit rows only (dtype %d)", dtype);
+  if (d != 64 && d != 128) return set_error(ATMA_ERR_UNSUPPORTED, "gated_delta_prefill: d 64 or 128");
+  if (B < 0 || H <= 0 || Hkv <= 0 || H % Hkv || num_slots < 0 || num_slots > 0x7fffffff || (!seq_lens && T < 1) ||
+      B * H > 0x7fffffff)
+    return set_error(ATMA_ERR_INVALID, "gated_delta_prefill: bad sizes");
+  if (B == 0) return ATMA_OK;
+  if (!q || !k || !v || !g || !beta || !state_table || !slots || !o)
+    return set_error(ATMA_ERR_INVALID, "gated_delta_prefill: null pointer");
+  if (q_st >= (1 << 24) || k_st >= (1 << 24) || v_st >= (1 << 24) || q_st < d || k_st < d || v_st < d)
+    return set_error(ATMA_ERR_UNSUPPORTED, "gated_delta_prefill: q/k/v token stride out of range");
+  if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)o) % 16 ||
+      (q_sb | q_st | q_sh | k_sb | k_st | k_sh | v_sb | v_st | v_sh) % 8)
+    return set_error(ATMA_ERR_INVALID, "gated_delta_prefill: rows must be 16-byte aligned");
+  int64_t longest = T, total = 0;
+  if (seq_lens) {
+    longest = 0;
+    for (int64_t b = 0; b < B; ++b) {
+      if (seq_lens[b] < 0) return set_error(ATMA_ERR_INVALID, "gated_delta_prefill: negative sequence length");
+      longest = std::max(longest, seq_lens[b]);
+      total += seq_lens[b];
+    }
+    if (total == 0) return ATMA_OK;
+  }
+  const int64_t chunks = (longest + kChunk - 1) / kChunk;
+  if (longest > 1 << 30 || total > 1 << 30 || longest * H * d * 2 >= (1ll << 32) ||
+      std::min<int64_t>(B, seq_lens ? kVarSeqs : B) * H * chunks >= (1ll << 31))
+    return set_error(ATMA_ERR_UNSUPPORTED, "gated_delta_prefill: sizes too large");
+  if (!workspace || workspace_bytes < atma_gated_delta_prefill_workspace_bytes(B, T, H, d, seq_lens))
+    return set_error(ATMA_ERR_WORKSPACE, "gated_delta_prefill: workspace too small");
+  GdnArgs a{};
+  a.q = q; a.q_sb = q_sb; a.q_st = q_st; a.q_sh = q_sh;
+  a.k = k; a.k_sb = k_sb; a.k_st = k_st; a.k_sh = k_sh;
+  a.v = v; a.v_sb = v_sb; a.v_st = v_st; a.v_sh = v_sh;
+  a.g = g; a.beta = beta; a.s0 = state_table; a.s_out = state_table; a.o = o;
+  a.B = (int)B; a.T = (int)T; a.H = (int)H; a.NC = (int)chunks;
+  a.G = (int)(H / Hkv);
+  a.scale = scale; a.l2norm = use_qk_l2norm ? 1 : 0; a.ws = workspace;
+  a.gate_logits = gate_logits ? 1 : 0; a.g_bias = g_bias; a.b_bias = b_bias;
+  a.start_flag = start_flag; a.start_epoch = start_epoch;
+  a.slots = slots; a.num_slots = num_slots;
+  hipStream_t s = (hipStream_t)stream;
+  if (!seq_lens) return launch_gdn16(a, nullptr, dtype, (int)d, s);
+  const bool split = gdn_split_long(B, H, d, seq_lens);
+  int64_t start = 0;
+  for (int64_t b0 = 0; b0 < B; b0 += kVarSeqs) {
+    int order[kVarSeqs], starts[kVarSeqs], n = 0;
+    for (int64_t b = b0; b < B && b < b0 + kVarSeqs; ++b) {
+      starts[b - b0] = (int)start;
+      if (split && gdn_long(H, d, seq_lens[b])) {
+        GdnArgs l = a;
+        l.q = (const char*)q + start * q_st * 2;
+        l.k = (const char*)k + start * k_st * 2;
+        l.v = (const char*)v + start * v_st * 2;
+        l.g = g + start * H;
+        l.beta = beta + start * H;
+        l.o = (char*)o + start * H * d * 2;
+        l.slots = slots + b;
+        l.B = 1; l.T = (int)seq_lens[b]; l.NC = (int)((seq_lens[b] + kChunk - 1) / kChunk);
+        const int rc = launch_gdn16(l, nullptr, dtype, (int)d, s);
+        if (rc) return rc;
+      } else if (seq_lens[b] > 0) {
+        order[n++] = (int)(b - b0);
+      }
+      start += seq_lens[b];
+    }
+    if (n == 0) continue;
+    std::stable_sort(order, order + n, [&](int x, int y) { return seq_lens[b0 + x] > seq_lens[b0 + y]; });
+    VarSeqs vs{};
+    vs.n = n;
+    for (int i = 0, c = 0; i < n; ++i) {
+      vs.start[i] = starts[order[i]];
+      vs.len[i] = (int)seq_lens[b0 + order[i]];
+      vs.chunk0[i] = c;
+      vs.row[i] = (int)b0 + order[i];
+      c += (vs.len[i] + kChunk - 1) / kChunk;
+    }
+    const int rc = launch_gdn16(a, &vs, dtype, (int)d, s);
+    if (rc) return rc;
+  }
+  return ATMA_OK;
 }
 
 namespace atma {

@@ -69,8 +69,32 @@ __device__ __forceinline__ u32x4 pack8(const f32x4& lo, const f32x4& hi) {
   return u32x4{pack2<T>(lo[0], lo[1]), pack2<T>(lo[2], lo[3]), pack2<T>(hi[0], hi[1]), pack2<T>(hi[2], hi[3])};
 }
 
-template <typename T, int D>
-__global__ void __launch_bounds__(256) gdn_prep16_kernel(GdnArgs a) {
+// Sequence, head and chunk of a prep item (items: sequence by sequence, head by head, chunk by chunk); false past the last.
+__device__ __forceinline__ bool gdn_item(const GdnArgs& a, const DenseSeqs&, uint32_t item, int& b, int& h, int& c) {
+  if (item >= (uint32_t)(a.B * a.H * a.NC)) return false;
+  const int bh = (int)(item / (uint32_t)a.NC);
+  c = (int)(item % (uint32_t)a.NC);
+  b = bh / a.H;
+  h = bh % a.H;
+  return true;
+}
+__device__ __forceinline__ bool gdn_item(const GdnArgs& a, const VarSeqs& v, uint32_t item, int& b, int& h, int& c) {
+  const uint32_t chunk = item / (uint32_t)a.H;  // compare chunk counts: item < (chunk0 + NC) H
+  int lo = 0, hi = v.n - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) / 2;
+    if ((uint32_t)v.chunk0[mid] <= chunk) lo = mid;
+    else hi = mid - 1;
+  }
+  const uint32_t nc = (uint32_t)(v.len[lo] + 63) / 64, left = item - (uint32_t)v.chunk0[lo] * (uint32_t)a.H;
+  b = lo;
+  h = (int)(left / nc);
+  c = (int)(left % nc);
+  return h < a.H;
+}
+
+template <typename T, int D, typename SEQ>
+__global__ void __launch_bounds__(256) gdn_prep16_kernel(GdnArgs a, SEQ seqs) {
   constexpr int C = kChunk, KS = D / 32;
   __shared__ __attribute__((aligned(16))) float Nb[4][4 * 256];  // per wave: N^T of the diagonal blocks
   __shared__ __attribute__((aligned(16))) float Mb[4][4 * 256];  // per wave: T^T of the diagonal blocks
@@ -80,10 +104,10 @@ __global__ void __launch_bounds__(256) gdn_prep16_kernel(GdnArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, c16 = lane & 15;
   const uint32_t item = blockIdx.x * 4u + (uint32_t)wave;  // B H NC < 2^31 (the entry checks)
-  if (item >= (uint32_t)(a.B * a.H * a.NC)) return;          // a whole wave; the kernel has no barrier
-  const int bh = (int)(item / (uint32_t)a.NC), c = (int)(item % (uint32_t)a.NC);
-  const int b = bh / a.H, h = bh % a.H;
-  const int rows = min(a.T - c * C, C);
+  int b, h, c;
+  if (!gdn_item(a, seqs, item, b, h, c)) return;             // a whole wave; the kernel has no barrier
+  const SeqView sq = gdn_seq(a, seqs, b);
+  const int rows = min(sq.T - c * C, C);
   float* tbt = Tk[wave][0];   // beta
   float* tik = Tk[wave][1];   // 1 / |k| (1 without l2norm, 0 past T)
   float* tiq = Tk[wave][2];   // scale / |q|
@@ -100,9 +124,9 @@ __global__ void __launch_bounds__(256) gdn_prep16_kernel(GdnArgs a) {
 
   // ---- k and q rows as MFMA fragments: lane (g, r) holds row 16p + r, columns 32s + 8g ..
   // (rows past T read as zeros)
-  const auto krs = buffer_rsrc((const T*)a.k + b * a.k_sb + (int64_t)c * C * a.k_st + (h / a.G) * a.k_sh,
+  const auto krs = buffer_rsrc((const T*)a.k + sq.ko + (int64_t)c * C * a.k_st + (h / a.G) * a.k_sh,
                                (uint32_t)(((rows - 1) * a.k_st + D) * 2));
-  const auto qrs = buffer_rsrc((const T*)a.q + b * a.q_sb + (int64_t)c * C * a.q_st + h * a.q_sh,
+  const auto qrs = buffer_rsrc((const T*)a.q + sq.qo + (int64_t)c * C * a.q_st + h * a.q_sh,
                                (uint32_t)(((rows - 1) * a.q_st + D) * 2));
   u32x4 kf[4][KS], qf[4][KS];
 #pragma unroll
@@ -116,7 +140,7 @@ __global__ void __launch_bounds__(256) gdn_prep16_kernel(GdnArgs a) {
   // ---- gates (lane = token) and the inclusive prefix sum of the log-decays
   float gl = 0.f, bt = 0.f;
   if (lane < rows) {
-    const int64_t gi = ((int64_t)b * a.T + c * C + lane) * a.H + h;
+    const int64_t gi = (sq.tok0 + c * C + lane) * a.H + h;
     gl = gdn_load_g(a, gi);
     bt = gdn_load_beta(a, gi);
   }
@@ -588,8 +612,8 @@ __global__ void __launch_bounds__(256, 1) gdn_summary16_kernel(GdnArgs a) {
 // LDS; after B1 it updates S and writes S_{c+1}'s fragments.  The output wave reads S_c's
 // fragments before B1 (the chain overwrites them only after B1) and U_c's after B1 (the
 // chain overwrites them only after the next B0).
-template <typename T, int D>
-__global__ void __launch_bounds__(256, 1) gdn_scan16_pair_kernel(GdnArgs a) {
+template <typename T, int D, typename SEQ>
+__global__ void __launch_bounds__(256, 1) gdn_scan16_pair_kernel(GdnArgs a, SEQ seqs) {
   constexpr int C = kChunk, KS = D / 32, ST = D / 16;
   constexpr int CPR = D / 8;                    // 16-byte chunks per k / q row
   constexpr int KB = C * D, VB = C * 32;        // elements of one slot's k (q) rows, v slab
@@ -616,26 +640,34 @@ __global__ void __launch_bounds__(256, 1) gdn_scan16_pair_kernel(GdnArgs a) {
   const int vw = 32 * blockIdx.y;    // the workgroup's 32 state columns
   const int v0 = vw + 16 * pw;       // this wave pair's 16
   const int seg = blockIdx.z;
-  const int c_begin = seg * a.seg_len, c_end = min(a.NC, c_begin + a.seg_len);
+  const SeqView sq = gdn_seq(a, seqs, b);
+  const int c_begin = std::is_same_v<SEQ, VarSeqs> ? 0 : seg * a.seg_len;
+  const int c_end = std::is_same_v<SEQ, VarSeqs> ? sq.NC : min(a.NC, c_begin + a.seg_len);
 
-  // a replay's entry state: segment 0's, or the one over the previous segment's summary
-  const float* seg_in = seg ? a.seg_sum + ((int64_t)bh * (a.nseg - 1) + seg - 1) * D * 2 * D : a.seg_in + (int64_t)bh * D * D;
-  const int sld = seg ? 2 * D : D;
+  // the entry state: the call's; a replay's is segment 0's copy of it, or lies over the previous segment's summary
+  const float* s0;
+  int ld0 = D;
+  if (a.seg_mode == 0) {
+    s0 = gdn_state(a, a.s0, sq.row, h, D);
+  } else if (seg == 0) {
+    s0 = a.seg_in + (int64_t)bh * D * D;
+  } else {
+    s0 = a.seg_sum + ((int64_t)bh * (a.nseg - 1) + seg - 1) * D * 2 * D;
+    ld0 = 2 * D;
+  }
 
   // ---- chain: state tile t, register i <-> row k = 32 (t/2) + 8g + 4 (t%2) + i, column v0 + c16
   f32x4 S[ST];
   u32x4 sf[KS];
   if (chain) {
 #pragma unroll
-    for (int t = 0; t < ST; ++t)
+    for (int t = 0; t < ST; ++t) S[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (s0) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int kx = 32 * (t >> 1) + 8 * g + 4 * (t & 1) + i;
-        float x;
-        if (a.seg_mode == 0) x = a.s0 ? a.s0[((int64_t)bh * D + kx) * D + v0 + c16] : 0.f;
-        else x = seg_in[kx * sld + v0 + c16];
-        S[t][i] = x;
-      }
+      for (int t = 0; t < ST; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S[t][i] = s0[(32 * (t >> 1) + 8 * g + 4 * (t & 1) + i) * ld0 + v0 + c16];
+    }
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       sf[s] = pack8<T>(S[2 * s], S[2 * s + 1]);
@@ -671,10 +703,10 @@ __global__ void __launch_bounds__(256, 1) gdn_scan16_pair_kernel(GdnArgs a) {
 #pragma unroll
   for (int r = 0; r < 2; ++r) vvo[r] = (32 * cw + 16 * r + lane / 4) * vst2 + 16u * (lane % 4);
   const uint32_t rvo = 16u * lane;
-  const T* kb = (const T*)a.k + b * a.k_sb + hk * a.k_sh;
-  const T* qb = (const T*)a.q + b * a.q_sb + h * a.q_sh;
-  const T* vb = (const T*)a.v + b * a.v_sb + hk * a.v_sh + vw;
-  const char* rb0 = (const char*)a.ws + (int64_t)bh * a.NC * RB;
+  const T* kb = (const T*)a.k + sq.ko + hk * a.k_sh;
+  const T* qb = (const T*)a.q + sq.qo + h * a.q_sh;
+  const T* vb = (const T*)a.v + sq.vo + hk * a.v_sh + vw;
+  const char* rb0 = (const char*)a.ws + (sq.chunk0 * a.H + (int64_t)h * sq.NC) * RB;
   const int last = c_end - 1;
   const uint32_t mk = __builtin_amdgcn_readfirstlane(lds_offset(Ks + 32 * cw * D));
   const uint32_t mq = __builtin_amdgcn_readfirstlane(lds_offset(Qs + 32 * cw * D));
@@ -682,7 +714,7 @@ __global__ void __launch_bounds__(256, 1) gdn_scan16_pair_kernel(GdnArgs a) {
   const uint32_t mr = __builtin_amdgcn_readfirstlane(lds_offset(Rs));
   auto copy_chunk = [&](int j, auto slot_c) {
     constexpr int sl = decltype(slot_c)::value;
-    const int rows = min(a.T - j * C, C);
+    const int rows = min(sq.T - j * C, C);
     const auto krs = buffer_rsrc(kb + (int64_t)j * C * a.k_st, (uint32_t)((rows - 1) * a.k_st + D) * 2u);
     const auto qrs = buffer_rsrc(qb + (int64_t)j * C * a.q_st, (uint32_t)((rows - 1) * a.q_st + D) * 2u);
     const auto vrs = buffer_rsrc(vb + (int64_t)j * C * a.v_st, (uint32_t)((rows - 1) * a.v_st + 32) * 2u);
@@ -701,7 +733,7 @@ __global__ void __launch_bounds__(256, 1) gdn_scan16_pair_kernel(GdnArgs a) {
     }
   };
 
-  const auto orsrc = buffer_rsrc((const T*)a.o + (int64_t)b * a.T * a.H * D, (uint32_t)((int64_t)a.T * a.H * D * 2));
+  const auto orsrc = buffer_rsrc((const T*)a.o + sq.tok0 * a.H * D, (uint32_t)((int64_t)sq.T * a.H * D * 2));
   const uint32_t oo = (uint32_t)((c16 * a.H + h) * D + v0 + 4 * g) * 2u;
   const uint32_t otok = (uint32_t)a.H * D * 2u;
   f32x4 o[4];
@@ -884,8 +916,8 @@ __global__ void __launch_bounds__(256, 1) gdn_scan16_pair_kernel(GdnArgs a) {
     if (c + 2 < c_end) body(c + 2, S2{});
   }
 
-  if (chain && seg == a.nseg - 1 && a.s_out) {
-    float* sdst = a.s_out + (int64_t)bh * D * D;
+  float* sdst = chain && seg == a.nseg - 1 ? gdn_state(a, a.s_out, sq.row, h, D) : nullptr;
+  if (sdst) {
 #pragma unroll
     for (int t = 0; t < ST; ++t)
 #pragma unroll
@@ -911,7 +943,7 @@ __global__ void __launch_bounds__(256) gdn_seg_combine_kernel(GdnArgs a) {
   __shared__ __attribute__((aligned(16))) float cur[2][16][D + 4];  // the entry state's columns, [column][row]
   const int bh = blockIdx.x, j0 = 16 * blockIdx.y;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
-  const float* s0 = a.s0 ? a.s0 + (int64_t)bh * D * D : nullptr;
+  const float* s0 = gdn_state(a, a.s0, bh / a.H, bh % a.H, D);
   f32x4 S[RT];
 #pragma unroll
   for (int t = 0; t < RT; ++t)
@@ -1000,7 +1032,7 @@ template <typename T, int D>
 static int launch16(const GdnArgs& a0, hipStream_t s) {
   GdnArgs a = a0;
   const int64_t BH = (int64_t)a.B * a.H, items = (int64_t)a.NC * BH;
-  gdn_prep16_kernel<T, D><<<dim3((unsigned)((items + 3) / 4)), dim3(256), 0, s>>>(a);
+  gdn_prep16_kernel<T, D, DenseSeqs><<<dim3((unsigned)((items + 3) / 4)), dim3(256), 0, s>>>(a, {});
   int rc = check_launch("chunk_gated_delta_rule(prep16)");
   if (rc) return rc;
   gdn16_plan(BH, a.NC, D, a.nseg, a.seg_len);
@@ -1013,7 +1045,7 @@ static int launch16(const GdnArgs& a0, hipStream_t s) {
   }
   if (a.nseg == 1) {
     a.seg_mode = 0;
-    gdn_scan16_pair_kernel<T, D><<<dim3((unsigned)BH, D / 32, 1), dim3(256), 0, s>>>(a);
+    gdn_scan16_pair_kernel<T, D, DenseSeqs><<<dim3((unsigned)BH, D / 32, 1), dim3(256), 0, s>>>(a, {});
     return check_launch("chunk_gated_delta_rule(scan16)");
   }
   // long sequences with few heads: segment summaries, their entry states, then the replays
@@ -1027,13 +1059,34 @@ static int launch16(const GdnArgs& a0, hipStream_t s) {
   rc = check_launch("chunk_gated_delta_rule(combine16)");
   if (rc) return rc;
   a.seg_mode = 2;
-  gdn_scan16_pair_kernel<T, D><<<dim3((unsigned)BH, D / 32, a.nseg), dim3(256), 0, s>>>(a);
+  gdn_scan16_pair_kernel<T, D, DenseSeqs><<<dim3((unsigned)BH, D / 32, a.nseg), dim3(256), 0, s>>>(a, {});
   return check_launch("chunk_gated_delta_rule(replay16)");
 }
 
-int launch_gdn16(const GdnArgs& a, int dtype, int D, hipStream_t s) {
-  if (dtype == ATMA_BF16) return D == 128 ? launch16<bf16, 128>(a, s) : launch16<bf16, 64>(a, s);
-  return D == 128 ? launch16<f16, 128>(a, s) : launch16<f16, 64>(a, s);
+// Ragged sequences packed along tokens: the plain scan of all of them in one launch each (a batch of prompts has heads
+// enough to fill the device; the longest sequence's chunks set the time).  12 prompts of 64 .. 2,048 tokens, 8 heads: prep
+// 22 and scan 48 us; one by one 157 and 187 with 43 + 35 for the split ones, and a gather and a scatter of the state each.
+template <typename T, int D>
+static int launch16_var(const GdnArgs& a0, const VarSeqs& v, hipStream_t s) {
+  GdnArgs a = a0;
+  a.nseg = 1;
+  a.seg_mode = 0;
+  const int64_t items = (int64_t)(v.chunk0[v.n - 1] + (v.len[v.n - 1] + 63) / 64) * a.H;
+  gdn_prep16_kernel<T, D, VarSeqs><<<dim3((unsigned)((items + 3) / 4)), dim3(256), 0, s>>>(a, v);
+  const int rc = check_launch("gated_delta_prefill(prep16)");
+  if (rc) return rc;
+  gdn_scan16_pair_kernel<T, D, VarSeqs><<<dim3((unsigned)(v.n * a.H), D / 32, 1), dim3(256), 0, s>>>(a, v);
+  return check_launch("gated_delta_prefill(scan16)");
+}
+
+template <typename T>
+static int launch16_d(const GdnArgs& a, const VarSeqs* v, int D, hipStream_t s) {
+  if (v) return D == 128 ? launch16_var<T, 128>(a, *v, s) : launch16_var<T, 64>(a, *v, s);
+  return D == 128 ? launch16<T, 128>(a, s) : launch16<T, 64>(a, s);
+}
+
+int launch_gdn16(const GdnArgs& a, const VarSeqs* v, int dtype, int D, hipStream_t s) {
+  return dtype == ATMA_BF16 ? launch16_d<bf16>(a, v, D, s) : launch16_d<f16>(a, v, D, s);
 }
 
 }  // namespace atma

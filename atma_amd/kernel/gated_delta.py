@@ -203,6 +203,47 @@ def _chunk_gated_delta_train(q, k, v, g, beta, scale, initial_state, output_fina
     return o.to(q.dtype), (S if output_final_state else None)
 
 
+def gated_delta_prefill_supported(q, state_table):
+    """Rows and tables ``gated_delta_prefill`` serves: 16-bit GPU rows, heads of 64 or 128, a contiguous fp32 table."""
+    return (q.is_cuda and q.dtype in (torch.bfloat16, torch.float16) and q.shape[-1] in (64, 128)
+            and state_table.dtype == torch.float32 and state_table.is_contiguous()
+            and tuple(state_table.shape[1:]) == (q.shape[-2], q.shape[-1], q.shape[-1])
+            and not torch.is_grad_enabled())
+
+
+@torch.no_grad()
+def gated_delta_prefill(q, k, v, g, beta, state_table, slots, gate_bias, seq_lens=None, start_signal=None):
+    """The serving routes' prefill recurrence (q and k L2-normalised, raw gate logits with ``gate_bias``, scale 1), each
+    sequence's state read from and advanced in its row ``slots[b]`` of ``state_table`` (rows, H, d, d) fp32.
+    q (B, T, H, d), k, v (B, T, Hkv, d), g, beta (B, T, H) fp32; or, with ``seq_lens`` (host ints), ragged sequences
+    packed along tokens: q (tokens, H, d), k, v (tokens, Hkv, d), g, beta (tokens, H), all in one launch pair.
+    Returns the readout in q's shape and dtype."""
+    packed, lens = seq_lens is not None, None
+    if packed:
+        q, k, v, g, beta = (t.unsqueeze(0) for t in (q, k, v, g, beta))
+        lens = [int(n) for n in seq_lens]
+        if sum(lens) != q.shape[1] or slots.numel() != len(lens):
+            raise ValueError("seq_lens must cover the packed tokens, with one table row each")
+    _check_args(q, k, v, g, beta, None)
+    B, T, H, d = q.shape
+    n = len(seq_lens) if packed else B
+    if v.shape[3] != d or slots.numel() != n:
+        raise ValueError("gated_delta_prefill: dv == dk and one table row per sequence")
+    if not gated_delta_prefill_supported(q, state_table):
+        raise ValueError("gated_delta_prefill: 16-bit rows and a contiguous fp32 state table")
+    g, beta = g.to(torch.float32).contiguous(), beta.to(torch.float32).contiguous()
+    slots = slots.to(device=q.device, dtype=torch.int64).reshape(-1).contiguous()
+    o = torch.empty((B, T, H, d), device=q.device, dtype=q.dtype)
+    if start_signal is not None and (packed or B * T == 0):
+        start_signal.flag.fill_(start_signal.epoch)   # nothing to overlap with: release the waiting stream now
+        start_signal = None
+    if B * T > 0:
+        torch.ops.atma_hip.gated_delta_prefill(
+            q, k, v, g, beta, state_table, slots, o, lens, float(gate_bias[0]), float(gate_bias[1]),
+            None if start_signal is None else start_signal.flag, 0 if start_signal is None else start_signal.epoch)
+    return o[0] if packed else o
+
+
 def recurrence_pays_to_overlap(B, H, dv, dtype, device):
     """True when the recurrence kernel's grid (B*H workgroups per column slab: 32 columns
     for 16-bit inputs, 16 for fp32) takes at most a quarter of the CUs, so running Polar

@@ -46,6 +46,7 @@ from ..kernel.decode_fusions import (PartialSums, chunk_width, global_decode_gat
                                      linear_tokens_chunks, linear_tokens_gated, linear_tokens_multi,
                                      linear_tokens_multi_supported,
                                      residual_rms_norm, residual_rms_norm_supported)
+from ..kernel.gated_delta import gated_delta_prefill, gated_delta_prefill_supported
 from ..kernel.inference_ops import (linear_tokens, linear_tokens_supported, packed_causal_conv1d,
                                      squared_relu_gate)
 from ..kernel.layer_fusions import (global_gate, head_rms_norm, linear_gated, linear_gated_supported,
@@ -140,6 +141,15 @@ class TitansMemory(nn.Module):
         return chunk_gated_delta_rule(q, k, v, zg, zb, scale=1.0, initial_state=initial_state,
                                       output_final_state=output_final_state, use_qk_l2norm_in_kernel=True,
                                       gate_bias=(self.gamma_bias, self.beta_bias), start_signal=start_signal)
+
+    def readout_table(self, x, q, k, v, table, slots, seq_lens=None, start_signal=None):
+        """``readout`` with the states read from and advanced in rows ``slots`` of ``table``; with ``seq_lens`` over
+        ragged sequences packed along tokens (x (tokens, dim), q, k, v (tokens, heads, dk))."""
+        zg, zb = self.raw_logits(x if seq_lens is None else x.unsqueeze(0))
+        if seq_lens is not None:
+            zg, zb = zg[0], zb[0]
+        return gated_delta_prefill(q, k, v, zg, zb, table, slots, (self.gamma_bias, self.beta_bias), seq_lens,
+                                   start_signal)
 
     def decode_gates(self, x):
         """(gamma, beta) of one decode step: retention sigmoid(w_gamma x + gamma_bias) and
@@ -405,9 +415,21 @@ class PolarAttention(nn.Module):
         """Causal full-sequence mixer (``model/reference.py:127-195``): x (B, T, dim)."""
         B, T, _ = x.shape
         q, gate, k, v = (t.unflatten(0, (B, T)) for t in self._project_canon(x, B, T))
-        return self._attend_prefill(x, q, gate, k, v, None, None)
+        return self._attend_prefill(x, q, gate, k, v)
 
-    def _attend_prefill(self, x, q, gate, k, v, S0, final_sink, defer=False):
+    def _memory(self, x, q, k, v, fused, cache, slots, signal):
+        """The memory branch of a prefill from zero states (``cache`` None) or from and to the table's rows: its readout
+        (``fused``, what ``_fused_out`` takes) or its output."""
+        if cache is not None and fused and gated_delta_prefill_supported(q, cache.mem_table):
+            return self.mem.readout_table(x, q, k, v, cache.mem_table, slots, start_signal=signal)
+        S0 = None if cache is None else cache.mem_table[slots]
+        r, S = (self.mem.readout if fused else self.mem)(x, q, k, v, initial_state=S0,
+                                                         output_final_state=cache is not None, start_signal=signal)
+        if cache is not None:
+            cache.mem_table[slots] = S
+        return r
+
+    def _attend_prefill(self, x, q, gate, k, v, cache=None, slots=None, defer=False):
         """``defer`` (16-bit inference): return the output as a ``PartialSums`` over B T rows."""
         B, T = q.shape[:2]
         H, dk = self.num_heads, self.head_dim
@@ -425,21 +447,14 @@ class PolarAttention(nn.Module):
                 return c, mag
             return self._combine(c.transpose(1, 2), mag.transpose(1, 2), gate)
 
-        def memory(signal):
-            fn = self.mem.readout if fused else self.mem
-            return fn(x, q, k, v, initial_state=S0, output_final_state=final_sink is not None, start_signal=signal)
-
-        out, m = self._with_memory(polar, memory, (x, q, k, v))
-        if m is not None and final_sink is not None:
-            final_sink(m[1])
+        out, m = self._with_memory(polar, lambda signal: self._memory(x, q, k, v, fused, cache, slots, signal),
+                                   (x, q, k, v))
         if fused:
             c, mag = out
             res = self._fused_out(x.reshape(B * T, -1), c.transpose(1, 2), mag.transpose(1, 2).reshape(B * T, H),
-                                  gate.reshape(B * T, H, dk), m[0].reshape(B * T, H, dk))
+                                  gate.reshape(B * T, H, dk), m.reshape(B * T, H, dk))
             return res if defer else res.materialize().view(B, T, -1)
-        if m is not None:
-            out = out + m[0]
-        return out
+        return out if m is None else out + m
 
     def prefill(self, x, cache: GlobalLayerCache, slots, slot_mapping, defer=False):
         """Dense fresh prefill of B equal-length sequences (``inference/models/atma.py:397-437``).
@@ -450,12 +465,7 @@ class PolarAttention(nn.Module):
         H, Hkv, dk = self.num_heads, self.num_kv_heads, self.head_dim
         q, gate, k, v = (t.unflatten(0, (B, T)) for t in
                          self._project_canon(x, B, T, cache, slots, slot_mapping))
-        S0 = cache.mem_table[slots] if self.mem is not None else None
-
-        def sink(S):
-            cache.mem_table[slots] = S
-
-        return self._attend_prefill(x, q, gate, k, v, S0, sink, defer)
+        return self._attend_prefill(x, q, gate, k, v, cache, slots, defer)
 
     def prefill_packed(self, x, cache: GlobalLayerCache, seq_lens, slots, slot_mapping, tile_maps, token_maps,
                        defer=False):
@@ -463,7 +473,7 @@ class PolarAttention(nn.Module):
         (``inference/models/atma.py:431-507``): the Canon convs as one packed launch each
         (tails written per sequence), the K/V rows to the pages, ONE tile-mapped Polar
         launch over every sequence (``polar_attention_packed_fwd``, 16-bit inputs), and the
-        memory per sequence from its table state.
+        memory of all of them from their table states.
 
         x: (tokens, dim) packed in sequence order; seq_lens: the B prompt lengths; slots: (B,)
         int64 table rows; slot_mapping: (tokens,) int32 cache slots; tile_maps: (tile_seq_starts,
@@ -473,17 +483,10 @@ class PolarAttention(nn.Module):
         H, Hkv, dk = self.num_heads, self.num_kv_heads, self.head_dim
         q, gate, k, v = self._project_canon(x, 1, total, cache, slots, slot_mapping, token_maps=token_maps)
         c, mag = polar_attention_packed_fwd(q, k, v, *tile_maps, window=self.window, **self.polar_params())
-        if self._glue_fusable(x):
-            rs, start = [], 0
-            for i, n in enumerate(int(t) for t in seq_lens):
-                sl = slots[i:i + 1]
-                seg = slice(start, start + n)
-                r, S = self.mem.readout(x[seg][None], q[seg][None], k[seg][None], v[seg][None],
-                                        initial_state=cache.mem_table[sl], output_final_state=True)
-                cache.mem_table[sl] = S
-                rs.append(r[0])
-                start += n
-            res = self._fused_out(x, c.view(1, total, H, dk), mag, gate, torch.cat(rs, 0))
+        fused = self._glue_fusable(x)
+        if fused and gated_delta_prefill_supported(q, cache.mem_table):
+            r = self.mem.readout_table(x, q, k, v, cache.mem_table, slots, seq_lens)
+            res = self._fused_out(x, c.view(1, total, H, dk), mag, gate, r)
             return res if defer else res.materialize()
         out = self._combine(c, mag, gate)
         if self.mem is not None:
@@ -537,20 +540,14 @@ class PolarAttention(nn.Module):
             return (cs[0], ms[0]) if B == 1 else (torch.cat(cs), torch.cat(ms))
 
         fused = self._glue_fusable(x)
-        S0 = cache.mem_table[slots] if self.mem is not None else None
-
-        def memory(signal):
-            return (self.mem.readout if fused else self.mem)(x, q, k, v, initial_state=S0, output_final_state=True,
-                                                             start_signal=signal)
-
-        (c, mag), m = self._with_memory(attend, memory, (x, q, k, v))
-        if m is not None:
-            cache.mem_table[slots] = m[1]
+        (c, mag), m = self._with_memory(attend,
+                                        lambda signal: self._memory(x, q, k, v, fused, cache, slots, signal),
+                                        (x, q, k, v))
         if fused:
             return self._fused_out(x.reshape(B * T, -1), c, mag.reshape(B * T, H), gate.reshape(B * T, H, dk),
-                                   m[0].reshape(B * T, H, dk)).materialize().view(B, T, -1)
+                                   m.reshape(B * T, H, dk)).materialize().view(B, T, -1)
         out = self._combine(c, mag, gate)
-        return out if m is None else out + m[0]
+        return out if m is None else out + m
 
     def _decode_fusable(self, x, cache, block_tables):
         H, Hkv, dk = self.num_heads, self.num_kv_heads, self.head_dim

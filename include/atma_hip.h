@@ -734,6 +734,24 @@ int atma_paged_kv_concat(const void* k_cache, const void* v_cache, int64_t num_p
                          int64_t v_st, int64_t n_new, void* k_out, void* v_out, int64_t row_elems, int dtype,
                          void* stream);
 
+/*
+ * atma_chunk_gated_delta_rule for the serving routes (inference/models/atma.py:262-339): the states are rows of a table
+ * (num_slots, H, d, d) fp32, sequence b's read and advanced in place at row slots[b] (negative: from the end; a
+ * row outside the table starts from zero and is not kept; the slots of one call are distinct), and the sequences may be ragged: seq_lens (host, B
+ * entries) non-NULL: sequence b is the next seq_lens[b] tokens of the packed axis (batch strides unused, T ignored;
+ * empty sequences leave their state), all of them in one prep and one scan launch per 64 sequences (a few far longer than
+ * the rest are split along tokens in launches of their own).  16-bit rows,
+ * 16-byte aligned; other arguments as there.
+ */
+size_t atma_gated_delta_prefill_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t d, const int64_t* seq_lens);
+int atma_gated_delta_prefill(const void* q, int64_t q_sb, int64_t q_st, int64_t q_sh, const void* k, int64_t k_sb,
+                             int64_t k_st, int64_t k_sh, const void* v, int64_t v_sb, int64_t v_st, int64_t v_sh,
+                             const float* g, const float* beta, float* state_table, const int64_t* slots,
+                             int64_t num_slots, void* o, int64_t B, int64_t T, const int64_t* seq_lens, int64_t H,
+                             int64_t Hkv, int64_t d, int dtype, float scale, int use_qk_l2norm, int gate_logits,
+                             float g_bias, float b_bias, void* workspace, size_t workspace_bytes, int32_t* start_flag,
+                             int32_t start_epoch, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -472,7 +472,7 @@ def _bwd16_prep(q, k, v, d_out, g, beta, scale, l2norm):
     return [kr, kt, qr, qt, tm, tt, rt, vt, ot, got, f]
 
 
-def _bwd16_chain(kr, kt, qt, tm, tt, rt, vt, ot, got, f, s0, dst):
+def _bwd16_chain(kr, qr, tm, tt, rt, vt, ot, f, s0, dst):
     lib = _lib.load()
     BH, NC, C, d = kr.shape
     t16 = dict(device=kr.device, dtype=kr.dtype)
@@ -480,8 +480,8 @@ def _bwd16_chain(kr, kt, qt, tm, tt, rt, vt, ot, got, f, s0, dst):
     u = torch.empty((BH, NC, C, d), **t16)
     dy = torch.empty((BH, NC, C, d), device=kr.device, dtype=torch.float32)
     ds0 = torch.empty((BH, d, d), device=kr.device, dtype=torch.float32)
-    rc = lib.atma_gated_delta_bwd16_chain(kr.data_ptr(), kt.data_ptr(), qt.data_ptr(), tm.data_ptr(), tt.data_ptr(),
-                                          rt.data_ptr(), vt.data_ptr(), ot.data_ptr(), got.data_ptr(), f.data_ptr(),
+    rc = lib.atma_gated_delta_bwd16_chain(kr.data_ptr(), qr.data_ptr(), tm.data_ptr(), tt.data_ptr(), rt.data_ptr(),
+                                          vt.data_ptr(), ot.data_ptr(), f.data_ptr(),
                                           _lib.ptr(s0), _lib.ptr(dst), s_entry.data_ptr(), ds_end.data_ptr(),
                                           u.data_ptr(), dy.data_ptr(), ds0.data_ptr(), BH, NC, d,
                                           _lib.dtype_code(kr.dtype), _lib.stream_handle(kr.device))
@@ -531,7 +531,7 @@ def gated_delta_bwd16_op(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tenso
         return [torch.zeros_like(q), torch.zeros_like(k), torch.zeros_like(v), torch.zeros_like(g),
                 torch.zeros_like(beta), ds0]
     kr, kt, qr, qt, tm, tt, rt, vt, ot, got, f = _bwd16_prep(q, k, v, d_out, g, beta, scale, l2norm)
-    s_entry, ds_end, u, dy, ds0 = _bwd16_chain(kr, kt, qt, tm, tt, rt, vt, ot, got, f, s0, dst)
+    s_entry, ds_end, u, dy, ds0 = _bwd16_chain(kr, qr, tm, tt, rt, vt, ot, f, s0, dst)
     dq, dk, dv, dg, db = _bwd16_local(kr, kt, qr, qt, q, k, v, d_out, f, s_entry, ds_end, u, dy)
     return [dq, dk, dv, dg, db, ds0.reshape(B, H, d, d)]
 
@@ -553,7 +553,7 @@ def gated_delta_bwd16_stages(q, k, v, g, beta, initial_state, d_out, d_final_sta
     s0, dst = _bwd16_states(initial_state, d_final_state, B, H, d)
     names = ["kr", "kt", "qr", "qt", "tm", "tt", "rt", "vt", "ot", "got", "f"]
     out = dict(zip(names, _bwd16_prep(q, k, v, d_out, g, beta, scale, l2norm)))
-    chain = _bwd16_chain(*(out[n] for n in ("kr", "kt", "qt", "tm", "tt", "rt", "vt", "ot", "got", "f")), s0, dst)
+    chain = _bwd16_chain(*(out[n] for n in ("kr", "qr", "tm", "tt", "rt", "vt", "ot", "f")), s0, dst)
     out.update(zip(["s_entry", "ds_end", "u", "dy", "ds0"], chain))
     loc = _bwd16_local(out["kr"], out["kt"], out["qr"], out["qt"], q, k, v, d_out, out["f"], out["s_entry"],
                        out["ds_end"], out["u"], out["dy"])

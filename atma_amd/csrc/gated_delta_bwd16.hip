@@ -9,20 +9,23 @@
 // and the backward carries dS = dL/dS' from the last chunk to the first:
 //   dU = Rq^T dO + diag(w) K dS,   dY = T^T dU,
 //   dS <- Ga_C dS + Q^T diag(Ga) dO - K^T diag(Ga beta) dY.
-// This kernel runs both chains (the forward one to recover each chunk's entry state,
-// then the backward one) and writes, per chunk, the entry state S, the exit-state
+// This kernel runs both chains (the forward one to recover each chunk's entry state
+// and the backward one, which do not depend on each other, beside each other) and writes, per chunk, the entry state S, the exit-state
 // gradient dS and dY; every other gradient is a product within one chunk, formed by the
 // caller from these (dV = diag(beta) dY, the rest batched over chunks).
 //
-// MI355X mapping: one workgroup of kChainWaves waves per (sequence-head, 16 kChainWaves
+// MI355X mapping: one workgroup of kChainWaves waves per (chain, sequence-head, 16 kChainWaves
 // state columns), each wave owning 16 columns (the recurrence never mixes V columns).
-// The chunk's shared operands -- k rows, k^T, q^T, T (forward) or T^T (backward), Rq^T,
-// 64 x 64 or 64 x d bf16 tiles the caller lays out -- are staged in LDS with rows padded
-// by 16 bytes (the
-// 16-lane fragment reads then touch 16 distinct bank groups).  Products run on
+// The chunk's shared operands -- k rows, q rows, T (forward) or T^T (backward), Rq^T,
+// 64 x 64 or 64 x d 16-bit tiles -- are staged in LDS with rows padded
+// by 16 bytes (the 16-lane fragment reads then touch 16 distinct bank groups); k^T and q^T
+// fragments come from the rows by transposing reads.  Products run on
 // v_mfma_f32_16x16x32 (fp32 accumulation); the state and every per-column intermediate
 // (Y, U, dU, dY) go through a per-wave transposed bf16 buffer ([column][k], 16 bytes per
 // lane per fragment) to become the B operand of the next product.
+// Bound by the latency of a chunk's chain of products and LDS exchanges, with one wave per
+// SIMD: 8 sequences of 2,048 tokens, 8 heads, d = 128 take 167 us; 247 with one chain after the
+// other on two of a CU's four SIMDs and with k^T, q^T and (diag(Ga) dO)^T read as tiles of their own.
 #include <initializer_list>
 #include <type_traits>
 
@@ -38,14 +41,12 @@ constexpr int kFRows = 9;
 
 struct Bwd16ChainArgs {
   const void* kr;    // [N][64][D]  k rows of each chunk (N = BH * NC, chunk-head major)
-  const void* kt;    // [N][D][64]  k^T
-  const void* qt;    // [N][D][64]  q^T (scaled, normalised)
+  const void* qr;    // [N][64][D]  q rows (scaled, normalised)
   const void* tm;    // [N][64][64] T
   const void* tt;    // [N][64][64] T^T
   const void* rt;    // [N][64][64] Rq^T
   const void* vt;    // [N][D][64]  v^T
   const void* ot;    // [N][D][64]  dO^T
-  const void* got;   // [N][D][64]  (diag(Ga) dO)^T
   const float* f;    // [N][5][64]  Ga, w, beta, Ga_C (all 64 entries), lg
   const float* s0;   // [BH][D][D] initial state, or null (zero)
   const float* dst;  // [BH][D][D] final-state cotangent, or null (zero)
@@ -55,6 +56,16 @@ struct Bwd16ChainArgs {
   float* dy;         // [N][64][D] out: dY
   float* ds0;        // [BH][D][D] out: the gradient of the initial state
   int BH, NC;
+};
+
+// LDS bytes of a chain workgroup: two of them share a CU, one per SIMD pair.
+template <int D>
+struct ChainLds {
+  static constexpr int NW = 2, C = 64, PD = D + 8, PC = C + 8;  // padded pitches (elements)
+  static constexpr int Kr = 0, Tm = Kr + 2 * C * PD, Fs = Tm + 2 * C * PC, Sb = Fs + 4 * 4 * C, X1 = Sb + NW * 32 * PD,
+                       X2 = X1 + NW * 32 * PC, Fwd = X2 + NW * 32 * PC;
+  static constexpr int Qr = Fwd, Rt = Qr + 2 * C * PD, XO = Rt + 2 * C * PC, Bwd = XO + NW * 32 * PC;
+  static_assert(Bwd <= 80 * 1024, "two workgroups per CU");
 };
 
 // A contiguous 16-bit tile of N * NTH 16-byte chunks: thread tid (of NTH) holds chunks
@@ -75,35 +86,44 @@ __device__ __forceinline__ void tile_store(T* dst, const u32x4 (&r)[N], int tid)
   }
 }
 
-// Waves (16 state columns each) per workgroup of the chain kernel: two, so a configs[1]
-// shape (64 sequence-heads, d = 128) runs 256 workgroups, one per CU (the LDS of one
-// workgroup's tiles allows no second).
+// Waves (16 state columns each) per workgroup of the chain kernel: two, so that 64
+// sequence-heads of d = 128 run 256 workgroups of each chain, one of both per CU.
 constexpr int kChainWaves = 2;
 
 template <typename T, int D>
 __global__ void __launch_bounds__(64 * kChainWaves, 1) gdn_bwd16_chain_kernel(Bwd16ChainArgs a) {
   constexpr int NW = kChainWaves, NTH = 64 * NW, WC = 16 * NW;  // waves, threads, columns
-  constexpr int C = 64, PD = D + 8, PC = C + 8;  // padded LDS pitches (elements)
+  using L = ChainLds<D>;
+  constexpr int C = 64, PD = L::PD, PC = L::PC;
+  static_assert(L::NW == NW, "waves");
   constexpr int KS = D / 32;                      // 32-wide k steps over D
   constexpr int DT = D / 16;                      // 16-row tiles over D
   static_assert(D % WC == 0 && 4 * C % NTH == 0, "whole column slabs and factor rows");
-  __shared__ __attribute__((aligned(16))) T Kr[C * PD];
-  __shared__ __attribute__((aligned(16))) T Kt[D * PC];
-  __shared__ __attribute__((aligned(16))) T Qt[D * PC];
-  __shared__ __attribute__((aligned(16))) T Tm[C * PC];  // T in the forward chain, T^T in the backward
-  __shared__ __attribute__((aligned(16))) T Rt[C * PC];
-  __shared__ float Fs[4 * C];
-  __shared__ __attribute__((aligned(16))) T Sb[NW][16 * PD];  // S^T / dS^T of the wave's columns
-  __shared__ __attribute__((aligned(16))) T X1[NW][16 * PC];
-  __shared__ __attribute__((aligned(16))) T X2[NW][16 * PC];
-  __shared__ __attribute__((aligned(16))) T XO[NW][16 * PC];  // dO^T rows of the wave's columns
-  __shared__ __attribute__((aligned(16))) T XG[NW][16 * PC];  // (Ga dO)^T rows
-
+  __shared__ __attribute__((aligned(16))) char lds[L::Bwd];
+  T* Kr = (T*)(lds + L::Kr);
+  T* Qr = (T*)(lds + L::Qr);
+  T* Tm = (T*)(lds + L::Tm);  // T in the forward chain, T^T in the backward
+  T* Rt = (T*)(lds + L::Rt);
+  float* Fs = (float*)(lds + L::Fs);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, c16 = lane & 15;
-  const int bh = blockIdx.x / (D / WC);
-  const int v0 = WC * (blockIdx.x % (D / WC)) + 16 * wave;  // the wave's first column
+  T* Sb = (T*)(lds + L::Sb) + wave * 16 * PD;  // S^T / dS^T of the wave's columns
+  T* X1 = (T*)(lds + L::X1) + wave * 16 * PC;
+  T* X2 = (T*)(lds + L::X2) + wave * 16 * PC;
+  T* XO = (T*)(lds + L::XO) + wave * 16 * PC;  // dO^T rows of the wave's columns
+  // the forward chains first, then the backward ones; the column slabs of one sequence-head
+  // go to one XCD (workgroup i runs on XCD i % 8), whose L2 then serves its tiles
+  constexpr int SL = D / WC;
+  const int nwg = a.BH * SL;
+  const bool fwd = (int)blockIdx.x < nwg;
+  const int wg = fwd ? blockIdx.x : blockIdx.x - nwg;
+  int bh = wg / SL, slab = wg % SL;
+  if (a.BH % 8 == 0) {
+    bh = (wg >> 3) / SL * 8 + (wg & 7);
+    slab = (wg >> 3) % SL;
+  }
+  const int v0 = WC * slab + 16 * wave;  // the wave's first column
   const int col = v0 + c16;                                  // the lane's column (C layout)
 
   constexpr int NT = C * D / 8 / NTH;   // chunks per thread of a 64 x D or D x 64 tile
@@ -127,6 +147,13 @@ __global__ void __launch_bounds__(64 * kChainWaves, 1) gdn_bwd16_chain_kernel(Bw
   auto frag = [&](const T* tile, int pitch, int row0, int k0) {
     return *(const u32x4*)(tile + (row0 + c16) * pitch + k0 + 8 * g);
   };
+  // fragment of the transpose: rows col0 + [0, 16) are columns of a row tile, k its rows k0 + 8 g + [0, 8), by
+  // transposing reads (lane s of a 16-lane group reads row + s / 4, columns 4 (s % 4) .., lane i gets column i)
+  auto frag_t = [&](const T* tile, int col0, int k0) {
+    const T* p = tile + (k0 + 8 * g + (c16 >> 2)) * PD + col0 + 4 * (c16 & 3);
+    const u32x2 lo = lds_read_tr16(p), hi = lds_read_tr16(p + 4 * PD);
+    return u32x4{lo[0], lo[1], hi[0], hi[1]};
+  };
   // C tile t (rows 16 t + 4 g + i, column c16) into a [column][row] buffer
   auto put_t = [&](T* buf, int pitch, int t, const f32x4& x) {
     const u32x2 pk = {pack2<T>(x[0], x[1]), pack2<T>(x[2], x[3])};
@@ -149,103 +176,105 @@ __global__ void __launch_bounds__(64 * kChainWaves, 1) gdn_bwd16_chain_kernel(Bw
   };
 
   // ---------------------------------------------------------------- forward chain
-  f32x4 S[DT];
-#pragma unroll
-  for (int t = 0; t < DT; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      S[t][i] = a.s0 ? a.s0[((int64_t)bh * D + rows_of(t, i)) * D + col] : 0.f;
-
   // the next chunk's operands are loaded into registers while this one computes
-  u32x4 rk[NT], rkt[NT], rtm[NTM];
-  u32x2 rv[4];
+  u32x4 rk[NT], rtm[NTM];
   float rf[NF];
-  auto fwd_load = [&](int64_t n) {
-    tile_load<NT, NTH>(rk, (const T*)a.kr + n * C * D, tid);
-    tile_load<NT, NTH>(rkt, (const T*)a.kt + n * D * C, tid);
-    tile_load<NTM, NTH>(rtm, (const T*)a.tm + n * C * C, tid);
+  if (fwd) {
+    f32x4 S[DT];
 #pragma unroll
-    for (int j = 0; j < NF; ++j) rf[j] = a.f[n * kFRows * C + tid + NTH * j];
-    const T* vrow = (const T*)a.vt + (n * D + col) * C;
+    for (int t = 0; t < DT; ++t)
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) rv[rt] = *(const u32x2*)(vrow + 16 * rt + 4 * g);
-  };
-  fwd_load((int64_t)bh * a.NC);
-  for (int c = 0; c < a.NC; ++c) {
-    const int64_t n = (int64_t)bh * a.NC + c;
-    __syncthreads();  // every wave is done with the previous chunk's tiles
-    tile_store<NT, D / 8, PD, NTH>(Kr, rk, tid);
-    tile_store<NT, 8, PC, NTH>(Kt, rkt, tid);
-    tile_store<NTM, 8, PC, NTH>(Tm, rtm, tid);
-#pragma unroll
-    for (int j = 0; j < NF; ++j) Fs[tid + NTH * j] = rf[j];
-    f32x4 Vc[4];  // v of the lane's column, C layout (rows = tokens)
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      const u32x4 x = {rv[rt][0], rv[rt][1], 0, 0};
-      Vc[rt] = f32x4{elem16<T>(x, 0), elem16<T>(x, 1), elem16<T>(x, 2), elem16<T>(x, 3)};
-    }
-    if (c + 1 < a.NC) fwd_load(n + 1);
-#pragma unroll
-    for (int t = 0; t < DT; ++t) put_t(Sb[wave], PD, t, S[t]);
-    __syncthreads();
+      for (int i = 0; i < 4; ++i)
+        S[t][i] = a.s0 ? a.s0[((int64_t)bh * D + rows_of(t, i)) * D + col] : 0.f;
 
-    // Z = K S
-    f32x4 Z[4];
+    u32x2 rv[4];
+    auto fwd_load = [&](int64_t n) {
+      tile_load<NT, NTH>(rk, (const T*)a.kr + n * C * D, tid);
+      tile_load<NTM, NTH>(rtm, (const T*)a.tm + n * C * C, tid);
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) Z[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < NF; ++j) rf[j] = a.f[n * kFRows * C + tid + NTH * j];
+      const T* vrow = (const T*)a.vt + (n * D + col) * C;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const u32x4 bf = frag(Sb[wave], PD, 0, 32 * s);
+      for (int rt = 0; rt < 4; ++rt) rv[rt] = *(const u32x2*)(vrow + 16 * rt + 4 * g);
+    };
+    fwd_load((int64_t)bh * a.NC);
+    for (int c = 0; c < a.NC; ++c) {
+      const int64_t n = (int64_t)bh * a.NC + c;
+      __syncthreads();  // every wave is done with the previous chunk's tiles
+      tile_store<NT, D / 8, PD, NTH>(Kr, rk, tid);
+      tile_store<NTM, 8, PC, NTH>(Tm, rtm, tid);
 #pragma unroll
-      for (int rt = 0; rt < 4; ++rt) Z[rt] = mfma16x16x32<T>(frag(Kr, PD, 16 * rt, 32 * s), bf, Z[rt]);
-    }
-    // Y = diag(beta) (V - diag(Ga) Z)
+      for (int j = 0; j < NF; ++j) Fs[tid + NTH * j] = rf[j];
+      f32x4 Vc[4];  // v of the lane's column, C layout (rows = tokens)
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      f32x4 y;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int p = rows_of(rt, i);
-        y[i] = Fs[2 * C + p] * (Vc[rt][i] - Fs[p] * Z[rt][i]);
+      for (int rt = 0; rt < 4; ++rt) {
+        const u32x4 x = {rv[rt][0], rv[rt][1], 0, 0};
+        Vc[rt] = f32x4{elem16<T>(x, 0), elem16<T>(x, 1), elem16<T>(x, 2), elem16<T>(x, 3)};
       }
-      put_t(X1[wave], PC, rt, y);
+      if (c + 1 < a.NC) fwd_load(n + 1);
+#pragma unroll
+      for (int t = 0; t < DT; ++t) put_t(Sb, PD, t, S[t]);
+      __syncthreads();
+
+      // Z = K S
+      f32x4 Z[4];
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) Z[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const u32x4 bf = frag(Sb, PD, 0, 32 * s);
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt) Z[rt] = mfma16x16x32<T>(frag(Kr, PD, 16 * rt, 32 * s), bf, Z[rt]);
+      }
+      // Y = diag(beta) (V - diag(Ga) Z)
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) {
+        f32x4 y;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int p = rows_of(rt, i);
+          y[i] = Fs[2 * C + p] * (Vc[rt][i] - Fs[p] * Z[rt][i]);
+        }
+        put_t(X1, PC, rt, y);
+      }
+      wave_sync();
+      // U = T Y, then w U
+      f32x4 U[4];
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) U[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const u32x4 bf = frag(X1, PC, 0, 32 * s);
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt) U[rt] = mfma16x16x32<T>(frag(Tm, PC, 16 * rt, 32 * s), bf, U[rt]);
+      }
+      // U out through the wave's X1 buffer (its Y^T operand reads are done: in order, one wave)
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) put_t(X1, PC, rt, U[rt]);
+      wave_sync();
+      store_cols(X1, PC, std::integral_constant<int, C>{}, (T*)a.u + n * C * D);
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) {
+        f32x4 x;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = Fs[C + rows_of(rt, i)] * U[rt][i];
+        put_t(X2, PC, rt, x);
+      }
+      wave_sync();
+      // the entry state, then S <- Ga_C S + K^T diag(w) U
+      store_cols(Sb, PD, std::integral_constant<int, D>{}, (T*)a.s_entry + n * D * D);  // S^T of this step
+      const float gC = Fs[3 * C];
+#pragma unroll
+      for (int t = 0; t < DT; ++t) S[t] *= gC;
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const u32x4 bf = frag(X2, PC, 0, 32 * s);
+#pragma unroll
+        for (int t = 0; t < DT; ++t) S[t] = mfma16x16x32<T>(frag_t(Kr, 16 * t, 32 * s), bf, S[t]);
+      }
     }
-    wave_sync();
-    // U = T Y, then w U
-    f32x4 U[4];
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) U[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const u32x4 bf = frag(X1[wave], PC, 0, 32 * s);
-#pragma unroll
-      for (int rt = 0; rt < 4; ++rt) U[rt] = mfma16x16x32<T>(frag(Tm, PC, 16 * rt, 32 * s), bf, U[rt]);
-    }
-    // U out through the wave's X1 buffer (its Y^T operand reads are done: in order, one wave)
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) put_t(X1[wave], PC, rt, U[rt]);
-    wave_sync();
-    store_cols(X1[wave], PC, std::integral_constant<int, C>{}, (T*)a.u + n * C * D);
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      f32x4 x;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) x[i] = Fs[C + rows_of(rt, i)] * U[rt][i];
-      put_t(X2[wave], PC, rt, x);
-    }
-    wave_sync();
-    // the entry state, then S <- Ga_C S + K^T diag(w) U
-    store_cols(Sb[wave], PD, std::integral_constant<int, D>{}, (T*)a.s_entry + n * D * D);  // S^T of this step
-    const float gC = Fs[3 * C];
-#pragma unroll
-    for (int t = 0; t < DT; ++t) S[t] *= gC;
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const u32x4 bf = frag(X2[wave], PC, 0, 32 * s);
-#pragma unroll
-      for (int t = 0; t < DT; ++t) S[t] = mfma16x16x32<T>(frag(Kt, PC, 16 * t, 32 * s), bf, S[t]);
-    }
+
+    return;
   }
 
   // ---------------------------------------------------------------- backward chain
@@ -256,37 +285,33 @@ __global__ void __launch_bounds__(64 * kChainWaves, 1) gdn_bwd16_chain_kernel(Bw
     for (int i = 0; i < 4; ++i)
       dS[t][i] = a.dst ? a.dst[((int64_t)bh * D + rows_of(t, i)) * D + col] : 0.f;
 
-  u32x4 rq[NT], rrt[NTM], ro[2], rgo[2];
+  u32x4 rq[NT], rrt[NTM], ro[2];
   auto bwd_load = [&](int64_t n) {
     tile_load<NT, NTH>(rk, (const T*)a.kr + n * C * D, tid);
-    tile_load<NT, NTH>(rkt, (const T*)a.kt + n * D * C, tid);
-    tile_load<NT, NTH>(rq, (const T*)a.qt + n * D * C, tid);
+    tile_load<NT, NTH>(rq, (const T*)a.qr + n * C * D, tid);
     tile_load<NTM, NTH>(rtm, (const T*)a.tt + n * C * C, tid);
     tile_load<NTM, NTH>(rrt, (const T*)a.rt + n * C * C, tid);
 #pragma unroll
     for (int j = 0; j < NF; ++j) rf[j] = a.f[n * kFRows * C + tid + NTH * j];
     rows16_load(ro, (const T*)a.ot + (n * D + v0) * C);
-    rows16_load(rgo, (const T*)a.got + (n * D + v0) * C);
   };
   bwd_load((int64_t)bh * a.NC + a.NC - 1);
   for (int c = a.NC - 1; c >= 0; --c) {
     const int64_t n = (int64_t)bh * a.NC + c;
     __syncthreads();
     tile_store<NT, D / 8, PD, NTH>(Kr, rk, tid);
-    tile_store<NT, 8, PC, NTH>(Kt, rkt, tid);
-    tile_store<NT, 8, PC, NTH>(Qt, rq, tid);
+    tile_store<NT, D / 8, PD, NTH>(Qr, rq, tid);
     tile_store<NTM, 8, PC, NTH>(Tm, rtm, tid);
     tile_store<NTM, 8, PC, NTH>(Rt, rrt, tid);
 #pragma unroll
     for (int j = 0; j < NF; ++j) Fs[tid + NTH * j] = rf[j];
-    rows16_store(XO[wave], ro);
-    rows16_store(XG[wave], rgo);
+    rows16_store(XO, ro);
     if (c > 0) bwd_load(n - 1);
 #pragma unroll
-    for (int t = 0; t < DT; ++t) put_t(Sb[wave], PD, t, dS[t]);
+    for (int t = 0; t < DT; ++t) put_t(Sb, PD, t, dS[t]);
     __syncthreads();
     // the exit-state gradient of this chunk, from its 16-bit transpose
-    store_cols(Sb[wave], PD, std::integral_constant<int, D>{}, (T*)a.ds_end + n * D * D);
+    store_cols(Sb, PD, std::integral_constant<int, D>{}, (T*)a.ds_end + n * D * D);
 
     // dU = diag(w) K dS + Rq^T dO
     f32x4 dU[4];
@@ -294,7 +319,7 @@ __global__ void __launch_bounds__(64 * kChainWaves, 1) gdn_bwd16_chain_kernel(Bw
     for (int rt = 0; rt < 4; ++rt) dU[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-      const u32x4 bf = frag(Sb[wave], PD, 0, 32 * s);
+      const u32x4 bf = frag(Sb, PD, 0, 32 * s);
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) dU[rt] = mfma16x16x32<T>(frag(Kr, PD, 16 * rt, 32 * s), bf, dU[rt]);
     }
@@ -304,12 +329,12 @@ __global__ void __launch_bounds__(64 * kChainWaves, 1) gdn_bwd16_chain_kernel(Bw
       for (int i = 0; i < 4; ++i) dU[rt][i] *= Fs[C + rows_of(rt, i)];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      const u32x4 bf = frag(XO[wave], PC, 0, 32 * s);
+      const u32x4 bf = frag(XO, PC, 0, 32 * s);
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) dU[rt] = mfma16x16x32<T>(frag(Rt, PC, 16 * rt, 32 * s), bf, dU[rt]);
     }
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) put_t(X1[wave], PC, rt, dU[rt]);
+    for (int rt = 0; rt < 4; ++rt) put_t(X1, PC, rt, dU[rt]);
     wave_sync();
     // dY = T^T dU
     f32x4 dY[4];
@@ -317,7 +342,7 @@ __global__ void __launch_bounds__(64 * kChainWaves, 1) gdn_bwd16_chain_kernel(Bw
     for (int rt = 0; rt < 4; ++rt) dY[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      const u32x4 bf = frag(X1[wave], PC, 0, 32 * s);
+      const u32x4 bf = frag(X1, PC, 0, 32 * s);
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) dY[rt] = mfma16x16x32<T>(frag(Tm, PC, 16 * rt, 32 * s), bf, dY[rt]);
     }
@@ -331,7 +356,7 @@ __global__ void __launch_bounds__(64 * kChainWaves, 1) gdn_bwd16_chain_kernel(Bw
         dyo[p * D + col] = dY[rt][i];
         x[i] = -Fs[p] * Fs[2 * C + p] * dY[rt][i];
       }
-      put_t(X2[wave], PC, rt, x);
+      put_t(X2, PC, rt, x);
     }
     wave_sync();
     // dS <- Ga_C dS + Q^T diag(Ga) dO - K^T diag(Ga beta) dY
@@ -340,12 +365,17 @@ __global__ void __launch_bounds__(64 * kChainWaves, 1) gdn_bwd16_chain_kernel(Bw
     for (int t = 0; t < DT; ++t) dS[t] *= gC;
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      const u32x4 b1 = frag(XG[wave], PC, 0, 32 * s);
-      const u32x4 b2 = frag(X2[wave], PC, 0, 32 * s);
+      u32x4 b1 = frag(XO, PC, 0, 32 * s);  // diag(Ga) dO, rounded as a 16-bit operand
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float* ga = Fs + 32 * s + 8 * g + 2 * e;
+        b1[e] = pack2<T>(ga[0] * elem16<T>(b1, 2 * e), ga[1] * elem16<T>(b1, 2 * e + 1));
+      }
+      const u32x4 b2 = frag(X2, PC, 0, 32 * s);
 #pragma unroll
       for (int t = 0; t < DT; ++t) {
-        dS[t] = mfma16x16x32<T>(frag(Qt, PC, 16 * t, 32 * s), b1, dS[t]);
-        dS[t] = mfma16x16x32<T>(frag(Kt, PC, 16 * t, 32 * s), b2, dS[t]);
+        dS[t] = mfma16x16x32<T>(frag_t(Qr, 16 * t, 32 * s), b1, dS[t]);
+        dS[t] = mfma16x16x32<T>(frag_t(Kr, 16 * t, 32 * s), b2, dS[t]);
       }
     }
   }
@@ -1020,26 +1050,25 @@ extern "C" int atma_gated_delta_bwd16_prep(const void* q, const void* k, const v
   return check_launch("gated_delta_bwd16_prep");
 }
 
-extern "C" int atma_gated_delta_bwd16_chain(const void* kr, const void* kt, const void* qt, const void* tm,
-                                            const void* tt, const void* rt, const void* vt, const void* ot,
-                                            const void* got, const float* f, const float* s0, const float* dst,
+extern "C" int atma_gated_delta_bwd16_chain(const void* kr, const void* qr, const void* tm, const void* tt,
+                                            const void* rt, const void* vt, const void* ot, const float* f, const float* s0, const float* dst,
                                             void* s_entry, void* ds_end, void* u, float* dy, float* ds0,
                                             int64_t BH, int64_t NC, int64_t d, int dtype, void* stream) {
   using namespace atma;
   if (!bwd16_dims_ok(d, dtype, "gated_delta_bwd16_chain")) return ATMA_ERR_UNSUPPORTED;
   if (BH < 0 || NC < 0) return set_error(ATMA_ERR_INVALID, "gated_delta_bwd16_chain: bad sizes");
   if (BH == 0 || NC == 0) return ATMA_OK;
-  if (!kr || !kt || !qt || !tm || !tt || !rt || !vt || !ot || !got || !f || !s_entry || !ds_end || !u || !dy ||
+  if (!kr || !qr || !tm || !tt || !rt || !vt || !ot || !f || !s_entry || !ds_end || !u || !dy ||
       !ds0)
     return set_error(ATMA_ERR_INVALID, "gated_delta_bwd16_chain: null pointer");
-  if (!aligned16({kr, kt, qt, tm, tt, rt, vt, ot, got, s_entry, ds_end, u, dy}))
+  if (!aligned16({kr, qr, tm, tt, rt, vt, ot, s_entry, ds_end, u, dy}))
     return set_error(ATMA_ERR_INVALID, "gated_delta_bwd16_chain: tiles and outputs must be 16-byte aligned");
   const int64_t slabs = d / (16 * kChainWaves);  // column slabs (workgroups) per sequence-head
-  if (BH * slabs > 0x7fffffff || BH * NC > 0x7fffffff)
+  if (2 * BH * slabs > 0x7fffffff || BH * NC > 0x7fffffff)
     return set_error(ATMA_ERR_INVALID, "gated_delta_bwd16_chain: sizes too large");
-  Bwd16ChainArgs a{kr, kt, qt, tm, tt, rt, vt, ot, got, f, s0, dst, s_entry, ds_end, u, dy, ds0,
+  Bwd16ChainArgs a{kr, qr, tm, tt, rt, vt, ot, f, s0, dst, s_entry, ds_end, u, dy, ds0,
                    (int)BH, (int)NC};
-  const dim3 grid((unsigned)(BH * slabs));
+  const dim3 grid((unsigned)(2 * BH * slabs));
   ATMA_BWD16_DISPATCH_NT(gdn_bwd16_chain_kernel, grid, 64 * kChainWaves, (hipStream_t)stream, a);
   return check_launch("gated_delta_bwd16_chain");
 }

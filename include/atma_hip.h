@@ -365,7 +365,7 @@ int atma_gated_delta_bwd(const float* q, const float* k, const float* v, const f
  * ik = 1 / max(|k|, eps), uq2 = 1 / |q|^2, uk2 = 1 / |k|^2 (0 where |x| <= eps; without
  * l2norm: scale, 1, 0, 0) -- f is (N, 9, 64).
  *
- * chain: the prep's tiles (BH = B * H); s0, dst (BH, d, d) [K, V] fp32 initial state and
+ * chain: the prep's kr, qr, tm, tt, rt, vt, ot, f (BH = B * H); s0, dst (BH, d, d) [K, V] fp32 initial state and
  * final-state cotangent, or NULL (zero).  Runs the state forward over the chunks, then the
  * state gradient backwards (dU = Rq^T dO + diag(w) K dS, dY = T^T dU,
  * dS <- Ga_C dS + Q^T diag(Ga) dO - K^T diag(Ga beta) dY), writing s_entry and ds_end
@@ -382,9 +382,8 @@ int atma_gated_delta_bwd16_prep(const void* q, const void* k, const void* v, con
                                 void* tm, void* tt, void* rt, void* vt, void* ot, void* got, float* f,
                                 int64_t B, int64_t T, int64_t H, int64_t d, float scale, int l2norm, int dtype,
                                 void* stream);
-int atma_gated_delta_bwd16_chain(const void* kr, const void* kt, const void* qt, const void* tm,
-                                 const void* tt, const void* rt, const void* vt, const void* ot,
-                                 const void* got, const float* f, const float* s0, const float* dst,
+int atma_gated_delta_bwd16_chain(const void* kr, const void* qr, const void* tm, const void* tt,
+                                 const void* rt, const void* vt, const void* ot, const float* f, const float* s0, const float* dst,
                                  void* s_entry, void* ds_end, void* u, float* dy, float* ds0, int64_t BH,
                                  int64_t NC, int64_t d, int dtype, void* stream);
 int atma_gated_delta_bwd16_local(const void* kr, const void* kt, const void* qr, const void* qt,

@@ -460,16 +460,16 @@ def _bwd16_prep(q, k, v, d_out, g, beta, scale, l2norm):
     BH = B * H
     t16 = dict(device=q.device, dtype=v.dtype)
     kr, qr = (torch.empty((BH, NC, 64, d), **t16) for _ in range(2))
-    kt, qt, vt, ot, got = (torch.empty((BH, NC, d, 64), **t16) for _ in range(5))
+    vt, ot = (torch.empty((BH, NC, d, 64), **t16) for _ in range(2))
     tm, tt, rt = (torch.empty((BH, NC, 64, 64), **t16) for _ in range(3))
     f = torch.empty((BH, NC, 9, 64), device=q.device, dtype=torch.float32)
     rc = lib.atma_gated_delta_bwd16_prep(q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), g.data_ptr(),
-                                         beta.data_ptr(), kr.data_ptr(), kt.data_ptr(), qr.data_ptr(), qt.data_ptr(),
-                                         tm.data_ptr(), tt.data_ptr(), rt.data_ptr(), vt.data_ptr(), ot.data_ptr(),
-                                         got.data_ptr(), f.data_ptr(), B, T, H, d, float(scale), 1 if l2norm else 0,
-                                         _lib.dtype_code(v.dtype), _lib.stream_handle(q.device))
+                                         beta.data_ptr(), kr.data_ptr(), qr.data_ptr(), tm.data_ptr(), tt.data_ptr(),
+                                         rt.data_ptr(), vt.data_ptr(), ot.data_ptr(), f.data_ptr(), B, T, H,
+                                         k.shape[2], d, float(scale), 1 if l2norm else 0, _lib.dtype_code(v.dtype),
+                                         _lib.stream_handle(q.device))
     _lib.check(rc, "gated_delta_bwd16_prep")
-    return [kr, kt, qr, qt, tm, tt, rt, vt, ot, got, f]
+    return [kr, qr, tm, tt, rt, vt, ot, f]
 
 
 def _bwd16_chain(kr, qr, tm, tt, rt, vt, ot, f, s0, dst):
@@ -489,17 +489,17 @@ def _bwd16_chain(kr, qr, tm, tt, rt, vt, ot, f, s0, dst):
     return [s_entry, ds_end, u, dy, ds0]
 
 
-def _bwd16_local(kr, kt, qr, qt, q, k, v, d_out, f, s_entry, ds_end, u, dy):
+def _bwd16_local(q, k, v, d_out, f, s_entry, ds_end, u, dy):
     lib = _lib.load()
     B, T, H, d = q.shape
     t16 = dict(device=q.device, dtype=q.dtype)
     dq, dk, dv = (torch.empty((B, T, H, d), **t16) for _ in range(3))
     dg, db = (torch.empty((B, T, H), device=q.device, dtype=torch.float32) for _ in range(2))
-    rc = lib.atma_gated_delta_bwd16_local(kr.data_ptr(), kt.data_ptr(), qr.data_ptr(), qt.data_ptr(), q.data_ptr(),
-                                          k.data_ptr(), v.data_ptr(), d_out.data_ptr(), f.data_ptr(),
+    rc = lib.atma_gated_delta_bwd16_local(q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), f.data_ptr(),
                                           s_entry.data_ptr(), ds_end.data_ptr(), u.data_ptr(), dy.data_ptr(),
                                           dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dg.data_ptr(), db.data_ptr(),
-                                          B, T, H, d, _lib.dtype_code(q.dtype), _lib.stream_handle(q.device))
+                                          B, T, H, k.shape[2], d, _lib.dtype_code(q.dtype),
+                                          _lib.stream_handle(q.device))
     _lib.check(rc, "gated_delta_bwd16_local")
     return [dq, dk, dv, dg, db]
 
@@ -530,9 +530,9 @@ def gated_delta_bwd16_op(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tenso
             dst.reshape(B, H, d, d).clone()
         return [torch.zeros_like(q), torch.zeros_like(k), torch.zeros_like(v), torch.zeros_like(g),
                 torch.zeros_like(beta), ds0]
-    kr, kt, qr, qt, tm, tt, rt, vt, ot, got, f = _bwd16_prep(q, k, v, d_out, g, beta, scale, l2norm)
+    kr, qr, tm, tt, rt, vt, ot, f = _bwd16_prep(q, k, v, d_out, g, beta, scale, l2norm)
     s_entry, ds_end, u, dy, ds0 = _bwd16_chain(kr, qr, tm, tt, rt, vt, ot, f, s0, dst)
-    dq, dk, dv, dg, db = _bwd16_local(kr, kt, qr, qt, q, k, v, d_out, f, s_entry, ds_end, u, dy)
+    dq, dk, dv, dg, db = _bwd16_local(q, k, v, d_out, f, s_entry, ds_end, u, dy)
     return [dq, dk, dv, dg, db, ds0.reshape(B, H, d, d)]
 
 
@@ -545,18 +545,20 @@ def _(q, k, v, g, beta, initial_state, d_out, d_final_state, scale, l2norm):
 
 def gated_delta_bwd16_stages(q, k, v, g, beta, initial_state, d_out, d_final_state, scale, l2norm):
     """The three launches of ``gated_delta_bwd16`` with every intermediate returned (for
-    tests): dict of the prep's tiles (kr, kt, qr, qt, tm, tt, rt, vt, ot, got, f; chunk-head
-    tensors shaped (B*H, NC, ...)), the chain's outputs (s_entry, ds_end, u, dy, ds0) and
-    the local gradients (dq, dk, dv, dg, db)."""
+    tests): dict of the prep's tiles (kr, qr, tm, tt, rt, vt, ot, f; chunk-head tensors shaped
+    (B*H, NC, ...)) with the transposes and the decayed output gradient that the other two form
+    from them (kt, qt, got), the chain's outputs (s_entry, ds_end, u, dy, ds0) and the local
+    gradients (dq, dk, dv, dg, db)."""
     q, k, v, d_out, g, beta = _bwd16_check(q, k, v, d_out, g, beta)
     B, T, H, d = q.shape
     s0, dst = _bwd16_states(initial_state, d_final_state, B, H, d)
-    names = ["kr", "kt", "qr", "qt", "tm", "tt", "rt", "vt", "ot", "got", "f"]
+    names = ["kr", "qr", "tm", "tt", "rt", "vt", "ot", "f"]
     out = dict(zip(names, _bwd16_prep(q, k, v, d_out, g, beta, scale, l2norm)))
-    chain = _bwd16_chain(*(out[n] for n in ("kr", "qr", "tm", "tt", "rt", "vt", "ot", "f")), s0, dst)
+    out.update(kt=out["kr"].transpose(-1, -2), qt=out["qr"].transpose(-1, -2),
+               got=(out["f"][:, :, None, 0] * out["ot"].float()).to(v.dtype))
+    chain = _bwd16_chain(*(out[n] for n in names), s0, dst)
     out.update(zip(["s_entry", "ds_end", "u", "dy", "ds0"], chain))
-    loc = _bwd16_local(out["kr"], out["kt"], out["qr"], out["qt"], q, k, v, d_out, out["f"], out["s_entry"],
-                       out["ds_end"], out["u"], out["dy"])
+    loc = _bwd16_local(q, k, v, d_out, out["f"], out["s_entry"], out["ds_end"], out["u"], out["dy"])
     out.update(zip(["dq", "dk", "dv", "dg", "db"], loc))
     return out
 

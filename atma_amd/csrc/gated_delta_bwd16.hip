@@ -393,20 +393,20 @@ __global__ void __launch_bounds__(64 * kChainWaves, 1) gdn_bwd16_chain_kernel(Bw
 // N = diag(beta) A (fp32, LDS); then wave 0 inverts I + N -- the four diagonal blocks by
 // forward substitution (lane (g, c) solves column c of block g), the blocks below them by
 // fp32 block products on v_mfma_f32_16x16x4f32 -- while waves 1-3 write the transposed
-// tiles k^T, q^T, v^T, dO^T and (diag(Ga) dO)^T from the LDS rows by transposing reads;
+// tiles v^T and dO^T from the LDS rows by transposing reads;
 // last, every wave writes T and T^T.
 struct Bwd16PrepArgs {
   const void* q;      // (B, T, H, D) 16-bit, raw
-  const void* k;      // (B, T, H, D) 16-bit, raw
-  const void* v;      // (B, T, H, D) 16-bit
   const void* dO;     // (B, T, H, D) 16-bit
+  const void* k;      // (B, T, H / G, D) 16-bit, raw
+  const void* v;      // (B, T, H / G, D) 16-bit
   const float* g;     // (B, T, H) log decay
   const float* beta;  // (B, T, H)
-  void *kr, *kt, *qr, *qt, *tm, *tt, *rt, *vt, *ot, *got;
+  void *kr, *qr, *tm, *tt, *rt, *vt, *ot;
   float* f;
   float scale;
   int l2norm;
-  int B, T, H, NC;
+  int B, T, H, NC, G;
 };
 
 // Sum over each group of 8 lanes (the two quads of each half row), in every lane.
@@ -435,7 +435,7 @@ __global__ void __launch_bounds__(256) gdn_bwd16_prep_kernel(Bwd16PrepArgs a) {
   // overwrites all of it at the end (84 KiB in all would allow one workgroup per CU; 79 KiB
   // allows two, so one's loads overlap the other's products)
   __shared__ __attribute__((aligned(16))) float Nd[4 * 256 + 6 * 256];
-  __shared__ float Lg[C], Bt[C], Gs[C];
+  __shared__ float Lg[C], Bt[C];
   float* Mb = Nd;  // T^T of the diagonal blocks
   T* Tl = (T*)Nd;  // T, row-major, pitch PT
   static_assert(C * PT * (int)sizeof(T) <= (int)sizeof(Nd), "T fits the N blocks' bytes");
@@ -448,8 +448,8 @@ __global__ void __launch_bounds__(256) gdn_bwd16_prep_kernel(Bwd16PrepArgs a) {
   const int b = bh / a.H, h = bh % a.H;
   const int rows = min(a.T - c * C, C);
   const int64_t tok0 = (int64_t)b * a.T + (int64_t)c * C;
-  const int64_t rs = (int64_t)a.H * D;  // token stride (elements)
-  const int64_t base = tok0 * rs + (int64_t)h * D;
+  const int64_t rs = (int64_t)a.H * D, krs = (int64_t)(a.H / a.G) * D;  // token strides (elements)
+  const int64_t base = tok0 * rs + (int64_t)h * D, kbase = tok0 * krs + (int64_t)(h / a.G) * D;
 
   // rows (zero past the sequence's end), all loads issued before the stores
   {
@@ -459,10 +459,10 @@ __global__ void __launch_bounds__(256) gdn_bwd16_prep_kernel(Bwd16PrepArgs a) {
       const int i = tid + 256 * j, r = i / (D / 8), ch = i % (D / 8);
       kx[j] = qx[j] = vx[j] = ox[j] = u32x4{0u, 0u, 0u, 0u};
       if (r < rows) {
-        const int64_t o = base + r * rs + 8 * ch;
-        kx[j] = *(const u32x4*)((const T*)a.k + o);
+        const int64_t o = base + r * rs + 8 * ch, ok = kbase + r * krs + 8 * ch;
+        kx[j] = *(const u32x4*)((const T*)a.k + ok);
         qx[j] = *(const u32x4*)((const T*)a.q + o);
-        vx[j] = *(const u32x4*)((const T*)a.v + o);
+        vx[j] = *(const u32x4*)((const T*)a.v + ok);
         ox[j] = *(const u32x4*)((const T*)a.dO + o);
       }
     }
@@ -523,7 +523,6 @@ __global__ void __launch_bounds__(256) gdn_bwd16_prep_kernel(Bwd16PrepArgs a) {
       const float ga = exp_hw(lg);
       Lg[lane] = lg;
       Bt[lane] = bt;
-      Gs[lane] = ga;
       fo[lane] = ga;
       fo[C + lane] = exp_hw(lgC - lg);
       fo[2 * C + lane] = bt;
@@ -651,21 +650,14 @@ __global__ void __launch_bounds__(256) gdn_bwd16_prep_kernel(Bwd16PrepArgs a) {
     // tokens r0 .. r0 + 7 of column c0 + i, one 16-byte chunk of row d = c0 + i of the tile
     const int gi = (tid - 64) >> 4, sl = lane & 15;  // 12 groups of 16 lanes
     const int rr = sl >> 2, cc = 4 * (sl & 3);
-    constexpr int UNITS = 5 * (D / 16) * 8;          // (tile, 16-column block, 8-row block)
+    constexpr int UNITS = 2 * (D / 16) * 8;          // (tile, 16-column block, 8-row block)
     for (int u = gi; u < UNITS; u += 12) {
       const int tile = u / ((D / 16) * 8), rem = u % ((D / 16) * 8);
       const int c0 = 16 * (rem / 8), r0 = 8 * (rem % 8);
-      const T* src = tile == 0 ? Ks : tile == 1 ? Qs : tile == 2 ? Vs : Os;
+      const T* src = tile == 0 ? Vs : Os;
       const u32x2 lo = lds_read_tr16(src + (r0 + rr) * PD + c0 + cc);
       const u32x2 hi = lds_read_tr16(src + (r0 + 4 + rr) * PD + c0 + cc);
-      u32x4 w = {lo[0], lo[1], hi[0], hi[1]};
-      if (tile == 4) {  // (diag(Ga) dO)^T
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          w[e] = pack2<T>(Gs[r0 + 2 * e] * elem16<T>(w, 2 * e), Gs[r0 + 2 * e + 1] * elem16<T>(w, 2 * e + 1));
-      }
-      void* dst = tile == 0 ? a.kt : tile == 1 ? a.qt : tile == 2 ? a.vt : tile == 3 ? a.ot : a.got;
-      *(u32x4*)((T*)dst + (n * D + c0 + sl) * C + r0) = w;
+      *(u32x4*)((T*)(tile == 0 ? a.vt : a.ot) + (n * D + c0 + sl) * C + r0) = u32x4{lo[0], lo[1], hi[0], hi[1]};
     }
   }
   __syncthreads();
@@ -690,44 +682,47 @@ __global__ void __launch_bounds__(256) gdn_bwd16_prep_kernel(Bwd16PrepArgs a) {
 }
 
 // ------------------------------------------------------------------------------ local
-// One workgroup per chunk-head item n (4 waves); wave w owns token rows 16 w .. 16 w + 15 of
-// every row-indexed product.  Staged in LDS: the entry state S0 (then the exit-state
-// gradient dS, same buffer), U, k rows, k^T, q^T, and the 64 x 64 weight matrices
-// GA + GA^T, GR, GR^T built by the waves.  Products on v_mfma_f32_16x16x32 (16-bit
-// operands, fp32 accumulation): K K^T, Q K^T, dY U^T, dO U^T (64 x 64), dY S0^T, dO S0^T,
-// U dS^T (64 x d), then dK = (GA + GA^T) K + GR^T Q - diag(Ga beta) dY S0^T + diag(w) U dS^T
+// One workgroup per chunk-head item n (4 waves); wave w owns tokens 16 w .. 16 w + 15.
+// Products on v_mfma_f32_16x16x32 (16-bit operands, fp32 accumulation): K K^T, Q K^T,
+// dY U^T, dO U^T (64 x 64) give the weights GA, GR; then, transposed (rows = d, columns = the
+// wave's tokens, so that a lane holds four consecutive d of one token),
+// dK = (GA + GA^T) K + GR^T Q - diag(Ga beta) dY S0^T + diag(w) U dS^T
 // and dQ = GR K + diag(Ga) dO S0^T.  The sums over d that the gradients of beta and the
 // log decays take reduce to row sums of these products with k and q:
 // rowsum(dY o K S0) = rowsum(K o dY S0^T), rowsum(dO o Q S0) = rowsum(Q o dO S0^T),
 // rowsum(K dS o U) = rowsum(K o U dS^T).
+// The k and q rows are normalised and rounded from the raw ones as the prep does (the raw
+// ones are needed for the l2 norm's backward anyway).  LDS: k rows, GA^T and GR^T (their
+// transposes, like those of the rows, by transposing reads), and two row tiles that hold U and q
+// first and the entry state S0, then the exit-state gradient dS, afterwards: 75 KiB and at most 256
+// registers, so two workgroups share a CU and one's loads pass under the other's products.
+// Bound by memory: an item reads 192 KiB and writes 49 at d = 128.  8 sequences of 2,048
+// tokens, 8 heads: 123 us; 249 with one workgroup per CU (147 KiB of LDS: each transpose a tile
+// of its own, S0 and dS beside the rest), k^T and q^T read from memory and 2-byte accesses to
+// the raw rows and the outputs.
 struct Bwd16LocalArgs {
-  const void *kr, *kt, *qr, *qt;
-  const void* v;   // (B, T, H, D) 16-bit
-  const void* dO;  // (B, T, H, D) 16-bit
-  const void *q, *k;  // (B, T, H, D) 16-bit, raw (the l2 norm's backward)
-  const float* f;  // [N][kFRows][64]
+  const void *q, *dO;  // (B, T, H, D) 16-bit (q raw)
+  const void *k, *v;   // (B, T, H / G, D) 16-bit (k raw)
+  const float* f;      // [N][kFRows][64]
   const void *s_entry, *ds_end, *u;
   const float* dy;
   void *dq, *dk, *dv;  // (B, T, H, D) 16-bit
-  float *dg, *db;  // (B, T, H)
-  int B, T, H, NC;
+  float *dg, *db;      // (B, T, H)
+  int B, T, H, NC, G;
 };
 
 template <typename T, int D>
-__global__ void __launch_bounds__(256, 1) gdn_bwd16_local_kernel(Bwd16LocalArgs a) {
+__global__ void __launch_bounds__(256, 2) gdn_bwd16_local_kernel(Bwd16LocalArgs a) {
   constexpr int C = 64, PD = D + 8, PC = C + 8, KS = D / 32, DT = D / 16, NT = D / 32, NSS = D * D / 2048;
-  __shared__ __attribute__((aligned(16))) T SS[D * PD];
-  __shared__ __attribute__((aligned(16))) T Us[C * PD];
   __shared__ __attribute__((aligned(16))) T Kr[C * PD];
-  __shared__ __attribute__((aligned(16))) T Kt[D * PC];
-  __shared__ __attribute__((aligned(16))) T Qt[D * PC];
-  __shared__ __attribute__((aligned(16))) T M1[C * PC];   // GA
-  __shared__ __attribute__((aligned(16))) T M1t[C * PC];  // GA^T
-  __shared__ __attribute__((aligned(16))) T GRs[C * PC];  // GR
-  __shared__ __attribute__((aligned(16))) T GRt[C * PC];  // GR^T
+  __shared__ __attribute__((aligned(16))) T SS[2 * C * PD];  // U and q rows, then S0 rows, then dS rows
+  __shared__ __attribute__((aligned(16))) T GAt[C * PC];     // GA^T
+  __shared__ __attribute__((aligned(16))) T GRt[C * PC];     // GR^T
   __shared__ float Fs[kFRows * C];
   __shared__ float colp[4][C];
-  __shared__ float dyv[C], dlgs[C], red[2][4];
+  __shared__ float dyv[C], dbv[C], dlgs[C], red[2][4];
+  T* Us = SS;
+  T* Qr = SS + C * PD;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -737,65 +732,66 @@ __global__ void __launch_bounds__(256, 1) gdn_bwd16_local_kernel(Bwd16LocalArgs 
   const int b = bh / a.H, h = bh % a.H;
   const int rows = min(a.T - c * C, C);
   const int64_t tok0 = (int64_t)b * a.T + (int64_t)c * C;
-  const int64_t rs = (int64_t)a.H * D;
-  const int64_t base = tok0 * rs + (int64_t)h * D;
-  const int ra = 16 * wave + c16;  // the lane's row as an A operand
+  const int64_t rs = (int64_t)a.H * D, krs = (int64_t)(a.H / a.G) * D;  // token strides
+  const int64_t base = tok0 * rs + (int64_t)h * D, kbase = tok0 * krs + (int64_t)(h / a.G) * D;
+  const int ra = 16 * wave + c16;  // the lane's token
+  const float* fn = a.f + n * kFRows * C;
 
-  // staged tiles and the wave's A-operand rows, all loads first
-  u32x4 rss[NSS], rds[NSS], ru[NT], rk[NT], rkt[NT], rqt[NT];
-  tile_load(rss, (const T*)a.s_entry + n * D * D, tid);
-  tile_load(rds, (const T*)a.ds_end + n * D * D, tid);
-  tile_load(ru, (const T*)a.u + n * C * D, tid);
-  tile_load(rk, (const T*)a.kr + n * C * D, tid);
-  tile_load(rkt, (const T*)a.kt + n * D * C, tid);
-  tile_load(rqt, (const T*)a.qt + n * D * C, tid);
-  f32x4 dyl[KS][2];
-  u32x4 doA[KS], vA[KS], uA[KS], kA[KS], qA[KS];
+  // fragment of rows row0 .. of a row tile; of its transpose (rows col0 .., k = the tile's rows k0 + 8 g ..)
+  auto frag = [&](const T* tile, int pitch, int row0, int k0) {
+    return *(const u32x4*)(tile + (row0 + c16) * pitch + k0 + 8 * g);
+  };
+  auto frag_t = [&](const T* tile, int pitch, int col0, int k0) {
+    const T* p = tile + (k0 + 8 * g + (c16 >> 2)) * pitch + col0 + 4 * (c16 & 3);
+    const u32x2 lo = lds_read_tr16(p), hi = lds_read_tr16(p + 4 * pitch);
+    return u32x4{lo[0], lo[1], hi[0], hi[1]};
+  };
+
+  // ---- k, q (normalised, rounded) and U rows into LDS; the wave's dY, dO and v rows
+  u32x4 doA[KS], dyA[KS], kA[KS], qA[KS];
+  {
+    u32x4 rk[NT], rq[NT], ru[NT], vA[KS];
+    float fk[NT], fq[NT];
+    tile_load(ru, (const T*)a.u + n * C * D, tid);
 #pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    const float* yr = a.dy + (n * C + ra) * D + 32 * s + 8 * g;
-    dyl[s][0] = *(const f32x4*)yr;
-    dyl[s][1] = *(const f32x4*)(yr + 4);
-    doA[s] = vA[s] = u32x4{0u, 0u, 0u, 0u};
-    if (ra < rows) {
-      doA[s] = *(const u32x4*)((const T*)a.dO + base + ra * rs + 32 * s + 8 * g);
-      vA[s] = *(const u32x4*)((const T*)a.v + base + ra * rs + 32 * s + 8 * g);
+    for (int j = 0; j < NT; ++j) {
+      const int i = tid + 256 * j, r = i / (D / 8), ch = i % (D / 8);
+      rk[j] = rq[j] = u32x4{0u, 0u, 0u, 0u};
+      if (r < rows) {
+        rk[j] = *(const u32x4*)((const T*)a.k + kbase + r * krs + 8 * ch);
+        rq[j] = *(const u32x4*)((const T*)a.q + base + r * rs + 8 * ch);
+      }
+      fq[j] = fn[5 * C + r];
+      fk[j] = fn[6 * C + r];
     }
-    uA[s] = *(const u32x4*)((const T*)a.u + (n * C + ra) * D + 32 * s + 8 * g);
-    kA[s] = *(const u32x4*)((const T*)a.kr + (n * C + ra) * D + 32 * s + 8 * g);
-    qA[s] = *(const u32x4*)((const T*)a.qr + (n * C + ra) * D + 32 * s + 8 * g);
-  }
-  for (int i = tid; i < kFRows * C; i += 256) Fs[i] = a.f[n * kFRows * C + i];
-  // the raw k and q elements of the lane's dK / dQ tile entries (row 16 wave + 4g + i, column
-  // 16 t + c16), for the l2 norm's backward at the end: loaded now, so their latency passes
-  // under the products
-  T kraw16[DT][4], qraw16[DT][4];
+    f32x4 dyl[KS][2];
 #pragma unroll
-  for (int t = 0; t < DT; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int p = 16 * wave + 4 * g + i;
-      kraw16[t][i] = qraw16[t][i] = from_f32<T>(0.f);
-      if (p < rows) {
-        kraw16[t][i] = ((const T*)a.k)[base + p * rs + 16 * t + c16];
-        qraw16[t][i] = ((const T*)a.q)[base + p * rs + 16 * t + c16];
+    for (int s = 0; s < KS; ++s) {
+      const float* yr = a.dy + (n * C + ra) * D + 32 * s + 8 * g;
+      dyl[s][0] = *(const f32x4*)yr;
+      dyl[s][1] = *(const f32x4*)(yr + 4);
+      doA[s] = vA[s] = u32x4{0u, 0u, 0u, 0u};
+      if (ra < rows) {
+        doA[s] = *(const u32x4*)((const T*)a.dO + base + ra * rs + 32 * s + 8 * g);
+        vA[s] = *(const u32x4*)((const T*)a.v + kbase + ra * krs + 32 * s + 8 * g);
       }
     }
-  tile_store<NSS, D / 8, PD>(SS, rss, tid);
-  tile_store<NT, D / 8, PD>(Us, ru, tid);
-  tile_store<NT, D / 8, PD>(Kr, rk, tid);
-  tile_store<NT, 8, PC>(Kt, rkt, tid);
-  tile_store<NT, 8, PC>(Qt, rqt, tid);
-  const float* Ga = Fs;
-  const float* Wf = Fs + C;
-  const float* Bf = Fs + 2 * C;
-  const float* Lgf = Fs + 4 * C;
-  __syncthreads();
-
-  // dV = diag(beta) dY and rowsum(dY o V) from the wave's rows; dY as A operand
-  u32x4 dyA[KS];
-  {
-    const float bt = Bf[ra];
+    const float bt = fn[2 * C + ra];
+    for (int i = tid; i < kFRows * C; i += 256) Fs[i] = fn[i];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int i = tid + 256 * j, r = i / (D / 8), ch = i % (D / 8);
+      u32x4 kp, qp;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        kp[e] = pack2<T>(fk[j] * elem16<T>(rk[j], 2 * e), fk[j] * elem16<T>(rk[j], 2 * e + 1));
+        qp[e] = pack2<T>(fq[j] * elem16<T>(rq[j], 2 * e), fq[j] * elem16<T>(rq[j], 2 * e + 1));
+      }
+      *(u32x4*)(Kr + r * PD + 8 * ch) = kp;
+      *(u32x4*)(Qr + r * PD + 8 * ch) = qp;
+    }
+    tile_store<NT, D / 8, PD>(Us, ru, tid);
+    // dV = diag(beta) dY and rowsum(dY o V) from the wave's rows; dY as an operand
     float part = 0.f;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
@@ -812,68 +808,137 @@ __global__ void __launch_bounds__(256, 1) gdn_bwd16_local_kernel(Bwd16LocalArgs 
     part += __shfl_xor(part, 32, 64);
     if (g == 0) dyv[ra] = part;
   }
+  const float* Bf = Fs + 2 * C;
+  const float* Lgf = Fs + 4 * C;
+  u32x4 rss[NSS];  // S0, stored to LDS once U and q are done with
+  tile_load(rss, (const T*)a.s_entry + n * D * D, tid);
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    kA[s] = frag(Kr, PD, 16 * wave, 32 * s);
+    qA[s] = frag(Qr, PD, 16 * wave, 32 * s);
+  }
 
-  // 64 x 64 products of the wave's rows: A, Rq, dL, dRq, and the weights GA, GR
-  float dbl[4] = {0.f, 0.f, 0.f, 0.f}, lgl[4] = {0.f, 0.f, 0.f, 0.f};
+  // ---- 64 x 64 products of the wave's rows: A, Rq, dL, dRq, and the weights GA, GR
+  {
+    float dbl[4] = {0.f, 0.f, 0.f, 0.f}, lgl[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int S = 0; S < 4; ++S) {
-    f32x4 kk = {0.f, 0.f, 0.f, 0.f}, qk = kk, yl = kk, ou = kk;
+    for (int S = 0; S < 4; ++S) {
+      f32x4 kk = {0.f, 0.f, 0.f, 0.f}, qk = kk, yl = kk, ou = kk;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const u32x4 kb = *(const u32x4*)(Kr + (16 * S + c16) * PD + 32 * s + 8 * g);
-      const u32x4 ub = *(const u32x4*)(Us + (16 * S + c16) * PD + 32 * s + 8 * g);
-      kk = mfma16x16x32<T>(kA[s], kb, kk);
-      qk = mfma16x16x32<T>(qA[s], kb, qk);
-      yl = mfma16x16x32<T>(dyA[s], ub, yl);
-      ou = mfma16x16x32<T>(doA[s], ub, ou);
+      for (int s = 0; s < KS; ++s) {
+        const u32x4 kb = frag(Kr, PD, 16 * S, 32 * s), ub = frag(Us, PD, 16 * S, 32 * s);
+        kk = mfma16x16x32<T>(kA[s], kb, kk);
+        qk = mfma16x16x32<T>(qA[s], kb, qk);
+        yl = mfma16x16x32<T>(dyA[s], ub, yl);
+        ou = mfma16x16x32<T>(doA[s], ub, ou);
+      }
+      const int sc = 16 * S + c16, p0 = 16 * wave + 4 * g;
+      const float lgs = Lgf[sc];
+      f32x4 ga, gr;
+      float colv = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int p = p0 + i;
+        const float e = sc <= p ? exp_hw(Lgf[p] - lgs) : 0.f;
+        const float A = sc < p ? e * kk[i] : 0.f;
+        const float Rq = e * qk[i];
+        const float dL = sc < p ? -yl[i] : 0.f;
+        const float dA = Bf[p] * dL;
+        const float dRq = sc <= p ? ou[i] : 0.f;
+        ga[i] = dA * e;
+        gr[i] = dRq * e;
+        dbl[i] = fmaf(dL, A, dbl[i]);
+        const float x = fmaf(dA, A, dRq * Rq);
+        lgl[i] += x;
+        colv += x;
+      }
+      *(u32x2*)(GAt + sc * PC + p0) = u32x2{pack2<T>(ga[0], ga[1]), pack2<T>(ga[2], ga[3])};
+      *(u32x2*)(GRt + sc * PC + p0) = u32x2{pack2<T>(gr[0], gr[1]), pack2<T>(gr[2], gr[3])};
+      colv += __shfl_xor(colv, 16, 64);
+      colv += __shfl_xor(colv, 32, 64);
+      if (g == 0) colp[wave][sc] = colv;
     }
-    const int sc = 16 * S + c16;
-    const float lgs = Lgf[sc];
-    f32x4 ga, gr;
-    float colv = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int p = 16 * wave + 4 * g + i;
-      const float e = sc <= p ? exp_hw(Lgf[p] - lgs) : 0.f;
-      const float A = sc < p ? e * kk[i] : 0.f;
-      const float Rq = e * qk[i];
-      const float dL = sc < p ? -yl[i] : 0.f;
-      const float dA = Bf[p] * dL;
-      const float dRq = sc <= p ? ou[i] : 0.f;
-      ga[i] = dA * e;
-      gr[i] = dRq * e;
-      dbl[i] = fmaf(dL, A, dbl[i]);
-      const float x = fmaf(dA, A, dRq * Rq);
-      lgl[i] += x;
-      colv += x;
-      M1[p * PC + sc] = from_f32<T>(ga[i]);
-      GRs[p * PC + sc] = from_f32<T>(gr[i]);
+      const float x = row16_sum(dbl[i]), y = row16_sum(lgl[i]);
+      if (c16 == 0) {
+        dbv[16 * wave + 4 * g + i] = x;
+        dlgs[16 * wave + 4 * g + i] = y;
+      }
     }
-    const int p0 = 16 * wave + 4 * g;
-    *(u32x2*)(M1t + sc * PC + p0) = u32x2{pack2<T>(ga[0], ga[1]), pack2<T>(ga[2], ga[3])};
-    *(u32x2*)(GRt + sc * PC + p0) = u32x2{pack2<T>(gr[0], gr[1]), pack2<T>(gr[2], gr[3])};
-    colv += __shfl_xor(colv, 16, 64);
-    colv += __shfl_xor(colv, 32, 64);
-    if (g == 0) colp[wave][sc] = colv;
   }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    dbl[i] = row16_sum(dbl[i]);
-    lgl[i] = row16_sum(lgl[i]);
-  }
+  __syncthreads();
 
-  // dY S0^T and dO S0^T (B operand: S0 rows = output columns)
-  f32x4 P1[DT], P2[DT], P3[DT];
+  // ---- (GA + GA^T) K + GR^T Q and GR K, transposed: register i of tile t is d = 16 t + 4 g + i of token ra
+  f32x4 dKn[DT], dQs[DT];
+  {
+    u32x4 g1[2], grt[2], gr[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const u32x4 mt = frag(GAt, PC, 16 * wave, 32 * j), m = frag_t(GAt, PC, 16 * wave, 32 * j);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        g1[j][e] = pack2<T>(elem16<T>(m, 2 * e) + elem16<T>(mt, 2 * e), elem16<T>(m, 2 * e + 1) + elem16<T>(mt, 2 * e + 1));
+      grt[j] = frag(GRt, PC, 16 * wave, 32 * j);
+      gr[j] = frag_t(GRt, PC, 16 * wave, 32 * j);
+    }
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+      dKn[t] = dQs[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const u32x4 kb = frag_t(Kr, PD, 16 * t, 32 * j), qb = frag_t(Qr, PD, 16 * t, 32 * j);
+        dKn[t] = mfma16x16x32<T>(kb, g1[j], dKn[t]);
+        dKn[t] = mfma16x16x32<T>(qb, grt[j], dKn[t]);
+        dQs[t] = mfma16x16x32<T>(kb, gr[j], dQs[t]);
+      }
+    }
+  }
+  __syncthreads();  // U and q are done with
+  tile_store<NSS, D / 8, PD>(SS, rss, tid);
+  u32x4 rds[NSS];
+  tile_load(rds, (const T*)a.ds_end + n * D * D, tid);
+  // the token's raw k and q (the lane's d): their rounded normalised rows for the row sums, the l2 norm's backward
+  u32x2 kraw[DT], qraw[DT];
 #pragma unroll
   for (int t = 0; t < DT; ++t) {
-    P1[t] = P2[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const u32x4 sb = *(const u32x4*)(SS + (16 * t + c16) * PD + 32 * s + 8 * g);
-      P1[t] = mfma16x16x32<T>(dyA[s], sb, P1[t]);
-      P2[t] = mfma16x16x32<T>(doA[s], sb, P2[t]);
+    kraw[t] = qraw[t] = u32x2{0u, 0u};
+    if (ra < rows) {
+      kraw[t] = *(const u32x2*)((const T*)a.k + kbase + ra * krs + 16 * t + 4 * g);
+      qraw[t] = *(const u32x2*)((const T*)a.q + base + ra * rs + 16 * t + 4 * g);
     }
   }
+  const float Ga = Fs[ra], Wf = Fs[C + ra], Bt = Bf[ra], iq = Fs[5 * C + ra], ik = Fs[6 * C + ra];
+  auto raw = [&](const u32x2& x, int i) { return elem16<T>(u32x4{x[0], x[1], 0u, 0u}, i); };
+  auto unit = [&](float f, const u32x2& x, int i) {  // as rounded into the row tiles
+    return elem16<T>(u32x4{pack2<T>(f * raw(x, i & ~1), f * raw(x, i | 1)), 0u, 0u, 0u}, i & 1);
+  };
+  __syncthreads();
+
+  // ---- dY S0^T and dO S0^T, transposed
+  float k1 = 0.f, q2 = 0.f, k3 = 0.f, xk = 0.f, xq = 0.f;
+#pragma unroll
+  for (int t = 0; t < DT; ++t) {
+    f32x4 P1 = {0.f, 0.f, 0.f, 0.f}, P2 = P1;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const u32x4 sb = frag(SS, PD, 16 * t, 32 * s);
+      P1 = mfma16x16x32<T>(sb, dyA[s], P1);
+      P2 = mfma16x16x32<T>(sb, doA[s], P2);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      k1 = fmaf(unit(ik, kraw[t], i), P1[i], k1);
+      q2 = fmaf(unit(iq, qraw[t], i), P2[i], q2);
+      dKn[t][i] -= Ga * Bt * P1[i];
+      dQs[t][i] = fmaf(Ga, P2[i], dQs[t][i]);
+      xq = fmaf(raw(qraw[t], i), dQs[t][i], xq);
+    }
+  }
+  u32x4 uA[KS];  // (read again here: held from the start, they would not fit the registers)
+#pragma unroll
+  for (int s = 0; s < KS; ++s) uA[s] = *(const u32x4*)((const T*)a.u + (n * C + ra) * D + 32 * s + 8 * g);
   // <dS, S0> over the thread's chunks, then dS replaces S0
   {
     float part = 0.f;
@@ -890,87 +955,50 @@ __global__ void __launch_bounds__(256, 1) gdn_bwd16_local_kernel(Bwd16LocalArgs 
   __syncthreads();
   tile_store<NSS, D / 8, PD>(SS, rds, tid);
   __syncthreads();
-#pragma unroll
-  for (int t = 0; t < DT; ++t) {
-    P3[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-      P3[t] = mfma16x16x32<T>(uA[s], *(const u32x4*)(SS + (16 * t + c16) * PD + 32 * s + 8 * g), P3[t]);
-  }
 
-  // dK, dQ: A operands (GA + GA^T), GR^T, GR rows; B operands k^T, q^T rows (= columns d)
-  u32x4 g1A[2], grtA[2], grA[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const u32x4 m = *(const u32x4*)(M1 + ra * PC + 32 * j + 8 * g);
-    const u32x4 mt = *(const u32x4*)(M1t + ra * PC + 32 * j + 8 * g);
-    uint32_t w[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      w[e] = pack2<T>(elem16<T>(m, 2 * e) + elem16<T>(mt, 2 * e), elem16<T>(m, 2 * e + 1) + elem16<T>(mt, 2 * e + 1));
-    g1A[j] = u32x4{w[0], w[1], w[2], w[3]};
-    grtA[j] = *(const u32x4*)(GRt + ra * PC + 32 * j + 8 * g);
-    grA[j] = *(const u32x4*)(GRs + ra * PC + 32 * j + 8 * g);
-  }
-  float rk1[4] = {0.f, 0.f, 0.f, 0.f}, rq2[4] = {0.f, 0.f, 0.f, 0.f}, rk3[4] = {0.f, 0.f, 0.f, 0.f};
-  // gradients of the normalised rows (dKn, dQs), then the l2 norm's backward:
-  // dx = i_x dX - i_x u_x2 x (x . dX) with x the raw row
-  f32x4 dKn[DT], dQs[DT], kraw[DT], qraw[DT];
-  float xk[4] = {0.f, 0.f, 0.f, 0.f}, xq[4] = {0.f, 0.f, 0.f, 0.f};
+  // ---- U dS^T, transposed
 #pragma unroll
   for (int t = 0; t < DT; ++t) {
-    f32x4 dk = {0.f, 0.f, 0.f, 0.f}, dq = dk;
+    f32x4 P3 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const u32x4 kb = *(const u32x4*)(Kt + (16 * t + c16) * PC + 32 * j + 8 * g);
-      const u32x4 qb = *(const u32x4*)(Qt + (16 * t + c16) * PC + 32 * j + 8 * g);
-      dk = mfma16x16x32<T>(g1A[j], kb, dk);
-      dk = mfma16x16x32<T>(grtA[j], qb, dk);
-      dq = mfma16x16x32<T>(grA[j], kb, dq);
-    }
-    const int d = 16 * t + c16;
+    for (int s = 0; s < KS; ++s) P3 = mfma16x16x32<T>(frag(SS, PD, 16 * t, 32 * s), uA[s], P3);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int p = 16 * wave + 4 * g + i;
-      const float kv = to_f32(Kt[d * PC + p]), qv = to_f32(Qt[d * PC + p]);
-      rk1[i] = fmaf(kv, P1[t][i], rk1[i]);
-      rq2[i] = fmaf(qv, P2[t][i], rq2[i]);
-      rk3[i] = fmaf(kv, P3[t][i], rk3[i]);
-      dKn[t][i] = dk[i] - Ga[p] * Bf[p] * P1[t][i] + Wf[p] * P3[t][i];
-      dQs[t][i] = dq[i] + Ga[p] * P2[t][i];
-      kraw[t][i] = to_f32(kraw16[t][i]);
-      qraw[t][i] = to_f32(qraw16[t][i]);
-      xk[i] = fmaf(kraw[t][i], dKn[t][i], xk[i]);
-      xq[i] = fmaf(qraw[t][i], dQs[t][i], xq[i]);
+      k3 = fmaf(unit(ik, kraw[t], i), P3[i], k3);
+      dKn[t][i] = fmaf(Wf, P3[i], dKn[t][i]);
+      xk = fmaf(raw(kraw[t], i), dKn[t][i], xk);
     }
   }
+  // sums over d: the lane's, then the four lanes of the token
+  auto tok_sum = [&](float x) {
+    x += __shfl_xor(x, 16, 64);
+    return x + __shfl_xor(x, 32, 64);
+  };
+  k1 = tok_sum(k1);
+  q2 = tok_sum(q2);
+  k3 = tok_sum(k3);
+  // the l2 norm's backward: dx = i_x dX - i_x u_x2 x (x . dX) with x the raw row
+  const float pq = iq * Fs[7 * C + ra] * tok_sum(xq), pk = ik * Fs[8 * C + ra] * tok_sum(xk);
+  if (ra < rows) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int p = 16 * wave + 4 * g + i;
-    const float iq = Fs[5 * C + p], ik = Fs[6 * C + p];
-    const float pq = iq * Fs[7 * C + p] * row16_sum(xq[i]), pk = ik * Fs[8 * C + p] * row16_sum(xk[i]);
-    if (p < rows) {
+    for (int t = 0; t < DT; ++t) {
+      float x[4], y[4];
 #pragma unroll
-      for (int t = 0; t < DT; ++t) {
-        const int64_t o = base + p * rs + 16 * t + c16;
-        ((T*)a.dk)[o] = from_f32<T>(ik * dKn[t][i] - pk * kraw[t][i]);
-        ((T*)a.dq)[o] = from_f32<T>(iq * dQs[t][i] - pq * qraw[t][i]);
+      for (int i = 0; i < 4; ++i) {
+        x[i] = ik * dKn[t][i] - pk * raw(kraw[t], i);
+        y[i] = iq * dQs[t][i] - pq * raw(qraw[t], i);
       }
+      const int64_t o = base + ra * rs + 16 * t + 4 * g;
+      *(u32x2*)((T*)a.dk + o) = u32x2{pack2<T>(x[0], x[1]), pack2<T>(x[2], x[3])};
+      *(u32x2*)((T*)a.dq + o) = u32x2{pack2<T>(y[0], y[1]), pack2<T>(y[2], y[3])};
     }
   }
-  // gradients of beta and of the log decays, per row
-  float wsum = 0.f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int p = 16 * wave + 4 * g + i;
-    const float k1 = row16_sum(rk1[i]), q2 = row16_sum(rq2[i]), k3 = row16_sum(rk3[i]);
-    if (c16 == 0) {
-      if (p < rows) a.db[(tok0 + p) * a.H + h] = dyv[p] - Ga[p] * k1 + dbl[i];
-      dlgs[p] = lgl[i] + Ga[p] * (q2 - Bf[p] * k1) - Wf[p] * k3;
-      wsum = fmaf(Wf[p], k3, wsum);
-    }
+  // gradients of beta and of the log decays
+  if (g == 0) {
+    if (ra < rows) a.db[(tok0 + ra) * a.H + h] = dyv[ra] - Ga * k1 + dbv[ra];
+    dlgs[ra] += Ga * (q2 - Bt * k1) - Wf * k3;
   }
-  wsum = wave_sum(wsum);
+  const float wsum = wave_sum(g == 0 ? Wf * k3 : 0.f);
   if (lane == 0) red[1][wave] = wsum;
   __syncthreads();
   if (wave == 0) {
@@ -1027,24 +1055,22 @@ bool aligned16(std::initializer_list<const void*> ps) {
 #define ATMA_BWD16_DISPATCH(KERNEL, grid, stream, args) ATMA_BWD16_DISPATCH_NT(KERNEL, grid, 256, stream, args)
 
 extern "C" int atma_gated_delta_bwd16_prep(const void* q, const void* k, const void* v, const void* d_out,
-                                           const float* g, const float* beta, void* kr, void* kt, void* qr,
-                                           void* qt, void* tm, void* tt, void* rt, void* vt, void* ot, void* got,
-                                           float* f, int64_t B, int64_t T, int64_t H, int64_t d, float scale,
-                                           int l2norm, int dtype, void* stream) {
+                                           const float* g, const float* beta, void* kr, void* qr, void* tm, void* tt,
+                                           void* rt, void* vt, void* ot, float* f, int64_t B, int64_t T, int64_t H,
+                                           int64_t Hkv, int64_t d, float scale, int l2norm, int dtype, void* stream) {
   using namespace atma;
   if (!bwd16_dims_ok(d, dtype, "gated_delta_bwd16_prep")) return ATMA_ERR_UNSUPPORTED;
-  if (B < 0 || T < 0 || H <= 0) return set_error(ATMA_ERR_INVALID, "gated_delta_bwd16_prep: bad sizes");
+  if (B < 0 || T < 0 || H <= 0 || Hkv <= 0 || H % Hkv) return set_error(ATMA_ERR_INVALID, "gated_delta_bwd16_prep: bad sizes");
   const int64_t NC = (T + 63) / 64;
   if (B == 0 || NC == 0) return ATMA_OK;
-  if (!q || !k || !v || !d_out || !g || !beta || !kr || !kt || !qr || !qt || !tm || !tt || !rt || !vt || !ot ||
-      !got || !f)
+  if (!q || !k || !v || !d_out || !g || !beta || !kr || !qr || !tm || !tt || !rt || !vt || !ot || !f)
     return set_error(ATMA_ERR_INVALID, "gated_delta_bwd16_prep: null pointer");
-  if (!aligned16({q, k, v, d_out, kr, kt, qr, qt, tm, tt, rt, vt, ot, got}))
+  if (!aligned16({q, k, v, d_out, kr, qr, tm, tt, rt, vt, ot}))
     return set_error(ATMA_ERR_INVALID, "gated_delta_bwd16_prep: operands must be 16-byte aligned");
   if (B * H * NC > 0x7fffffff || B * T > 0x7fffffff)
     return set_error(ATMA_ERR_INVALID, "gated_delta_bwd16_prep: sizes too large");
-  Bwd16PrepArgs a{q, k, v, d_out, g, beta, kr, kt, qr, qt, tm, tt, rt, vt, ot, got, f, scale, l2norm ? 1 : 0,
-                  (int)B, (int)T, (int)H, (int)NC};
+  Bwd16PrepArgs a{q, d_out, k, v, g, beta, kr, qr, tm, tt, rt, vt, ot, f, scale, l2norm ? 1 : 0,
+                  (int)B, (int)T, (int)H, (int)NC, (int)(H / Hkv)};
   const dim3 grid((unsigned)(B * H * NC));
   ATMA_BWD16_DISPATCH(gdn_bwd16_prep_kernel, grid, (hipStream_t)stream, a);
   return check_launch("gated_delta_bwd16_prep");
@@ -1073,25 +1099,24 @@ extern "C" int atma_gated_delta_bwd16_chain(const void* kr, const void* qr, cons
   return check_launch("gated_delta_bwd16_chain");
 }
 
-extern "C" int atma_gated_delta_bwd16_local(const void* kr, const void* kt, const void* qr, const void* qt,
-                                            const void* q, const void* k, const void* v, const void* d_out,
+extern "C" int atma_gated_delta_bwd16_local(const void* q, const void* k, const void* v, const void* d_out,
                                             const float* f, const void* s_entry, const void* ds_end, const void* u,
                                             const float* dy, void* dq, void* dk, void* dv, float* dg, float* dbeta,
-                                            int64_t B, int64_t T, int64_t H, int64_t d, int dtype, void* stream) {
+                                            int64_t B, int64_t T, int64_t H, int64_t Hkv, int64_t d, int dtype,
+                                            void* stream) {
   using namespace atma;
   if (!bwd16_dims_ok(d, dtype, "gated_delta_bwd16_local")) return ATMA_ERR_UNSUPPORTED;
-  if (B < 0 || T < 0 || H <= 0) return set_error(ATMA_ERR_INVALID, "gated_delta_bwd16_local: bad sizes");
+  if (B < 0 || T < 0 || H <= 0 || Hkv <= 0 || H % Hkv) return set_error(ATMA_ERR_INVALID, "gated_delta_bwd16_local: bad sizes");
   const int64_t NC = (T + 63) / 64;
   if (B == 0 || NC == 0) return ATMA_OK;
-  if (!kr || !kt || !qr || !qt || !q || !k || !v || !d_out || !f || !s_entry || !ds_end || !u || !dy || !dq ||
-      !dk || !dv || !dg || !dbeta)
+  if (!q || !k || !v || !d_out || !f || !s_entry || !ds_end || !u || !dy || !dq || !dk || !dv || !dg || !dbeta)
     return set_error(ATMA_ERR_INVALID, "gated_delta_bwd16_local: null pointer");
-  if (!aligned16({kr, kt, qr, qt, v, d_out, s_entry, ds_end, u, dy, dv}))
+  if (!aligned16({q, k, v, d_out, s_entry, ds_end, u, dy, dq, dk, dv}))
     return set_error(ATMA_ERR_INVALID, "gated_delta_bwd16_local: operands must be 16-byte aligned");
   if (B * H * NC > 0x7fffffff || B * T > 0x7fffffff)
     return set_error(ATMA_ERR_INVALID, "gated_delta_bwd16_local: sizes too large");
-  Bwd16LocalArgs a{kr, kt, qr, qt, v, d_out, q, k, f, s_entry, ds_end, u, dy, dq, dk, dv, dg, dbeta,
-                   (int)B, (int)T, (int)H, (int)NC};
+  Bwd16LocalArgs a{q, d_out, k, v, f, s_entry, ds_end, u, dy, dq, dk, dv, dg, dbeta,
+                   (int)B, (int)T, (int)H, (int)NC, (int)(H / Hkv)};
   const dim3 grid((unsigned)(B * H * NC));
   ATMA_BWD16_DISPATCH(gdn_bwd16_local_kernel, grid, (hipStream_t)stream, a);
   return check_launch("gated_delta_bwd16_local");

@@ -65,6 +65,7 @@ SIGNATURES = {
     "atma_gated_delta_bwd": (_i32, [_p] * 14 + [_i64] * 5 + [_p, _sz, _p]),
     "atma_gated_delta_bwd16_prep": (_i32, [_p] * 14 + [_i64] * 5 + [_f32, _i32, _i32, _p]),
     "atma_gated_delta_bwd16_chain": (_i32, [_p] * 15 + [_i64] * 3 + [_i32, _p]),
+    "atma_gated_delta_bwd16_group_sum": (_i32, [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i32, _p]),
     "atma_gated_delta_bwd16_local": (_i32, [_p] * 14 + [_i64] * 5 + [_i32, _p]),
     "atma_squared_relu_gate": (_i32, [_p, _i64, _i64, _p, _i64, _i64, _p, _i64, _i64, _i32, _p]),
     "atma_softcap_logits": (_i32, [_p, _p, _i64, _i32, _p]),

@@ -441,8 +441,9 @@ def _(q, k, v, g, beta, initial_state, d_out, d_final_state):
 
 def _bwd16_check(q, k, v, d_out, g, beta):
     _need_cuda(q, k, v, d_out, g, beta)
-    if q.dim() != 4 or k.shape != q.shape or v.shape != q.shape or d_out.shape != q.shape:
-        raise ValueError("gated_delta_bwd16: q, k, v, d_out must all be (B, T, H, d)")
+    if q.dim() != 4 or k.dim() != 4 or v.shape != k.shape or d_out.shape != q.shape or k.shape[:2] != q.shape[:2] \
+            or k.shape[3] != q.shape[3] or k.shape[2] < 1 or q.shape[2] % k.shape[2]:
+        raise ValueError("gated_delta_bwd16: q, d_out (B, T, H, d) and k, v (B, T, Hkv, d) with H % Hkv == 0")
     B, T, H, d = q.shape
     if tuple(g.shape) != (B, T, H) or tuple(beta.shape) != (B, T, H):
         raise ValueError("gated_delta_bwd16: g and beta must be (B, T, H)")
@@ -501,6 +502,13 @@ def _bwd16_local(q, k, v, d_out, f, s_entry, ds_end, u, dy):
                                           B, T, H, k.shape[2], d, _lib.dtype_code(q.dtype),
                                           _lib.stream_handle(q.device))
     _lib.check(rc, "gated_delta_bwd16_local")
+    if k.shape[2] != H:   # each query head's dk and dv, summed over its group
+        out = [torch.empty(k.shape, **t16) for _ in range(2)]
+        rc = lib.atma_gated_delta_bwd16_group_sum(dk.data_ptr(), dv.data_ptr(), out[0].data_ptr(), out[1].data_ptr(),
+                                                  B * T, H, k.shape[2], d, _lib.dtype_code(q.dtype),
+                                                  _lib.stream_handle(q.device))
+        _lib.check(rc, "gated_delta_bwd16_group_sum")
+        dk, dv = out
     return [dq, dk, dv, dg, db]
 
 
@@ -518,7 +526,7 @@ def gated_delta_bwd16_op(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tenso
                          initial_state: Optional[Tensor], d_out: Tensor, d_final_state: Optional[Tensor],
                          scale: float, l2norm: bool) -> List[Tensor]:
     """Chunked (WY) backward for 16-bit training of ``chunk_gated_delta_rule`` with raw
-    q, k, v, d_out (B, T, H, d) of one 16-bit dtype (l2norm: q and k l2-normalised in the
+    q, d_out (B, T, H, d), k, v (B, T, Hkv, d) of one 16-bit dtype (l2norm: q and k l2-normalised in the
     recurrence, q then times scale); g (log decay), beta (B, T, H) fp32; initial_state,
     d_final_state (B, H, d, d) fp32 or None.  Returns dq, dk, dv (16-bit), dg, dbeta,
     d_initial_state (fp32).  Three launches: prep, chain, local."""

@@ -375,8 +375,11 @@ int atma_gated_delta_bwd(const float* q, const float* k, const float* v, const f
  *
  * local: the prep's f, the chain's s_entry, ds_end, u, dy, and q, k, v, d_out as given to
  * the prep.  Writes dq, dk, dv (B, T, H, d) 16-bit (dq, dk through the l2 norm and scale to
- * the raw rows; dk, dv per query head, for the caller to sum over a group), dg, dbeta (B, T, H) fp32 (dg the gradient of the
+ * the raw rows; dk, dv per query head), dg, dbeta (B, T, H) fp32 (dg the gradient of the
  * per-token log decay).
+ *
+ * group_sum: dk_out, dv_out (rows, Hkv, d) = dk, dv (rows, H, d) summed over each group of
+ * H / Hkv heads, 16-bit with fp32 accumulation (rows: the B * T tokens).
  */
 int atma_gated_delta_bwd16_prep(const void* q, const void* k, const void* v, const void* d_out,
                                 const float* g, const float* beta, void* kr, void* qr, void* tm, void* tt,
@@ -391,6 +394,8 @@ int atma_gated_delta_bwd16_local(const void* q, const void* k, const void* v, co
                                  const float* dy, void* dq, void* dk, void* dv, float* dg, float* dbeta,
                                  int64_t B, int64_t T, int64_t H, int64_t Hkv, int64_t d, int dtype,
                                  void* stream);
+int atma_gated_delta_bwd16_group_sum(const void* dk, const void* dv, void* dk_out, void* dv_out, int64_t rows,
+                                     int64_t H, int64_t Hkv, int64_t d, int dtype, void* stream);
 
 /*
  * Fused MLP activation out = gate * relu(x)^2.  Replaces squared_relu_gate

@@ -113,6 +113,13 @@ SIGNATURES = {
     "atma_gated_delta_prefill": (_i32, [
         _p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _p, _p, _p, _i64, _p, _i64, _i64, _p,
         _i64, _i64, _i64, _i32, _f32, _i32, _i32, _f32, _f32, _p, _sz, _p, _i32, _p]),
+    "atma_cast_blocks": (_i32, [_i32] + [_p] * 11),
+    "atma_gather_colsum_partials": (_sz, [_i64]),
+    "atma_gather_colsum": (_i32, [_i32, _p, _p, _p, _i64, _p, _p, _i64, _i32, _p]),
+    "atma_squared_relu_gate_bwd": (_i32, [_p, _i64, _p, _i64, _p, _i64, _i64, _i32, _p]),
+    "atma_head_norm_bwd": (_i32, [_p] * 6 + [_i64, _i64, _f32, _i32, _p]),
+    "atma_global_gate_bwd": (_i32, [_p] + [_i64] * 4 + [_p, _i64, _i64, _p, _p, _i64] + [_p] * 5 +
+                             [_i64, _i64, _i64, _f32, _i32, _p]),
     "atma_wait_start_flag": (_i32, [_p, _i32, _i64, _p]),
 }
 

@@ -40,26 +40,26 @@ def head_rms_norm(x, eps):
 
 
 @torch.no_grad()
-def global_gate(c, gate, r, mem_gate, mem_eps):
+def global_gate(c, gate, r, mem_gate, mem_eps, out=None):
     """The global layer's two gated projection inputs, rows m = b T + t:
     ``xa = (c * sigmoid(gate)).reshape(rows, H d)`` and
     ``xm = (rms_norm(r).to(dtype) * sigmoid(mem_gate.view(rows, H, d))).reshape(rows, H d)``.
     c: (B, T, H, d) view (Polar's head-major output transposed, or (1, tokens, H, d));
     gate: (rows, H, d) view; r: (rows, H, d) fp32 or c's dtype (heads contiguous) or None; mem_gate:
-    (rows, H d).  Returns (xa, xm or None)."""
+    (rows, H d).  ``out`` (rows, 2 H d): both side by side there.  Returns (xa, xm or None)."""
     _gpu16(c, gate, mem_gate)
     B, T, H, d = c.shape
     rows = B * T
     if gate.shape != (rows, H, d) or gate.stride(2) != 1 or c.stride(3) != 1 or gate.dtype != c.dtype:
         raise ValueError("global_gate: gate (rows, H, d) and c (B, T, H, d) with unit inner strides")
-    xa = torch.empty((rows, H * d), device=c.device, dtype=c.dtype)
+    xa = torch.empty((rows, H * d), device=c.device, dtype=c.dtype) if out is None else out[:, :H * d]
     xm = None
     if r is not None:
         if r.dtype not in (torch.float32, c.dtype) or r.shape != (rows, H, d) or r.stride(2) != 1 or r.stride(1) != d:
             raise ValueError("global_gate: r must be fp32 or c's dtype, (rows, H, d) with contiguous heads")
         if mem_gate.shape != (rows, H * d) or mem_gate.stride(1) != 1 or mem_gate.dtype != c.dtype:
             raise ValueError("global_gate: mem_gate must be (rows, H d)")
-        xm = torch.empty_like(xa)
+        xm = torch.empty_like(xa) if out is None else out[:, H * d:]
     rc = _lib.load().atma_global_gate(
         c.data_ptr(), c.stride(0), c.stride(1), c.stride(2), T, gate.data_ptr(), gate.stride(0), gate.stride(1),
         _lib.ptr(r), 0 if r is None else r.stride(0), _lib.dtype_code(torch.float32 if r is None else r.dtype),

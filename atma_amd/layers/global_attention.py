@@ -49,6 +49,8 @@ from ..kernel.decode_fusions import (PartialSums, chunk_width, global_decode_gat
 from ..kernel.gated_delta import gated_delta_prefill, gated_delta_prefill_supported
 from ..kernel.inference_ops import (linear_tokens, linear_tokens_supported, packed_causal_conv1d,
                                      squared_relu_gate)
+from ..kernel.train_glue import (gate_train, head_norm_train, linear_train, out_train, plain_module, project_train,
+                                 squared_relu_gate_train, train_glue_served)
 from ..kernel.layer_fusions import (global_gate, head_rms_norm, linear_gated, linear_gated_supported,
                                     memory_gate_logits, memory_gate_logits_supported, paged_kv_concat)
 from ..kernel.polar import global_decode_step_supported_shape
@@ -80,10 +82,13 @@ class Linear(nn.Linear):
     """``F.linear`` with weights cast to the input dtype (``model/reference.py:22-28``).
 
     Inference calls on a few token rows (a decode step: one row per sequence) at the shapes
-    ``linear_tokens`` serves run that HIP kernel, which streams the weights once; every
-    other call (training, prefill, other shapes) is ``F.linear``."""
+    ``linear_tokens`` serves run that HIP kernel, which streams the weights once; training on
+    16-bit GPU rows is ``linear_train`` (the same GEMMs, the conversions and the bias gradient one
+    launch each); every other call is ``F.linear``."""
 
     def forward(self, x):
+        if train_glue_served(x, self.weight, self.bias) and x.dim() >= 2:
+            return linear_train(x, self.weight, self.bias)
         w = self.weight.type_as(x)
         b = None if self.bias is None else self.bias.type_as(x)
         if x.is_cuda and not torch.is_grad_enabled() and x.dim() >= 1 and x.stride(-1) == 1:
@@ -414,8 +419,43 @@ class PolarAttention(nn.Module):
     def forward(self, x):
         """Causal full-sequence mixer (``model/reference.py:127-195``): x (B, T, dim)."""
         B, T, _ = x.shape
+        if self._train_fused(x):
+            return self._forward_train(x)
         q, gate, k, v = (t.unflatten(0, (B, T)) for t in self._project_canon(x, B, T))
         return self._attend_prefill(x, q, gate, k, v)
+
+    def _train_fused(self, x):
+        """Whether a training forward takes ``_forward_train``: shapes its launches serve, and submodules that are
+        what this file makes of them, without hooks (their calls are not made there)."""
+        m = self.mem
+        if m is None or x.dim() != 3 or not torch.is_grad_enabled() or not canon_supported(x, self.head_dim,
+                                                                                           self.kernel_size):
+            return False
+        lin = (self.q, self.k, self.v, m.gate, m.w_gamma, m.w_beta, self.proj, m.proj, self.mu_proj)
+        return (plain_module(m, TitansMemory) and all(plain_module(l, Linear) for l in lin)
+                and all(plain_module(c, nn.Conv1d) for c in (self.canon_q, self.canon_k, self.canon_v))
+                and train_glue_served(x, *[l.weight for l in lin], *[l.bias for l in lin])
+                and all(l.bias is not None for l in lin))
+
+    def _forward_train(self, x):
+        """The training forward with its projections as one GEMM, the two output projections as another, and the
+        norms, convs and gates one launch each way (``kernel/train_glue.py``, ``kernel/canon.py``)."""
+        B, T, dim = x.shape
+        H, Hkv, dk, rows, m = self.num_heads, self.num_kv_heads, self.head_dim, B * T, self.mem
+        q, gate, k, v, mg, zg, zb = project_train(x.reshape(rows, dim),
+                                                  (self.q, self.k, self.v, m.gate, m.w_gamma, m.w_beta), dk)
+        q, k = head_norm_train(q, k.unflatten(1, (Hkv, dk)), F32_EPS)
+        q, k, v = canon_conv(q.view(B, T, H * dk), k.view(B, T, Hkv * dk), v.reshape(B, T, Hkv * dk),
+                             *[c.weight for c in (self.canon_q, self.canon_k, self.canon_v)])
+        q, k, v = q.view(B, T, H, dk), k.view(B, T, Hkv, dk), v.view(B, T, Hkv, dk)
+        n_keys = torch.arange(1, T + 1, device=x.device, dtype=torch.float32)
+        c, mag = polar_attention(*(t.transpose(1, 2) for t in (q, k, v)), n_keys, is_causal=True, window=self.window,
+                                 **self.polar_params())
+        r, _ = chunk_gated_delta_rule(q, k, v, zg.float().view(B, T, H), zb.float().view(B, T, H), scale=1.0,
+                                      use_qk_l2norm_in_kernel=True, gate_bias=(m.gamma_bias, m.beta_bias))
+        xs = gate_train(c.transpose(1, 2), gate, r.reshape(rows, H, dk), mg, F32_EPS)
+        mu = linear_train(mag.transpose(1, 2).to(x.dtype).reshape(rows, H), self.mu_proj.weight, self.mu_proj.bias)
+        return (out_train(xs, (self.proj, m.proj)) + mu).view(B, T, -1)
 
     def _memory(self, x, q, k, v, fused, cache, slots, signal):
         """The memory branch of a prefill from zero states (``cache`` None) or from and to the table's rows: its readout
@@ -674,6 +714,9 @@ class MLP(nn.Module):
                 # that never writes the 8 dim-wide projection (linear_gated)
                 h = linear_gated(x.view(rows, K), self.fc.weight, self.fc.bias)
                 return self.proj(h.view(*x.shape[:-1], -1))
+        if train_glue_served(x) and plain_module(self.fc, Linear):
+            y = self.fc(x)
+            return self.proj(squared_relu_gate_train(y.view(-1, y.shape[-1])).view(*y.shape[:-1], -1))
         a, gate = torch.chunk(self.fc(x), 2, dim=-1)
         if x.is_cuda and not torch.is_grad_enabled():
             # InferenceMLP (inference/models/atma.py:87-96): the fused HIP activation,

@@ -756,6 +756,41 @@ int atma_gated_delta_prefill(const void* q, int64_t q_sb, int64_t q_st, int64_t 
                              float g_bias, float b_bias, void* workspace, size_t workspace_bytes, int32_t* start_flag,
                              int32_t start_epoch, void* stream);
 
+/*
+ * Training: the launches around the global block's GEMMs (16-bit rows; model/reference.py:22-28, 127-229,
+ * model/blocks.py:472-490, model/layers.py:19-31).  All rows 16-byte aligned, widths in multiples of 8.
+ *
+ * cast_blocks: up to 16 blocks (rows[i], cols[i]) from src[i] (row stride src_ld[i] elements, plus add[i] where non-NULL)
+ * to dst[i] (dst_ld[i]), converted between fp32 / bf16 / fp16; sum[i] > 1 (rows[i] = 1, fp32): the sum of that many source
+ * rows.  add and sum may be NULL.
+ *
+ * gather_colsum: n <= 8 parts (rows, width[i]), row stride ld[i], side by side in dst (rows, sum of widths; NULL: not
+ * written), a NULL part as zeros; inter > 0: parts 0 and 1 interleaved by heads of that width.  part (partials(rows),
+ * sum of widths) fp32: column sums over consecutive 128-row chunks.
+ *
+ * squared_relu_gate_bwd: dy = d(gate relu(a)^2) with y = [a | gate] (rows, 2 width), dh (rows, width), dy contiguous.
+ *
+ * head_norm_bwd: the per-head RMS norm's backward for two tensors (rows, heads[p], d): x strided, dn and dx contiguous.
+ *
+ * global_gate_bwd: dc, dgate, dr, dmgate (rows, H, d) contiguous from dx (rows, 2 H d), the gradient of global_gate's
+ * xa and xm side by side; c, gate, mgate as there, r (rows, H, d) contiguous in the rows' type.
+ */
+int atma_cast_blocks(int n, const void* const* src, const void* const* add, void* const* dst, const int64_t* rows,
+                     const int64_t* cols, const int64_t* src_ld, const int64_t* dst_ld, const int* src_dtype,
+                     const int* dst_dtype, const int64_t* sum, void* stream);
+size_t atma_gather_colsum_partials(int64_t rows);
+int atma_gather_colsum(int n, const void* const* src, const int64_t* ld, const int64_t* width, int64_t inter, void* dst,
+                       float* part, int64_t rows, int dtype, void* stream);
+int atma_squared_relu_gate_bwd(const void* y, int64_t ldy, const void* dh, int64_t ldh, void* dy, int64_t rows,
+                               int64_t width, int dtype, void* stream);
+int atma_head_norm_bwd(const void* const* x, const int64_t* ldr, const int64_t* ldh, const int64_t* heads,
+                       const void* const* dn, void* const* dx, int64_t rows, int64_t d, float eps, int dtype,
+                       void* stream);
+int atma_global_gate_bwd(const void* c, int64_t c_sb, int64_t c_st, int64_t c_sh, int64_t T, const void* gate,
+                         int64_t g_sr, int64_t g_sh, const void* r, const void* mgate, int64_t mg_sr, const void* dx,
+                         void* dc, void* dgate, void* dr, void* dmgate, int64_t rows, int64_t H, int64_t d, float eps,
+                         int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

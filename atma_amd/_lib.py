@@ -178,7 +178,9 @@ def ptr(t):
 
 
 def stream_handle(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream of ``device``, without building a Stream object (5 us of host time a launch)."""
+    index = device.index if isinstance(device, torch.device) else torch.device(device).index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def dtype_code(dtype) -> int:

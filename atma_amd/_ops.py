@@ -8,14 +8,58 @@ implementation: a CPU tensor raises, and a missing library raises
 ``HipLibraryMissing``.
 """
 
-from typing import List, Optional
-
 import ctypes
+import inspect
+from types import SimpleNamespace
+from typing import List, Optional
 
 import torch
 from torch import Tensor
 
 from . import _lib
+
+
+# run.name(*args): the op ``atma_hip::name``, called directly where nothing needs the dispatcher, which costs about 15 us
+# of host time a call, a third of a small decode step (two sequences: 47 us dispatched)
+run = SimpleNamespace()
+_PLAIN = (Tensor, torch.nn.Parameter)
+
+
+def _undispatched(args):
+    """Whether a call on these arguments has nothing to dispatch to: no tracing, autograd, transform, mode or subclass."""
+    if torch.compiler.is_compiling() or torch.is_grad_enabled() or torch._C._len_torch_dispatch_stack() \
+            or torch._C._len_torch_function_stack() or torch._C._are_functorch_transforms_active() \
+            or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    for a in args:
+        for t in a if type(a) is list else (a,):
+            if isinstance(t, Tensor) and type(t) not in _PLAIN:
+                return False
+    return True
+
+
+def _op(name, mutates_args=()):
+    """Register the op ``atma_hip::name`` and its direct call ``run.name``, which advances the version counters of the
+    mutated arguments as the dispatcher does."""
+    def register(fn):
+        names = list(inspect.signature(fn).parameters)
+        mutated = tuple(names.index(m) for m in mutates_args)
+        registered = torch.library.custom_op(f"atma_hip::{name}", fn, mutates_args=mutates_args)
+        op = getattr(torch.ops.atma_hip, name)
+
+        def call(*args):
+            if not _undispatched(args):
+                return op(*args)
+            out = fn(*args)
+            for i in mutated:
+                t = args[i] if i < len(args) else None
+                if t is not None and not t.is_inference():
+                    torch.autograd.graph.increment_version(t)
+            return out
+
+        setattr(run, name, call)
+        return registered
+    return register
 
 
 def _need_cuda(*ts):
@@ -41,7 +85,7 @@ def _polar_fwd_scratch(lib, q, Hkv, Tk, is_causal, window):
     return torch.empty(n, device=q.device, dtype=torch.uint8) if n else None, n
 
 
-@torch.library.custom_op("atma_hip::polar_attention_fwd", mutates_args=())
+@_op("polar_attention_fwd", mutates_args=())
 def polar_attention_fwd_op(q: Tensor, k: Tensor, v: Tensor, n_keys: Tensor, v_null: Tensor,
                            null_base: Tensor, null_slope_raw: Tensor, len_gain_raw: Tensor,
                            mag_beta_raw: Tensor, eps: float, is_causal: bool,
@@ -74,7 +118,7 @@ def _(q, k, v, n_keys, v_null, null_base, null_slope_raw, len_gain_raw, mag_beta
 
 
 # --------------------------------------------------------------------------- Polar training pair
-@torch.library.custom_op("atma_hip::polar_attention_fwd_train", mutates_args=())
+@_op("polar_attention_fwd_train", mutates_args=())
 def polar_attention_fwd_train_op(q: Tensor, k: Tensor, v: Tensor, n_keys: Tensor, v_null: Tensor,
                                  null_base: Tensor, null_slope_raw: Tensor, len_gain_raw: Tensor,
                                  mag_beta_raw: Tensor, eps: float, is_causal: bool, window: int,
@@ -112,7 +156,7 @@ def _(q, k, v, n_keys, v_null, null_base, null_slope_raw, len_gain_raw, mag_beta
             q.new_empty((B, Hq, Tq), **f), q.new_empty((B, Hq, Tq), **f), q.new_empty((B, Hq, Tq, d), **f)]
 
 
-@torch.library.custom_op("atma_hip::polar_attention_bwd_prep", mutates_args=())
+@_op("polar_attention_bwd_prep", mutates_args=())
 def polar_attention_bwd_prep_op(gc: Optional[Tensor], gm: Optional[Tensor], S: Tensor, M: Tensor,
                                 L: Tensor, Q2: Tensor, n_keys: Tensor, v_null: Tensor,
                                 null_base: Tensor, null_slope_raw: Tensor, len_gain_raw: Tensor,
@@ -150,7 +194,7 @@ def _(gc, gm, S, M, L, Q2, n_keys, v_null, null_base, null_slope_raw, len_gain_r
             S.new_empty((H, T)), S.new_empty((B * ((T + 15) // 16), H, d + 4))]
 
 
-@torch.library.custom_op("atma_hip::polar_attention_bwd", mutates_args=())
+@_op("polar_attention_bwd", mutates_args=())
 def polar_attention_bwd_op(q: Tensor, k: Tensor, v: Tensor, gs: Tensor, gL: Tensor, gQ2: Tensor,
                            M: Tensor, temp: Tensor, n_keys: Tensor, is_causal: bool,
                            window: int) -> List[Tensor]:
@@ -194,7 +238,7 @@ def _group_sum(lib, part, n_groups, elems, G, dtype):
     return out.view(part.shape) if G == 1 else out
 
 
-@torch.library.custom_op("atma_hip::polar_bwd_param_grads", mutates_args=())
+@_op("polar_bwd_param_grads", mutates_args=())
 def polar_bwd_param_grads_op(part: Tensor, dt: Tensor, n_keys: Tensor, len_gain_raw: Tensor,
                              null_slope_raw: Tensor, mag_beta_raw: Tensor, window: int,
                              preserve_length: bool) -> List[Tensor]:
@@ -237,7 +281,7 @@ def _(q, k, v, gs, gL, gQ2, M, temp, n_keys, is_causal, window):
 
 
 # --------------------------------------------------------------------------- Polar packed fwd
-@torch.library.custom_op("atma_hip::polar_attention_packed_fwd", mutates_args=())
+@_op("polar_attention_packed_fwd", mutates_args=())
 def polar_attention_packed_fwd_op(q: Tensor, k: Tensor, v: Tensor, tile_seq_starts: Tensor,
                                   tile_q_starts: Tensor, tile_seq_lens: Tensor, v_null: Tensor,
                                   null_base: Tensor, null_slope_raw: Tensor, len_gain_raw: Tensor,
@@ -268,7 +312,7 @@ def _(q, k, v, tile_seq_starts, tile_q_starts, tile_seq_lens, v_null, null_base,
 
 
 # --------------------------------------------------------------------------- Polar decode
-@torch.library.custom_op("atma_hip::polar_attention_decode", mutates_args=())
+@_op("polar_attention_decode", mutates_args=())
 def polar_attention_decode_op(q: Tensor, k_cache: Tensor, v_cache: Tensor, block_tables: Tensor,
                               context_lens: Tensor, v_null: Tensor, null_base: Tensor,
                               null_slope_raw: Tensor, len_gain_raw: Tensor, mag_beta_raw: Tensor,
@@ -304,7 +348,7 @@ def _(q, k_cache, v_cache, block_tables, context_lens, v_null, null_base, null_s
 
 
 # --------------------------------------------------------------------------- gated delta step
-@torch.library.custom_op("atma_hip::gated_delta_decode_step", mutates_args=("state_table",))
+@_op("gated_delta_decode_step", mutates_args=("state_table",))
 def gated_delta_decode_step_op(q: Tensor, k: Tensor, v: Tensor, gamma: Tensor, beta: Tensor,
                                state_table: Tensor, slots: Tensor, eps: float) -> Tensor:
     _need_cuda(q, k, v, gamma, beta, state_table, slots)
@@ -331,8 +375,7 @@ def _(q, k, v, gamma, beta, state_table, slots, eps):
 
 
 # --------------------------------------------------------------------------- fused decode step
-@torch.library.custom_op("atma_hip::global_decode_step",
-                         mutates_args=("k_cache", "v_cache", "state_table"))
+@_op("global_decode_step", mutates_args=("k_cache", "v_cache", "state_table"))
 def global_decode_step_op(q: Tensor, k_new: Tensor, v_new: Tensor, k_cache: Tensor, v_cache: Tensor,
                           slot_mapping: Tensor, block_tables: Tensor, context_lens: Tensor,
                           v_null: Tensor, null_base: Tensor, null_slope_raw: Tensor,
@@ -377,7 +420,7 @@ def _(q, k_new, v_new, k_cache, v_cache, slot_mapping, block_tables, context_len
 
 
 # --------------------------------------------------------------------------- conv decode step
-@torch.library.custom_op("atma_hip::causal_conv1d_decode_step", mutates_args=("state_table",))
+@_op("causal_conv1d_decode_step", mutates_args=("state_table",))
 def causal_conv1d_decode_step_op(x: Tensor, weight: Tensor, slots: Tensor, state_table: Tensor,
                                  residual: bool) -> Tensor:
     _need_cuda(x, weight, slots, state_table)
@@ -403,7 +446,7 @@ def _(x, weight, slots, state_table, residual):
 
 
 # --------------------------------------------------------------------------- gated delta backward
-@torch.library.custom_op("atma_hip::gated_delta_bwd", mutates_args=())
+@_op("gated_delta_bwd", mutates_args=())
 def gated_delta_bwd_op(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor,
                        initial_state: Optional[Tensor], d_out: Tensor,
                        d_final_state: Optional[Tensor]) -> List[Tensor]:
@@ -521,7 +564,7 @@ def _bwd16_states(initial_state, d_final_state, B, H, d):
     return out
 
 
-@torch.library.custom_op("atma_hip::gated_delta_bwd16", mutates_args=())
+@_op("gated_delta_bwd16", mutates_args=())
 def gated_delta_bwd16_op(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor,
                          initial_state: Optional[Tensor], d_out: Tensor, d_final_state: Optional[Tensor],
                          scale: float, l2norm: bool) -> List[Tensor]:
@@ -572,7 +615,7 @@ def gated_delta_bwd16_stages(q, k, v, g, beta, initial_state, d_out, d_final_sta
 
 
 # --------------------------------------------------------------------------- inference fusions
-@torch.library.custom_op("atma_hip::squared_relu_gate", mutates_args=())
+@_op("squared_relu_gate", mutates_args=())
 def squared_relu_gate_op(x: Tensor, gate: Tensor) -> Tensor:
     _need_cuda(x, gate)
     lib = _lib.load()
@@ -590,7 +633,7 @@ def _(x, gate):
     return x.new_empty(x.shape)
 
 
-@torch.library.custom_op("atma_hip::softcap_logits", mutates_args=())
+@_op("softcap_logits", mutates_args=())
 def softcap_logits_op(logits: Tensor) -> Tensor:
     _need_cuda(logits)
     lib = _lib.load()
@@ -607,7 +650,7 @@ def _(logits):
     return torch.empty_like(logits)
 
 
-@torch.library.custom_op("atma_hip::linear_tokens", mutates_args=())
+@_op("linear_tokens", mutates_args=())
 def linear_tokens_op(x: Tensor, weight: Tensor, bias: Optional[Tensor]) -> Tensor:
     """y = x weight^T (+ bias) for a few token rows (x (M, K), M <= 32): the decode
     projection of the served model, weights streamed once (``atma_linear_tokens``)."""
@@ -631,7 +674,7 @@ def _(x, weight, bias):
     return x.new_empty((x.shape[0], weight.shape[0]))
 
 
-@torch.library.custom_op("atma_hip::softcap_argmax", mutates_args=())
+@_op("softcap_argmax", mutates_args=())
 def softcap_argmax_op(logits: Tensor) -> List[Tensor]:
     _need_cuda(logits)
     rows, V = logits.shape
@@ -649,7 +692,7 @@ def _(logits):
     return [logits.new_empty(logits.shape), logits.new_empty((logits.shape[0],), dtype=torch.int64)]
 
 
-@torch.library.custom_op("atma_hip::packed_causal_conv1d", mutates_args=("state_table",))
+@_op("packed_causal_conv1d", mutates_args=("state_table",))
 def packed_causal_conv1d_op(x: Tensor, weight: Tensor, state_table: Tensor, token_seq_starts: Tensor,
                             token_seq_ends: Tensor, token_seq_slots: Tensor) -> Tensor:
     _need_cuda(x, weight, state_table, token_seq_starts, token_seq_ends, token_seq_slots)
@@ -673,7 +716,7 @@ def _(x, weight, state_table, token_seq_starts, token_seq_ends, token_seq_slots)
 
 
 # --------------------------------------------------------------------------- memory gates
-@torch.library.custom_op("atma_hip::gated_delta_gates", mutates_args=())
+@_op("gated_delta_gates", mutates_args=())
 def gated_delta_gates_op(zg: Tensor, zb: Tensor, g_bias: float, b_bias: float,
                          decay_as_prob: bool) -> List[Tensor]:
     _need_cuda(zg, zb)
@@ -720,7 +763,7 @@ def _chunk_gated_delta(q, k, v, g, beta, initial_state, scale, use_qk_l2norm, wa
     return [o, final] if want_final else [o]
 
 
-@torch.library.custom_op("atma_hip::chunk_gated_delta_rule", mutates_args=("start_flag",))
+@_op("chunk_gated_delta_rule", mutates_args=("start_flag",))
 def chunk_gated_delta_rule_op(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor,
                               initial_state: Optional[Tensor], scale: float, use_qk_l2norm: bool,
                               want_final: bool, start_flag: Optional[Tensor], start_epoch: int,
@@ -731,7 +774,7 @@ def chunk_gated_delta_rule_op(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: 
                               start_flag, start_epoch, gate_logits, g_bias, b_bias)
 
 
-@torch.library.custom_op("atma_hip::gated_delta_fwd", mutates_args=())
+@_op("gated_delta_fwd", mutates_args=())
 def gated_delta_fwd_op(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor,
                        initial_state: Optional[Tensor], scale: float = 1.0,
                        l2norm: bool = False) -> List[Tensor]:
@@ -758,7 +801,7 @@ def _(q, k, v, g, beta, initial_state, scale, use_qk_l2norm, want_final, start_f
     return [o, q.new_empty((B, H, dk, dv), dtype=torch.float32)] if want_final else [o]
 
 
-@torch.library.custom_op("atma_hip::gated_delta_prefill", mutates_args=("state_table", "o", "start_flag"))
+@_op("gated_delta_prefill", mutates_args=("state_table", "o", "start_flag"))
 def gated_delta_prefill_op(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, state_table: Tensor,
                            slots: Tensor, o: Tensor, seq_lens: Optional[List[int]], g_bias: float, b_bias: float,
                            start_flag: Optional[Tensor], start_epoch: int) -> None:
@@ -785,7 +828,7 @@ def _(q, k, v, g, beta, state_table, slots, o, seq_lens, g_bias, b_bias, start_f
     return None
 
 
-@torch.library.custom_op("atma_hip::wait_start_flag", mutates_args=("flag",))
+@_op("wait_start_flag", mutates_args=("flag",))
 def wait_start_flag_op(flag: Tensor, epoch: int, timeout_us: int) -> None:
     _need_cuda(flag)
     if flag.dtype != torch.int32 or flag.numel() < 1:
@@ -801,7 +844,7 @@ def _(flag, epoch, timeout_us):
 
 
 # --------------------------------------------------------------------------- paged KV write
-@torch.library.custom_op("atma_hip::store_kvcache", mutates_args=("k_cache", "v_cache"))
+@_op("store_kvcache", mutates_args=("k_cache", "v_cache"))
 def store_kvcache_op(key: Tensor, value: Tensor, k_cache: Tensor, v_cache: Tensor,
                      slot_mapping: Tensor) -> None:
     _need_cuda(key, value, k_cache, v_cache, slot_mapping)
@@ -830,7 +873,7 @@ def _canon_check(xs, ws):
             raise ValueError("canon_conv: contiguous rows (B, T, C) in one dtype and conv weights (C, 1, K)")
 
 
-@torch.library.custom_op("atma_hip::canon_conv", mutates_args=())
+@_op("canon_conv", mutates_args=())
 def canon_conv_op(xs: List[Tensor], ws: List[Tensor]) -> List[Tensor]:
     from .kernel.canon import _L3, _I3, _P3, _taps
     _canon_check(xs, ws)
@@ -856,7 +899,7 @@ def _(xs, ws):
     return [torch.empty_like(x) for x in xs]
 
 
-@torch.library.custom_op("atma_hip::canon_conv_bwd", mutates_args=())
+@_op("canon_conv_bwd", mutates_args=())
 def canon_conv_bwd_op(gs: List[Tensor], xs: List[Tensor], ws: List[Tensor]) -> List[Tensor]:
     """dx of every stream, then every weight's gradient (its weight's dtype)."""
     from .kernel.canon import _L3, _P3, _taps

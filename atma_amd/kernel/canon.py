@@ -98,7 +98,7 @@ class _CanonConvFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, wq, wk, wv):
         ctx.save_for_backward(q, k, v, wq, wk, wv)
-        return tuple(torch.ops.atma_hip.canon_conv([q, k, v], [wq, wk, wv]))
+        return tuple(_ops.run.canon_conv([q, k, v], [wq, wk, wv]))
 
     @staticmethod
     def backward(ctx, *gy):
@@ -108,7 +108,7 @@ class _CanonConvFn(torch.autograd.Function):
             for x, w, g in zip(saved[:3], saved[3:], gy):
                 grads.append(torch.autograd.grad(_conv_torch(x, w), (x, w), g, create_graph=True))
             return tuple(g[0] for g in grads) + tuple(g[1] for g in grads)
-        return tuple(torch.ops.atma_hip.canon_conv_bwd([g.contiguous() for g in gy], list(saved[:3]), list(saved[3:])))
+        return tuple(_ops.run.canon_conv_bwd([g.contiguous() for g in gy], list(saved[:3]), list(saved[3:])))
 
 
 def canon_conv(q, k, v, wq, wk, wv):

@@ -28,4 +28,4 @@ def causal_conv1d_decode_step(x, weight, slots, state_table, residual=False):
         raise ValueError("state_table must have x's dtype")
     weight = weight.to(dtype=x.dtype)
     slots = slots.to(device=x.device, dtype=torch.int64).reshape(B).contiguous()
-    return torch.ops.atma_hip.causal_conv1d_decode_step(x, weight, slots, state_table, bool(residual))
+    return _ops.run.causal_conv1d_decode_step(x, weight, slots, state_table, bool(residual))

@@ -41,7 +41,7 @@ def gated_delta_decode_step(q, k, v, gamma, beta, state_table, slots, eps=1e-12,
     gamma = gamma.to(torch.float32).reshape(B, H).contiguous()
     beta = beta.to(torch.float32).reshape(B, H).contiguous()
     slots = slots.to(device=q.device, dtype=torch.int64).reshape(B).contiguous()
-    return torch.ops.atma_hip.gated_delta_decode_step(q, k, v, gamma, beta, state_table, slots,
+    return _ops.run.gated_delta_decode_step(q, k, v, gamma, beta, state_table, slots,
                                                       float(eps))
 
 
@@ -120,7 +120,7 @@ def _chunk_gated_delta_infer(q, k, v, g, beta, scale, initial_state, output_fina
     g = g.to(torch.float32).contiguous()
     beta = beta.to(torch.float32).contiguous()
     gb, bb = (0.0, 0.0) if gate_bias is None else (float(gate_bias[0]), float(gate_bias[1]))
-    outs = torch.ops.atma_hip.chunk_gated_delta_rule(q, k, v, g, beta, initial_state, float(scale),
+    outs = _ops.run.chunk_gated_delta_rule(q, k, v, g, beta, initial_state, float(scale),
                                                      bool(use_qk_l2norm_in_kernel),
                                                      bool(output_final_state),
                                                      None if start_signal is None else start_signal.flag,
@@ -137,7 +137,7 @@ class _GatedDeltaFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, qs, kn, v, g, beta, S0):
-        o, S = torch.ops.atma_hip.gated_delta_fwd(qs, kn, v, g, beta, S0)
+        o, S = _ops.run.gated_delta_fwd(qs, kn, v, g, beta, S0)
         ctx.save_for_backward(qs, kn, v, g, beta, S0)
         return o, S
 
@@ -146,7 +146,7 @@ class _GatedDeltaFn(torch.autograd.Function):
         qs, kn, v, g, beta, S0 = ctx.saved_tensors
         dO = torch.zeros_like(v) if dO is None else dO.to(torch.float32).contiguous()
         dS = None if dS is None else dS.to(torch.float32).contiguous()
-        dq, dk, dv, dg, db, ds0 = torch.ops.atma_hip.gated_delta_bwd(qs, kn, v, g, beta, S0, dO, dS)
+        dq, dk, dv, dg, db, ds0 = _ops.run.gated_delta_bwd(qs, kn, v, g, beta, S0, dO, dS)
         return dq, dk, dv, dg, db, (ds0 if S0 is not None else None)
 
 
@@ -161,7 +161,7 @@ class _GatedDelta16Fn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, g, beta, S0, scale, l2norm):
-        o, S = torch.ops.atma_hip.gated_delta_fwd(q, k, v, g, beta, S0, scale, l2norm)
+        o, S = _ops.run.gated_delta_fwd(q, k, v, g, beta, S0, scale, l2norm)
         ctx.save_for_backward(q, k, v, g, beta, S0)
         ctx.scale, ctx.l2norm = scale, l2norm
         return o, S
@@ -170,7 +170,7 @@ class _GatedDelta16Fn(torch.autograd.Function):
     def backward(ctx, dO, dS):
         q, k, v, g, beta, S0 = ctx.saved_tensors
         dO = torch.zeros_like(q) if dO is None else dO.to(v.dtype)
-        dq, dk, dv, dg, db, ds0 = torch.ops.atma_hip.gated_delta_bwd16(q, k, v, g, beta, S0, dO, dS, ctx.scale,
+        dq, dk, dv, dg, db, ds0 = _ops.run.gated_delta_bwd16(q, k, v, g, beta, S0, dO, dS, ctx.scale,
                                                                       ctx.l2norm)
         return dq, dk, dv, dg, db, (ds0 if S0 is not None else None), None, None
 
@@ -238,7 +238,7 @@ def gated_delta_prefill(q, k, v, g, beta, state_table, slots, gate_bias, seq_len
         start_signal.flag.fill_(start_signal.epoch)   # nothing to overlap with: release the waiting stream now
         start_signal = None
     if B * T > 0:
-        torch.ops.atma_hip.gated_delta_prefill(
+        _ops.run.gated_delta_prefill(
             q, k, v, g, beta, state_table, slots, o, lens, float(gate_bias[0]), float(gate_bias[1]),
             None if start_signal is None else start_signal.flag, 0 if start_signal is None else start_signal.epoch)
     return o[0] if packed else o
@@ -277,7 +277,7 @@ class StartSignal:
         return self.epoch
 
     def wait(self, timeout_us=20000):
-        torch.ops.atma_hip.wait_start_flag(self.flag, self.epoch, int(timeout_us))
+        _ops.run.wait_start_flag(self.flag, self.epoch, int(timeout_us))
 
 
 @torch.no_grad()
@@ -287,6 +287,6 @@ def gated_delta_gates(g_logit, b_logit, g_bias=0.0, b_bias=0.0, decay_as_prob=Fa
     sigmoid(b_logit + b_bias))`` -- the log-decay and write strength
     ``chunk_gated_delta_rule`` takes -- or, with ``decay_as_prob``, the decode step's
     ``(sigmoid(g_logit + g_bias), sigmoid(b_logit + b_bias))``.  fp32 in and out."""
-    g, beta = torch.ops.atma_hip.gated_delta_gates(g_logit.float(), b_logit.float(), float(g_bias),
+    g, beta = _ops.run.gated_delta_gates(g_logit.float(), b_logit.float(), float(g_bias),
                                                    float(b_bias), bool(decay_as_prob))
     return g, beta

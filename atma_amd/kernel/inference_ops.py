@@ -27,13 +27,13 @@ def squared_relu_gate(x, gate):
         raise ValueError("expected x and gate of the same [rows, width] shape")
     if gate.dtype != x.dtype:
         raise ValueError("x and gate must share a dtype")
-    return torch.ops.atma_hip.squared_relu_gate(x, gate)
+    return _ops.run.squared_relu_gate(x, gate)
 
 
 @torch.no_grad()
 def softcap_logits(logits):
     """Fuse the elementwise 15*x/sqrt(x^2+225) output soft cap (any shape, logits' dtype)."""
-    return torch.ops.atma_hip.softcap_logits(logits)
+    return _ops.run.softcap_logits(logits)
 
 
 @torch.no_grad()
@@ -48,7 +48,7 @@ def softcap_argmax(logits, ids_out=None):
     if logits.dtype not in (torch.bfloat16, torch.float16):
         raise ValueError("softcap_argmax takes 16-bit logits")
     if ids_out is None:
-        return torch.ops.atma_hip.softcap_argmax(logits)
+        return _ops.run.softcap_argmax(logits)
     rows, V = logits.shape
     if ids_out.shape != (rows,) or ids_out.dtype != torch.int64 or not ids_out.is_contiguous() \
             or ids_out.device != logits.device:
@@ -86,7 +86,7 @@ def packed_causal_conv1d(x, weight, state_table, token_seq_starts, token_seq_end
     if any(m.numel() != x.shape[0] for m in maps):
         raise ValueError("token maps must have one entry per token")
     weight = weight.to(dtype=x.dtype)
-    return torch.ops.atma_hip.packed_causal_conv1d(x, weight, state_table, *maps)
+    return _ops.run.packed_causal_conv1d(x, weight, state_table, *maps)
 
 
 def linear_tokens_supported(rows, out_features, in_features, dtype):
@@ -109,4 +109,4 @@ def linear_tokens(x, weight, bias=None):
         raise ValueError(f"linear_tokens: unsupported shape {tuple(x.shape)} x {tuple(weight.shape)} {x.dtype}")
     if weight.dtype != x.dtype or (bias is not None and bias.dtype != x.dtype):
         raise ValueError("x, weight and bias must share a dtype")
-    return torch.ops.atma_hip.linear_tokens(x, weight, bias)
+    return _ops.run.linear_tokens(x, weight, bias)

@@ -73,7 +73,7 @@ def polar_attention_fwd(q, k, v, n_keys, *, v_null, null_base, null_slope_raw, l
     if n_keys.numel() != Tq:
         raise ValueError(f"n_keys must have Tq={Tq} entries (got {n_keys.numel()})")
     p = _params(q.device, v_null, null_base, null_slope_raw, len_gain_raw, mag_beta_raw)
-    c, mag = torch.ops.atma_hip.polar_attention_fwd(q, k, v, n_keys, *p, float(eps), bool(is_causal),
+    c, mag = _ops.run.polar_attention_fwd(q, k, v, n_keys, *p, float(eps), bool(is_causal),
                                                     _window_arg(window))
     return c, mag
 
@@ -109,7 +109,7 @@ def polar_attention_packed_fwd(q, k, v, tile_seq_starts, tile_q_starts, tile_seq
     maps = [t.to(device=q.device, dtype=torch.int32).reshape(-1).contiguous()
             for t in (tile_seq_starts, tile_q_starts, tile_seq_lens)]
     p = _params(q.device, v_null, null_base, null_slope_raw, len_gain_raw, mag_beta_raw)
-    c, mag = torch.ops.atma_hip.polar_attention_packed_fwd(q, k, v, *maps, *p, float(eps),
+    c, mag = _ops.run.polar_attention_packed_fwd(q, k, v, *maps, *p, float(eps),
                                                            _window_arg(window))
     return c, mag
 
@@ -141,7 +141,7 @@ def polar_attention_decode(q, k_cache, v_cache, block_tables, context_lens, *, v
         block_tables = block_tables.contiguous()
     context_lens = context_lens.to(device=q.device, dtype=torch.int32).contiguous()
     p = _params(q.device, v_null, null_base, null_slope_raw, len_gain_raw, mag_beta_raw)
-    c, mag = torch.ops.atma_hip.polar_attention_decode(q, k_cache, v_cache, block_tables,
+    c, mag = _ops.run.polar_attention_decode(q, k_cache, v_cache, block_tables,
                                                        context_lens, *p, float(eps),
                                                        _window_arg(window))
     return c, mag
@@ -202,7 +202,7 @@ def global_decode_step(q, k_new, v_new, k_cache, v_cache, slot_mapping, block_ta
     beta = beta.to(torch.float32).reshape(B, H).contiguous()
     slots = slots.to(device=q.device, dtype=torch.int64).reshape(B).contiguous()
     p = _params(q.device, v_null, null_base, null_slope_raw, len_gain_raw, mag_beta_raw)
-    c, mag, r = torch.ops.atma_hip.global_decode_step(
+    c, mag, r = _ops.run.global_decode_step(
         q, k_new, v_new, k_cache, v_cache, slot_mapping, block_tables, context_lens, *p, gamma, beta,
         state_table, slots, float(eps), float(mem_eps), _window_arg(window))
     return c, mag, r

@@ -26,7 +26,7 @@ class PolarAttentionHip(torch.autograd.Function):
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
         p = _params(q.device, v_null, null_base, null_slope_raw, len_gain_raw, mag_beta_raw)
         nk = n_keys.to(device=q.device, dtype=torch.float32).reshape(-1).contiguous()
-        c, mag, M, L, Q2, S = torch.ops.atma_hip.polar_attention_fwd_train(
+        c, mag, M, L, Q2, S = _ops.run.polar_attention_fwd_train(
             q, k, v, nk, *p, float(eps), bool(is_causal), _window_arg(window), bool(preserve_length))
         ctx.save_for_backward(q, k, v, nk, *p, M, L, Q2, S)
         ctx.eps, ctx.is_causal, ctx.window, ctx.preserve_length = eps, is_causal, window, preserve_length
@@ -41,18 +41,18 @@ class PolarAttentionHip(torch.autograd.Function):
         B, H, Tq, d = q.shape
         win = _window_arg(ctx.window)
         # per-query preamble + parameter partial sums (one HIP kernel)
-        gs, gL, gQ2, temp, part = torch.ops.atma_hip.polar_attention_bwd_prep(
+        gs, gL, gQ2, temp, part = _ops.run.polar_attention_bwd_prep(
             gc, gm, S, M, L, Q2, nk, v_null, null_base, null_slope_raw, len_gain_raw, mag_beta_raw,
             float(ctx.eps), win, bool(ctx.preserve_length), q.dtype)
         # the O(T^2) loops
-        dq, dt, dkv = torch.ops.atma_hip.polar_attention_bwd(
+        dq, dt, dkv = _ops.run.polar_attention_bwd(
             q, k, v, gs, gL, gQ2, M, temp, nk, bool(ctx.is_causal), win)
         dk, dv = dkv[0], dkv[1]
         # parameters (one HIP launch): temp = 1 + softplus(lg) log n,
         # nu = nb + softplus(ns) sqrt(log(n + 1)), mag = tanh(softplus(mb) log1p(m_eff));
         # d softplus = sigmoid.  The real keys' share of dL/dtemp is dt; the preamble summed
         # the sink's share and the rest per block.
-        grad_v_null, g4 = torch.ops.atma_hip.polar_bwd_param_grads(
+        grad_v_null, g4 = _ops.run.polar_bwd_param_grads(
             part, dt, nk, len_gain_raw, null_slope_raw, mag_beta_raw, win, bool(ctx.preserve_length))
         grad_null_base, grad_null_slope, grad_len_gain, grad_mag_beta = g4[0], g4[1], g4[2], g4[3]
 

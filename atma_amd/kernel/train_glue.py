@@ -11,7 +11,7 @@ import ctypes
 import torch
 import torch.nn.functional as F
 
-from .. import _lib
+from .. import _lib, _ops
 from .layer_fusions import global_gate, head_rms_norm
 
 _MAX = 16
@@ -263,7 +263,7 @@ class _SquaredReluGateFn(torch.autograd.Function):
     def forward(ctx, y):
         ctx.save_for_backward(y)
         W = y.shape[1] // 2
-        return torch.ops.atma_hip.squared_relu_gate(y[:, :W], y[:, W:])
+        return _ops.run.squared_relu_gate(y[:, :W], y[:, W:])
 
     @staticmethod
     def backward(ctx, dh):

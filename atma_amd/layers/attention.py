@@ -26,7 +26,7 @@ def store_kvcache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
         raise ValueError("k_cache / v_cache must be contiguous")
     if slot_mapping.dtype != torch.int32:
         slot_mapping = slot_mapping.to(torch.int32)
-    torch.ops.atma_hip.store_kvcache(key, value, k_cache, v_cache, slot_mapping.contiguous())
+    _ops.run.store_kvcache(key, value, k_cache, v_cache, slot_mapping.contiguous())
 
 
 class Attention(nn.Module):

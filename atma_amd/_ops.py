@@ -27,13 +27,13 @@ _PLAIN = (Tensor, torch.nn.Parameter)
 
 def _undispatched(args):
     """Whether a call on these arguments has nothing to dispatch to: no tracing, autograd, transform, mode or subclass."""
-    if torch.compiler.is_compiling() or torch.is_grad_enabled() or torch._C._len_torch_dispatch_stack() \
-            or torch._C._len_torch_function_stack() or torch._C._are_functorch_transforms_active() \
-            or torch.autograd.forward_ad._current_level >= 0:
+    if torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() \
+            or torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0:
         return False
+    grad = torch.is_grad_enabled()
     for a in args:
         for t in a if type(a) is list else (a,):
-            if isinstance(t, Tensor) and type(t) not in _PLAIN:
+            if isinstance(t, Tensor) and (type(t) not in _PLAIN or (grad and t.requires_grad)):
                 return False
     return True
 

@@ -17,8 +17,10 @@
 //
 // Pass 1 (prep) is parallel over every (sequence, head, chunk); pass 2 runs the
 // chunks in order, parallel over (sequence, head) x 16-column slabs of S (the
-// state columns are independent), with the slab resident in LDS for the whole
-// sequence.  All arithmetic is fp32.
+// state columns are independent), with the slab in registers for the whole
+// sequence.  All arithmetic is fp32, the products on v_mfma_f32_16x16x4f32 (which
+// rounds as fp32 fused multiply-adds do) with the contraction index permuted, step 4 j + e
+// taking k = 16 j + 4 g + e, so that a lane's A operand comes as 16-byte reads of its row.
 #include <algorithm>
 
 #include "gated_delta.h"
@@ -30,288 +32,334 @@ __host__ __device__ constexpr int64_t gdn_rec_floats() {
   return 5 * (int64_t)kChunk * D + 4;
 }
 
+// One workgroup of four waves per (sequence, head, chunk).  Wave P forms row block P of K K^T and Q K^T, wave 0 inverts
+// I + A by 16 x 16 blocks, then wave w takes d columns [D/4 w, D/4 (w + 1)) of the records: W and U0, whose accumulators
+// are the next product's B operand as they stand.  Bound by latency, one workgroup per CU (its rows in LDS): 2,048
+// tokens of 8 heads, d = 128 42 us; 104 with the products on VALU and the inverse column by column.
 template <typename T, int D>
-__global__ void __launch_bounds__(256) gdn_prep_kernel(GdnArgs a) {
-  constexpr int C = kChunk, P = D + 1;
-  constexpr int CPT = D / 16;  // output columns per thread
-  __shared__ float Ks[C * P], Qs[C * P], Vs[C * P];
-  __shared__ float As[C * (C + 1)], Rs[C * (C + 1)];
-  __shared__ float lg[C], bet[C], ge[C];
+__global__ void __launch_bounds__(256, 1) gdn_prep_kernel(GdnArgs a) {
+  constexpr int C = kChunk, P = D + 4, PC = C + 4;
+  constexpr int KJ = D / 16, DL = D / 64;  // 16-wide k blocks over D; elements of a row per lane
+  __shared__ __attribute__((aligned(16))) float Ks[C * P], Qs[C * P], Vs[C * P];
+  __shared__ __attribute__((aligned(16))) float Tl[C * PC], Rl[C * PC];  // N = A, then T; Rq
+  __shared__ __attribute__((aligned(16))) float Nd[4 * 256];            // diagonal blocks of N^T, then of T^T
+  __shared__ __attribute__((aligned(16))) float lg[C], bet[C], bge[C], tail[C], ge[C];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c16 = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = blockIdx.x, bh = blockIdx.y;
   const int b = bh / a.H, h = bh % a.H;
   const int t0 = c * C;
 
-  // ---- rows: load, L2-normalise q/k, scale q; padded rows are zero with g = beta = 0
-  for (int r = wave; r < C; r += 4) {
-    const int t = t0 + r;
-    const bool ok = t < a.T;
-    const T* qr = (const T*)a.q + b * a.q_sb + (int64_t)t * a.q_st + h * a.q_sh;
-    const T* kr = (const T*)a.k + b * a.k_sb + (int64_t)t * a.k_st + (h / a.G) * a.k_sh;
-    const T* vr = (const T*)a.v + b * a.v_sb + (int64_t)t * a.v_st + (h / a.G) * a.v_sh;
-    float qv[D / 64 > 0 ? D / 64 : 1], kv[D / 64 > 0 ? D / 64 : 1];
-    float qq = 0.f, kk = 0.f;
-#pragma unroll
-    for (int e = 0; e < D / 64; ++e) {
-      const int d = lane + 64 * e;
-      qv[e] = ok ? to_f32(qr[d]) : 0.f;
-      kv[e] = ok ? to_f32(kr[d]) : 0.f;
-      Vs[r * P + d] = ok ? to_f32(vr[d]) : 0.f;
-      qq += qv[e] * qv[e];
-      kk += kv[e] * kv[e];
-    }
-    float iq = 1.f, ik = 1.f;
-    if (a.l2norm) {
-      iq = 1.f / fmaxf(sqrtf(wave_sum(qq)), 1e-12f);
-      ik = 1.f / fmaxf(sqrtf(wave_sum(kk)), 1e-12f);
-    }
-#pragma unroll
-    for (int e = 0; e < D / 64; ++e) {
-      const int d = lane + 64 * e;
-      Qs[r * P + d] = qv[e] * iq * a.scale;
-      Ks[r * P + d] = kv[e] * ik;
-    }
-    if (lane == 0) {
-      const int64_t gi = ((int64_t)b * a.T + t) * a.H + h;
-      lg[r] = ok ? gdn_load_g(a, gi) : 0.f;
-      bet[r] = ok ? gdn_load_beta(a, gi) : 0.f;
-    }
-  }
-  __syncthreads();
-  if (tid == 0) {
-    float run = 0.f;
-    for (int r = 0; r < C; ++r) {
-      run += lg[r];
-      lg[r] = run;
-    }
-  }
-  __syncthreads();
-  if (tid < C) ge[tid] = expf(lg[tid]);
-
-  // ---- Gram blocks: A (strict lower, scaled by beta_p) and Rq (lower incl.)
+  // ---- rows, all loads first: L2-normalise q/k, scale q; padded rows are zero with g = beta = 0
   {
-    const int tp = tid >> 4, ts = tid & 15;
-    float kk[4][4] = {}, qk[4][4] = {};
-    for (int d = 0; d < D; ++d) {
-      float kp[4], qp[4], ks[4];
+    float qv[16][DL], kv[16][DL], vv[16][DL];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        kp[i] = Ks[(4 * tp + i) * P + d];
-        qp[i] = Qs[(4 * tp + i) * P + d];
-        ks[i] = Ks[(4 * ts + i) * P + d];
+    for (int i = 0; i < 16; ++i) {
+      const int t = t0 + wave + 4 * i;
+      const bool ok = t < a.T;
+      const T* qr = (const T*)a.q + b * a.q_sb + (int64_t)t * a.q_st + h * a.q_sh;
+      const T* kr = (const T*)a.k + b * a.k_sb + (int64_t)t * a.k_st + (h / a.G) * a.k_sh;
+      const T* vr = (const T*)a.v + b * a.v_sb + (int64_t)t * a.v_st + (h / a.G) * a.v_sh;
+#pragma unroll
+      for (int e = 0; e < DL; ++e) {
+        qv[i][e] = ok ? to_f32(qr[lane + 64 * e]) : 0.f;
+        kv[i][e] = ok ? to_f32(kr[lane + 64 * e]) : 0.f;
+        vv[i][e] = ok ? to_f32(vr[lane + 64 * e]) : 0.f;
       }
+    }
+    float gl = 0.f, bt = 0.f;
+    if (wave == 0 && t0 + lane < a.T) {
+      const int64_t gi = ((int64_t)b * a.T + t0 + lane) * a.H + h;
+      gl = gdn_load_g(a, gi);
+      bt = gdn_load_beta(a, gi);
+    }
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 16; ++i) {
+      const int r = wave + 4 * i;
+      float iq = 1.f, ik = 1.f;
+      if (a.l2norm) {
+        float qq = 0.f, kk = 0.f;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          kk[i][j] += kp[i] * ks[j];
-          qk[i][j] += qp[i] * ks[j];
+        for (int e = 0; e < DL; ++e) {
+          qq += qv[i][e] * qv[i][e];
+          kk += kv[i][e] * kv[i][e];
         }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int p = 4 * tp + i, s = 4 * ts + j;
-        const float dec = s <= p ? expf(lg[p] - lg[s]) : 0.f;
-        As[p * (C + 1) + s] = s < p ? bet[p] * dec * kk[i][j] : 0.f;
-        Rs[p * (C + 1) + s] = s <= p ? dec * qk[i][j] : 0.f;
+        iq = 1.f / fmaxf(sqrtf(wave_sum(qq)), 1e-12f);
+        ik = 1.f / fmaxf(sqrtf(wave_sum(kk)), 1e-12f);
       }
+#pragma unroll
+      for (int e = 0; e < DL; ++e) {
+        Qs[r * P + lane + 64 * e] = qv[i][e] * iq * a.scale;
+        Ks[r * P + lane + 64 * e] = kv[i][e] * ik;
+        Vs[r * P + lane + 64 * e] = vv[i][e];
+      }
+    }
+    if (wave == 0) {  // inclusive log decays and the per-token factors
+      float x = gl;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const float y = __shfl_up(x, off, 64);
+        if (lane >= off) x += y;
+      }
+      const float e = expf(x);
+      lg[lane] = x;
+      bet[lane] = bt;
+      ge[lane] = e;
+      bge[lane] = bt * e;
+      tail[lane] = expf(__shfl(x, 63, 64) - x);
+    }
   }
   __syncthreads();
 
-  // ---- T = (I + A)^-1 by forward substitution; lane s owns column s
+  auto row4 = [&](const float* tile, int pitch, int row0, int k0) {  // A operand (or B of the transpose): 4 k of a row
+    return *(const f32x4*)(tile + (row0 + c16) * pitch + k0 + 4 * g);
+  };
+  auto mac4 = [&](const f32x4& x, const f32x4& y, f32x4 acc) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], y[e], acc, 0, 0, 0);
+    return acc;
+  };
+  const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+
+  // ---- row block R = wave of N = A (strictly lower, scaled by beta_p) and Rq (lower): row p = 16 R + 4 g + i, column
+  // s = 16 S + c16
+  {
+    const int R = wave;
+    f32x4 ka[KJ], qa[KJ];
+#pragma unroll
+    for (int j = 0; j < KJ; ++j) {
+      ka[j] = row4(Ks, P, 16 * R, 16 * j);
+      qa[j] = row4(Qs, P, 16 * R, 16 * j);
+    }
+#pragma unroll
+    for (int S = 0; S < 4; ++S) {
+      if (S > R) break;
+      f32x4 kk[2] = {z, z}, qk[2] = {z, z};
+#pragma unroll
+      for (int j = 0; j < KJ; ++j) {
+        const f32x4 kb = row4(Ks, P, 16 * S, 16 * j);
+        kk[j & 1] = mac4(ka[j], kb, kk[j & 1]);
+        qk[j & 1] = mac4(qa[j], kb, qk[j & 1]);
+      }
+      const int sc = 16 * S + c16;
+      f32x4 n;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int p = 16 * R + 4 * g + i;
+        const float dec = sc <= p ? expf(lg[p] - lg[sc]) : 0.f;
+        n[i] = sc < p ? bet[p] * dec * (kk[0][i] + kk[1][i]) : 0.f;
+        Tl[p * PC + sc] = n[i];
+        Rl[p * PC + sc] = sc <= p ? dec * (qk[0][i] + qk[1][i]) : 0.f;
+      }
+      if (S == R) *(f32x4*)(Nd + R * 256 + c16 * 16 + 4 * g) = n;  // N^T rows
+    }
+  }
+  __syncthreads();
+
+  // ---- T = (I + N)^-1 (wave 0): the diagonal blocks by forward substitution, lane (g, c) solving column c of block g;
+  // below them, level L = P - S, T_PS = -T_PP sum_{k=S}^{P-1} N_Pk T_kS by block products (left factors transposed)
   if (wave == 0) {
-    const int s = lane;
-    float col[C];
+    {
+      const float* nt = Nd + g * 256;
+      float x[16];
 #pragma unroll
-    for (int p = 0; p < C; ++p) {
-      float accv = (p == s) ? 1.f : 0.f;
+      for (int r = 0; r < 16; ++r) x[r] = (r == c16) ? 1.f : 0.f;
 #pragma unroll
-      for (int j = 0; j < p; ++j) accv -= As[p * (C + 1) + j] * col[j];
-      col[p] = accv;
+      for (int j = 0; j < 15; ++j) {
+        float nv[16];
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+          const f32x4 v = *(const f32x4*)(nt + j * 16 + 4 * q4);  // column j of N
+#pragma unroll
+          for (int e = 0; e < 4; ++e) nv[4 * q4 + e] = v[e];
+        }
+#pragma unroll
+        for (int r = j + 1; r < 16; ++r) x[r] = fmaf(-nv[r], x[j], x[r]);
+      }
+      wave_sync();
+      float* mt = Nd + g * 256 + c16 * 16;  // T^T row c = column c of T
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) *(f32x4*)(mt + 4 * q4) = f32x4{x[4 * q4], x[4 * q4 + 1], x[4 * q4 + 2], x[4 * q4 + 3]};
     }
+    wave_sync();
+    f32x4 tpp[4], tppT[4];  // T_PP and T_PP^T in the accumulator layout
 #pragma unroll
-    for (int p = 0; p < C; ++p) As[p * (C + 1) + s] = col[p];
+    for (int B = 0; B < 4; ++B) {
+      tpp[B] = *(const f32x4*)(Nd + B * 256 + c16 * 16 + 4 * g);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) tppT[B][i] = Nd[B * 256 + (4 * g + i) * 16 + c16];
+    }
+    auto nt = [&](int S, int B) { return row4(Tl, PC, 16 * B, 16 * S); };  // block (B, S) of N, transposed layout
+    const f32x4 n10 = nt(0, 1), n20 = nt(0, 2), n30 = nt(0, 3), n21 = nt(1, 2), n31 = nt(1, 3), n32 = nt(2, 3);
+    const f32x4 y10 = blk_mul(n10, tpp[0], z), y21 = blk_mul(n21, tpp[1], z), y32 = blk_mul(n32, tpp[2], z);
+    const f32x4 t10 = -blk_mul(tppT[1], y10, z), t21 = -blk_mul(tppT[2], y21, z);
+    const f32x4 tt01 = -blk_mul(y10, tppT[1], z), tt12 = -blk_mul(y21, tppT[2], z), tt23 = -blk_mul(y32, tppT[3], z);
+    const f32x4 y20 = blk_mul(n21, t10, blk_mul(n20, tpp[0], z)), y31 = blk_mul(n32, t21, blk_mul(n31, tpp[1], z));
+    const f32x4 t20 = -blk_mul(tppT[2], y20, z);
+    const f32x4 tt02 = -blk_mul(y20, tppT[2], z), tt13 = -blk_mul(y31, tppT[3], z);
+    const f32x4 y30 = blk_mul(n32, t20, blk_mul(n31, t10, blk_mul(n30, tpp[0], z)));
+    const f32x4 tt03 = -blk_mul(y30, tppT[3], z);
+    wave_sync();
+    // the transposed-form block (S, B) is row 16 B + c, columns 16 S + 4 g .. + 3 of T; the blocks above stay unread
+    const f32x4 tb[4][4] = {{tppT[0], z, z, z}, {tt01, tppT[1], z, z}, {tt02, tt12, tppT[2], z}, {tt03, tt13, tt23, tppT[3]}};
+#pragma unroll
+    for (int B = 0; B < 4; ++B)
+#pragma unroll
+      for (int S = 0; S <= B; ++S) *(f32x4*)(Tl + (16 * B + c16) * PC + 16 * S + 4 * g) = tb[B][S];
   }
   __syncthreads();
 
+  // ---- the records' d columns 16 n + c16 of wave w
   float* rec = (float*)a.ws + ((int64_t)bh * a.NC + c) * gdn_rec_floats<D>();
-  float* Wg = rec;
-  float* U0g = rec + C * D;
-  float* Qtg = rec + 2 * C * D;
-  float* R0g = rec + 3 * C * D;
-  float* Kdg = rec + 4 * C * D;
-
-  const int rg = tid >> 4, cg = tid & 15;
-  float w[4][CPT], u[4][CPT];
+  if (tid == 0) rec[5 * C * D] = ge[C - 1];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int nn = 0; nn < DL; ++nn) {
+    const int d = 16 * (DL * wave + nn) + c16;
+    f32x4 kb[4], vb[4];  // B operands, k = s = 16 j + 4 g + e: diag(beta ge) K and diag(beta) V
 #pragma unroll
-    for (int e = 0; e < CPT; ++e) w[i][e] = u[i][e] = 0.f;
-  for (int s = 0; s < C; ++s) {
-    float tv[4];
+    for (int j = 0; j < 4; ++j) {
+      const f32x4 bk = *(const f32x4*)(bge + 16 * j + 4 * g), bv = *(const f32x4*)(bet + 16 * j + 4 * g);
+      const f32x4 tl = *(const f32x4*)(tail + 16 * j + 4 * g);
+      f32x4 kd;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) tv[i] = As[(4 * rg + i) * (C + 1) + s];
-    const float bk = bet[s] * ge[s], bv = bet[s];
+      for (int e = 0; e < 4; ++e) {
+        const int s = 16 * j + 4 * g + e;
+        const float kx = Ks[s * P + d];
+        kb[j][e] = kx * bk[e];
+        vb[j][e] = Vs[s * P + d] * bv[e];
+        kd[e] = tl[e] * kx;
+      }
+      *(f32x4*)(rec + 4 * C * D + d * C + 16 * j + 4 * g) = kd;
+    }
+    f32x4 w[4], u[4];
 #pragma unroll
-    for (int e = 0; e < CPT; ++e) {
-      const float kx = Ks[s * P + cg + 16 * e] * bk;
-      const float vx = Vs[s * P + cg + 16 * e] * bv;
+    for (int B = 0; B < 4; ++B) {
+      w[B] = u[B] = z;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        w[i][e] += tv[i] * kx;
-        u[i][e] += tv[i] * vx;
+      for (int j = 0; j <= B; ++j) {
+        const f32x4 t = row4(Tl, PC, 16 * B, 16 * j);
+        w[B] = mac4(t, kb[j], w[B]);
+        u[B] = mac4(t, vb[j], u[B]);
       }
     }
-  }
-  const float lgC = lg[C - 1];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int p = 4 * rg + i;
-    const float tail = expf(lgC - lg[p]);
+    for (int B = 0; B < 4; ++B) {
+      f32x4 qt = z, r0 = z;
 #pragma unroll
-    for (int e = 0; e < CPT; ++e) {
-      const int d = cg + 16 * e;
-      Wg[p * D + d] = w[i][e];
-      U0g[p * D + d] = u[i][e];
-      Kdg[p * D + d] = tail * Ks[p * P + d];
-    }
-  }
-  if (tid == 0) rec[5 * C * D] = expf(lgC);
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int e = 0; e < CPT; ++e) {
-      Ks[(4 * rg + i) * P + cg + 16 * e] = w[i][e];
-      Vs[(4 * rg + i) * P + cg + 16 * e] = u[i][e];
-    }
-  __syncthreads();
-  float qt[4][CPT], r0[4][CPT];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int e = 0; e < CPT; ++e) qt[i][e] = r0[i][e] = 0.f;
-  for (int s = 0; s < C; ++s) {
-    float rv[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) rv[i] = Rs[(4 * rg + i) * (C + 1) + s];
-#pragma unroll
-    for (int e = 0; e < CPT; ++e) {
-      const float wx = Ks[s * P + cg + 16 * e];
-      const float ux = Vs[s * P + cg + 16 * e];
+      for (int j = 0; j <= B; ++j) {
+        const f32x4 r = row4(Rl, PC, 16 * B, 16 * j);
+        qt = mac4(r, w[j], qt);
+        r0 = mac4(r, u[j], r0);
+      }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        qt[i][e] += rv[i] * wx;
-        r0[i][e] += rv[i] * ux;
+        const int p = 16 * B + 4 * g + i;
+        rec[p * D + d] = w[B][i];
+        rec[C * D + p * D + d] = u[B][i];
+        rec[2 * C * D + p * D + d] = ge[p] * Qs[p * P + d] - qt[i];
+        rec[3 * C * D + p * D + d] = r0[i];
       }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int p = 4 * rg + i;
-#pragma unroll
-    for (int e = 0; e < CPT; ++e) {
-      const int d = cg + 16 * e;
-      Qtg[p * D + d] = ge[p] * Qs[p * P + d] - qt[i][e];
-      R0g[p * D + d] = r0[i][e];
     }
   }
 }
 
+// One workgroup of four waves per (sequence-head, 16 state columns): wave w owns 16 tokens of U and O and D / 4 rows of
+// the state.  The state and U pass between the waves through LDS (two barriers a chunk); the records come straight into
+// operand registers, each part loaded for the next chunk as soon as this one's is consumed; O's product, off the chain,
+// runs while U is exchanged.  Bound by the chain of a chunk, D / 4 products and 2 exchanges: 2,048 tokens of 8 heads,
+// d = 128 111 us; 355 with the records staged through LDS and the products on VALU.
 template <typename T, int D>
-__global__ void __launch_bounds__(256) gdn_scan_kernel(GdnArgs a) {
-  constexpr int C = kChunk, VS = 16, P = D + 1;
-  __shared__ float Wl[C * P], Ql[C * P], Kl[C * P];
-  __shared__ float Ss[D * (VS + 1)], Ul[C * (VS + 1)];
-  __shared__ float U0l[C * VS], R0l[C * VS];
+__global__ void __launch_bounds__(256, 1) gdn_scan_kernel(GdnArgs a) {
+  constexpr int C = kChunk, VS = 16, KJ = D / 16, RT = D / 64;
+  __shared__ __attribute__((aligned(16))) float Sl[VS * (D + 4)], Ul[VS * (C + 4)];  // [column][row]
   gdn_signal_start(a);
 
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c16 = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int bh = blockIdx.x, v0 = blockIdx.y * VS;
   const int b = bh / a.H, h = bh % a.H;
+  const int p0 = 16 * wave + 4 * g;  // the lane's tokens p0 + i
 
-  // initial state slab S[k][v0 .. v0+VS)
-  for (int i = tid; i < D * VS; i += 256) {
-    const int kx = i / VS, vx = i % VS;
-    Ss[kx * (VS + 1) + vx] = a.s0 ? a.s0[((int64_t)bh * D + kx) * D + v0 + vx] : 0.f;
-  }
+  f32x4 S[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      S[t][i] = a.s0 ? a.s0[((int64_t)bh * D + 16 * (RT * wave + t) + 4 * g + i) * D + v0 + c16] : 0.f;
 
+  f32x4 w[KJ], q[KJ], kd[RT][4], u0, r0;
+  float gC;
+  const float* rec0 = (const float*)a.ws + (int64_t)bh * a.NC * gdn_rec_floats<D>();
+  auto load_w = [&](const float* rec) {
+#pragma unroll
+    for (int j = 0; j < KJ; ++j) w[j] = *(const f32x4*)(rec + (16 * wave + c16) * D + 16 * j + 4 * g);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) u0[i] = rec[C * D + (p0 + i) * D + v0 + c16];
+  };
+  auto load_q = [&](const float* rec) {
+#pragma unroll
+    for (int j = 0; j < KJ; ++j) q[j] = *(const f32x4*)(rec + 2 * C * D + (16 * wave + c16) * D + 16 * j + 4 * g);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r0[i] = rec[3 * C * D + (p0 + i) * D + v0 + c16];
+  };
+  auto load_k = [&](const float* rec) {
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        kd[t][j] = *(const f32x4*)(rec + 4 * C * D + (16 * (RT * wave + t) + c16) * C + 16 * j + 4 * g);
+    gC = rec[5 * C * D];
+  };
+  load_w(rec0);
+  load_q(rec0);
+  load_k(rec0);
   for (int c = 0; c < a.NC; ++c) {
-    const float* rec = (const float*)a.ws + ((int64_t)bh * a.NC + c) * gdn_rec_floats<D>();
-    __syncthreads();  // previous chunk finished with the LDS operands
-    for (int i = tid; i < C * D / 4; i += 256) {
-      const int p = (4 * i) / D, d = (4 * i) % D;
-      const f32x4 wv = *(const f32x4*)(rec + 4 * i);
-      const f32x4 qv = *(const f32x4*)(rec + 2 * C * D + 4 * i);
-      const f32x4 kv = *(const f32x4*)(rec + 4 * C * D + 4 * i);
+    const float* next = rec0 + (int64_t)(c + 1) * gdn_rec_floats<D>();
+    const bool more = c + 1 < a.NC;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        Wl[p * P + d + e] = wv[e];
-        Ql[p * P + d + e] = qv[e];
-        Kl[p * P + d + e] = kv[e];
-      }
-    }
-    for (int i = tid; i < C * VS; i += 256) {
-      const int p = i / VS, vx = i % VS;
-      U0l[i] = rec[C * D + p * D + v0 + vx];
-      R0l[i] = rec[3 * C * D + p * D + v0 + vx];
-    }
-    const float gC = rec[5 * C * D];
-    __syncthreads();
-
-    // U = U0 - W S ; O = Qt S + R0   (thread: row p, 4 columns)
-    {
-      const int p = tid >> 2, vq = (tid & 3) * 4;
-      float uu[4], oo[4];
+    for (int t = 0; t < RT; ++t) *(f32x4*)(Sl + c16 * (D + 4) + 16 * (RT * wave + t) + 4 * g) = S[t];
+    __syncthreads();  // the state is whole; every wave is done with the previous U
+    f32x4 sv[KJ];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        uu[e] = U0l[p * VS + vq + e];
-        oo[e] = R0l[p * VS + vq + e];
-      }
-      for (int kx = 0; kx < D; ++kx) {
-        const float wv = Wl[p * P + kx], qv = Ql[p * P + kx];
+    for (int j = 0; j < KJ; ++j) sv[j] = *(const f32x4*)(Sl + c16 * (D + 4) + 16 * j + 4 * g);
+    f32x4 x[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}}, o[2] = {r0, x[0]};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float sv = Ss[kx * (VS + 1) + vq + e];
-          uu[e] -= wv * sv;
-          oo[e] += qv * sv;
-        }
-      }
+    for (int j = 0; j < KJ; ++j)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) Ul[p * (VS + 1) + vq + e] = uu[e];
-      const int t = c * C + p;
-      if (t < a.T) {
-        T* op = (T*)a.o + (((int64_t)b * a.T + t) * a.H + h) * D + v0 + vq;
+      for (int e = 0; e < 4; ++e) x[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j][e], sv[j][e], x[e & 1], 0, 0, 0);
+    *(f32x4*)(Ul + c16 * (C + 4) + p0) = u0 - (x[0] + x[1]);
+    if (more) load_w(next);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) op[e] = from_f32<T>(oo[e]);
-      }
-    }
-    __syncthreads();
-    // S <- gC S + Kd^T U   (thread: D*VS/256 entries of one row)
-    {
-      constexpr int EPT = D * VS / 256;
-      const int kx = (tid * EPT) / VS, vq = (tid * EPT) % VS;
-      float sn[EPT];
+    for (int j = 0; j < KJ; ++j)
 #pragma unroll
-      for (int e = 0; e < EPT; ++e) sn[e] = gC * Ss[kx * (VS + 1) + vq + e];
-      for (int p = 0; p < C; ++p) {
-        const float kd = Kl[p * P + kx];
+      for (int e = 0; e < 4; ++e) o[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[j][e], sv[j][e], o[e & 1], 0, 0, 0);
+    if (more) load_q(next);
+    __syncthreads();  // U is whole; every wave has read the state
+    f32x4 uv[4];
 #pragma unroll
-        for (int e = 0; e < EPT; ++e) sn[e] += kd * Ul[p * (VS + 1) + vq + e];
-      }
+    for (int j = 0; j < 4; ++j) uv[j] = *(const f32x4*)(Ul + c16 * (C + 4) + 16 * j + 4 * g);
 #pragma unroll
-      for (int e = 0; e < EPT; ++e) Ss[kx * (VS + 1) + vq + e] = sn[e];
+    for (int t = 0; t < RT; ++t) S[t] *= gC;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int t = 0; t < RT; ++t) S[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kd[t][j][e], uv[j][e], S[t], 0, 0, 0);
+    if (more) load_k(next);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t = c * C + p0 + i;
+      if (t < a.T) ((T*)a.o)[(((int64_t)b * a.T + t) * a.H + h) * D + v0 + c16] = from_f32<T>(o[0][i] + o[1][i]);
     }
   }
-  __syncthreads();
   if (a.s_out) {
-    for (int i = tid; i < D * VS; i += 256) {
-      const int kx = i / VS, vx = i % VS;
-      a.s_out[((int64_t)bh * D + kx) * D + v0 + vx] = Ss[kx * (VS + 1) + vx];
-    }
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        a.s_out[((int64_t)bh * D + 16 * (RT * wave + t) + 4 * g + i) * D + v0 + c16] = S[t][i];
   }
 }
 

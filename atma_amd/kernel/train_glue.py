@@ -15,6 +15,7 @@ from .. import _lib, _ops
 from .layer_fusions import global_gate, head_rms_norm
 
 _MAX = 16
+_MAX_ROWS = 65535 * 128   # gather_colsum's grid
 _P, _L, _I = ctypes.c_void_p * _MAX, ctypes.c_int64 * _MAX, ctypes.c_int32 * _MAX
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 _HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
@@ -29,13 +30,13 @@ def train_glue_served(x, *params):
     """Whether rows ``x`` with these parameters (None allowed) take the fused training forms: eager autograd on 16-bit
     GPU rows, parameters in fp32 or the rows' type, nothing tracing, transforming or dispatching around it."""
     if not (torch.is_grad_enabled() and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and x.numel() > 0
-            and type(x) in _PLAIN):
+            and type(x) in _PLAIN and not x.is_inference() and x.numel() // x.shape[-1] <= _MAX_ROWS):
         return False
     if torch.compiler.is_compiling() or torch._C._are_functorch_transforms_active() \
             or torch._C._len_torch_dispatch_stack() or torch.autograd.forward_ad._current_level >= 0 \
             or torch.is_autocast_enabled("cuda"):
         return False
-    return all(p is None or (type(p) in _PLAIN and p.device == x.device and p.is_contiguous()
+    return all(p is None or (type(p) in _PLAIN and not p.is_inference() and p.device == x.device and p.is_contiguous()
                              and p.dtype in (torch.float32, x.dtype) and p.shape[-1] % 8 == 0 and p.shape[0] % 8 == 0)
                for p in params)
 
@@ -91,7 +92,10 @@ class _LinearsFn(torch.autograd.Function):
         y = F.linear(x, w16, b16)
         ctx.inter, ctx.cols, ctx.n = inter, cols, n
         ctx.set_materialize_grads(False)
-        ctx.save_for_backward(x, w16, *params)
+        # the parameters by reference, for their shapes and for create_graph: only the converted copy is needed otherwise, so
+        # they may change before the backward, as they may when the conversion is an autograd node of its own
+        ctx.params, ctx.versions = params, [None if p is None else p._version for p in params]
+        ctx.save_for_backward(x, w16)
         if cols or (n == 1 and not inter):
             return y
         outs, at = [], 0
@@ -107,13 +111,16 @@ class _LinearsFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, *gs):
-        x, w16, *params = ctx.saved_tensors
+        x, w16 = ctx.saved_tensors
+        params = ctx.params
         n, inter, rows = ctx.n, ctx.inter, x.shape[0]
         ws, bs = params[:n], params[n:]
         need = ctx.needs_input_grad
         if all(g is None for g in gs):
             return (None,) * len(need)
         if torch.is_grad_enabled():   # create_graph: the eager form
+            if ctx.versions != [None if p is None else p._version for p in params]:
+                raise RuntimeError("a parameter needed for the double backward has been modified by an inplace operation")
             return _linears_double(x, inter, ctx.cols, ws, bs, gs, need)
         widths = ([inter * (ws[0].shape[0] // (2 * inter))] * 2 if inter else []) + \
             [w.shape[0] for w in (ws[:1] if ctx.cols else ws[1 if inter else 0:])]

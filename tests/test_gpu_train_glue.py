@@ -113,7 +113,10 @@ def test_double_backward_frozen_and_hooks(dev):
     ref = torch.autograd.grad(g2.square().sum(), [x2, m.fc.weight, m.proj.weight])
     for a, b in zip(gg, ref):
         assert (a.float() - b).abs().max() <= 0.1 * b.abs().max()    # bf16 through four GEMMs, against fp32
-    m(x).float().sum().backward()
+    y = m(x)
+    with torch.no_grad():   # a parameter may change between forward and backward: its converted copy is what is saved
+        m.proj.weight.mul_(1.0)
+    y.float().sum().backward()
     assert m.fc.bias.grad is None and m.fc.weight.grad is not None and m.proj.bias.grad is not None
     lin = Linear(16, 16).to(dev)
     h = lin.register_forward_hook(lambda *a: None)

@@ -607,7 +607,7 @@ __global__ void __launch_bounds__(256, 1) gdn_summary16_kernel(GdnArgs a) {
 // compute the same columns' output rows and issue every copy.  A wave issues at most one
 // instruction per cycle slot of its SIMD, and with one wave per SIMD the chain's step time
 // is its instruction count; the output products, q reads, stores and copies move to the two
-// SIMDs the two-wave form leaves idle.  Per chunk c, between the top barrier B0 and the
+// SIMDs that the chain leaves idle.  Per chunk c, between the top barrier B0 and the
 // middle barrier B1 the chain reads S_c's fragments from its registers and writes U_c's to
 // LDS; after B1 it updates S and writes S_{c+1}'s fragments.  The output wave reads S_c's
 // fragments before B1 (the chain overwrites them only after B1) and U_c's after B1 (the

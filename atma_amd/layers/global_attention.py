@@ -11,9 +11,10 @@ gated-delta memory, with the reference's parameter names and three routes.
   cache; conv / memory states advance in place.  Fixed shapes, no host sync:
   graph capturable.
 
-The Polar and gated-delta arithmetic runs in the HIP kernels (``atma_amd.kernel``);
-projections, RMSNorm and the depthwise Canon conv stay eager, as in the reference.
-Unlike the reference, K/V reach the Polar and gated-delta kernels unexpanded (GQA is
+The Polar and gated-delta arithmetic runs in the HIP kernels (``atma_amd.kernel``), and so do the
+norms, the Canon convs and the gates at the shapes they serve (``canon_qkv``, ``global_gate``, in
+training ``kernel/train_glue``); projections are library GEMMs, and every other shape stays eager, as in
+the reference.  Unlike the reference, K/V reach the Polar and gated-delta kernels unexpanded (GQA is
 resolved in-kernel).
 Prefill schedule (``overlap``): the memory branch may run on a second HIP stream beside
 Polar attention (the two only share their inputs).  The gated-delta recurrence is
@@ -22,11 +23,13 @@ quarter of the CUs or less: long sequences, small batches), and only if its work
 start before Polar's fill the GPU; Polar's launch therefore waits on the recurrence's
 start signal (``StartSignal``).  ``overlap="auto"`` (default) takes the overlapped
 schedule for sequences of ``OVERLAP_TOKENS`` or more when ``recurrence_pays_to_overlap``
-says so, ``True`` always, ``False`` never.  Results are bitwise the same in every schedule.
+says so, ``True`` always, ``False`` never.  Results agree in every schedule: bitwise where the
+recurrence is not split along tokens, else to rounding.
 Training: when autograd must see the call (grad mode on and an input or parameter
 requiring grad), the full-sequence route runs the differentiable ops -- ``polar_attention``
 (HIP forward with saved statistics + HIP backward) and the autograd form of
-``chunk_gated_delta_rule`` -- back to back on one stream, as the reference's training
+``chunk_gated_delta_rule`` -- back to back on one stream, in 16 bits with the projections and the
+elementwise parts as the fused nodes of ``kernel/train_glue`` (``_forward_train``), as the reference's training
 layer is differentiable (``model/reference.py:172``, ``train/model.py:747-754``).
 """
 
@@ -714,7 +717,7 @@ class MLP(nn.Module):
                 # that never writes the 8 dim-wide projection (linear_gated)
                 h = linear_gated(x.view(rows, K), self.fc.weight, self.fc.bias)
                 return self.proj(h.view(*x.shape[:-1], -1))
-        if train_glue_served(x) and plain_module(self.fc, Linear):
+        if train_glue_served(x) and plain_module(self.fc, Linear) and self.fc.weight.shape[0] % 16 == 0:
             y = self.fc(x)
             return self.proj(squared_relu_gate_train(y.view(-1, y.shape[-1])).view(*y.shape[:-1], -1))
         a, gate = torch.chunk(self.fc(x), 2, dim=-1)

@@ -118,6 +118,8 @@ def test_double_backward_frozen_and_hooks(dev):
         m.proj.weight.mul_(1.0)
     y.float().sum().backward()
     assert m.fc.bias.grad is None and m.fc.weight.grad is not None and m.proj.bias.grad is not None
+    odd = MLP(5).to(dev)   # widths that the launches do not serve: eager
+    odd(torch.randn(3, 5, device=dev).bfloat16().requires_grad_()).float().sum().backward()
     lin = Linear(16, 16).to(dev)
     h = lin.register_forward_hook(lambda *a: None)
     assert not plain_module(lin, Linear)

@@ -25,10 +25,18 @@ run = SimpleNamespace()
 _PLAIN = (Tensor, torch.nn.Parameter)
 
 
+def watched():
+    """Whether something records or transforms the calls made now: a compiler, the JIT tracer, a dispatch mode, functorch,
+    forward-mode AD.  It sees torch ops and registered ops only: a launch made past them is missing from its record, whose
+    replay then reads memory that nobody wrote."""
+    return (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
+            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._are_functorch_transforms_active()
+            or torch.autograd.forward_ad._current_level >= 0)
+
+
 def _undispatched(args):
-    """Whether a call on these arguments has nothing to dispatch to: no tracing, autograd, transform, mode or subclass."""
-    if torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() \
-            or torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0:
+    """Whether a call on these arguments has nothing to dispatch to: no watcher, function mode, autograd or subclass."""
+    if watched() or torch._C._len_torch_function_stack():
         return False
     grad = torch.is_grad_enabled()
     for a in args:

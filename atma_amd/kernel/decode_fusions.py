@@ -19,7 +19,7 @@ import ctypes
 
 import torch
 
-from .. import _lib
+from .. import _lib, _ops
 
 _DT = (torch.bfloat16, torch.float16)
 
@@ -63,7 +63,7 @@ class PartialSums:
 
     def _summable(self):
         t = self.parts if self.base is None else self.base
-        return (not torch.is_grad_enabled() and t.is_cuda and self.dtype in _DT and t.shape[-1] % 8 == 0
+        return (not torch.is_grad_enabled() and not _ops.watched() and t.is_cuda and self.dtype in _DT and t.shape[-1] % 8 == 0
                 and 8 <= t.shape[-1] <= 4096 and len(self.biases) <= 3
                 and (t.dtype == torch.float32 and t.is_contiguous() and t.shape[0] <= 8 if self.base is None
                      else t.dtype == self.dtype and t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0)

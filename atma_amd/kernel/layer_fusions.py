@@ -11,7 +11,7 @@ Inference only (no autograd), 16-bit tensors on the GPU, graph capturable.
 
 import torch
 
-from .. import _lib
+from .. import _lib, _ops
 
 _DT = (torch.bfloat16, torch.float16)
 
@@ -129,8 +129,9 @@ def linear_gated(x, weight, bias=None):
 
 
 def memory_gate_logits_supported(x, wg, wb):
-    """Rows ``memory_gate_logits`` serves: contiguous 16-bit (..., K) with K a multiple of 128, at most 16 heads."""
-    return (x.is_cuda and x.dtype in _DT and x.is_contiguous() and x.data_ptr() % 16 == 0 and x.shape[-1] % 128 == 0
+    """Rows ``memory_gate_logits`` serves: contiguous 16-bit (..., K) with K a multiple of 128, at most 16 heads; not
+    where the call is recorded (``_ops.watched``)."""
+    return (not _ops.watched() and x.is_cuda and x.dtype in _DT and x.is_contiguous() and x.data_ptr() % 16 == 0 and x.shape[-1] % 128 == 0
             and x.shape[-1] > 0 and wg.shape == wb.shape and wg.shape[0] <= 16 and wg.shape[1] == x.shape[-1]
             and wg.dtype == wb.dtype == x.dtype and wg.is_contiguous() and wb.is_contiguous()
             and wg.data_ptr() % 16 == 0 and wb.data_ptr() % 16 == 0)
@@ -155,7 +156,7 @@ def memory_gate_logits(x, wg, bg, wb, bb):
 def paged_kv_concat(k_cache, v_cache, pages, cached, k_new, v_new):
     """A continued sequence's keys and values, contiguous: its first ``cached`` rows from the paged caches (num_pages,
     page_size, Hkv, d), ``pages`` (1-D int32) naming the page of each page_size rows, then the chunk's k_new, v_new
-    (T, Hkv, d).  Returns two (cached + T, Hkv, d) tensors, one launch."""
+    (T, Hkv, d).  Returns two (cached + T, Hkv, d) tensors, one launch (torch ops where the call is recorded)."""
     num_pages, page, Hkv, d = k_cache.shape
     T = k_new.shape[0]
     if k_cache.shape != v_cache.shape or not (k_cache.is_contiguous() and v_cache.is_contiguous()) \
@@ -163,6 +164,9 @@ def paged_kv_concat(k_cache, v_cache, pages, cached, k_new, v_new):
             or any(t.dtype != k_cache.dtype for t in (v_cache, k_new, v_new)) \
             or any(t.stride(2) != 1 or t.stride(1) != d for t in (k_new, v_new)):
         raise ValueError("paged_kv_concat: contiguous caches, chunk rows (T, Hkv, d) and pages for every cached row")
+    if _ops.watched():   # torch ops, which what records the call can see
+        rows = pages.long()
+        return tuple(torch.cat([c[rows].reshape(-1, Hkv, d)[:cached], t], 0) for c, t in ((k_cache, k_new), (v_cache, v_new)))
     pages = pages.to(device=k_cache.device, dtype=torch.int32).contiguous()
     kb, vb = (torch.empty((cached + T, Hkv, d), device=k_cache.device, dtype=k_cache.dtype) for _ in range(2))
     rc = _lib.load().atma_paged_kv_concat(k_cache.data_ptr(), v_cache.data_ptr(), num_pages, page, pages.data_ptr(), cached,

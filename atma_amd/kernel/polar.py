@@ -14,7 +14,7 @@ from .. import _lib, _ops  # noqa: F401  (_ops registers torch.ops.atma_hip.*)
 def _params(device, v_null, null_base, null_slope_raw, len_gain_raw, mag_beta_raw):
     """The five parameters in fp32 on ``device``; those of a 16-bit layer widened in one launch."""
     ps = (v_null, null_base, null_slope_raw, len_gain_raw, mag_beta_raw)
-    if v_null.dtype in (torch.bfloat16, torch.float16) and not torch.compiler.is_compiling() and v_null.dim() == 2 \
+    if v_null.dtype in (torch.bfloat16, torch.float16) and not _ops.watched() and v_null.dim() == 2 \
             and all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.device == device
                     and t.dtype == v_null.dtype and t.is_contiguous() for t in ps) \
             and all(t.numel() == v_null.shape[0] for t in ps[1:]):

@@ -40,6 +40,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from .. import _ops
 from ..kernel import (StartSignal, causal_conv1d_decode_step, chunk_gated_delta_rule,
                       gated_delta_decode_step, gated_delta_gates, global_decode_step, polar_attention,
                       polar_attention_decode, polar_attention_fwd, polar_attention_packed_fwd,
@@ -254,8 +255,8 @@ class PolarAttention(nn.Module):
 
     def _glue_fusable(self, x):
         """16-bit GPU inference with the memory branch: the per-head glue runs as the
-        layer-fusion kernels (``head_rms_norm``, ``global_gate``)."""
-        return (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and not torch.is_grad_enabled()
+        layer-fusion kernels (``head_rms_norm``, ``global_gate``).  Not where the call is recorded (``_ops.watched``)."""
+        return (not _ops.watched() and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and not torch.is_grad_enabled()
                 and self.head_dim in (64, 128) and self.mem is not None)
 
     def _project(self, x):
@@ -285,6 +286,7 @@ class PolarAttention(nn.Module):
         if cache is not None:
             served = served and all(t.dtype == x.dtype and t.is_contiguous()
                                     for t in (*tables, cache.k_cache, cache.v_cache))
+        served = served and (torch.is_grad_enabled() or not _ops.watched())   # (canon_conv is a registered op)
         if served and not torch.is_grad_enabled():
             qg = self.q(x).view(rows, H, 2 * dk)
             q, k, v = canon_qkv(qg[..., :dk], self.k(x).view(rows, Hkv, dk), self.v(x).view(rows, Hkv, dk),

@@ -122,9 +122,11 @@ class TitansMemory(nn.Module):
 
     def raw_logits(self, x):
         """Gate logits before the retention and write biases (fp32), which the fused gate kernel adds together with
-        the activations.  16-bit inference rows: both projections in one launch (``memory_gate_logits``)."""
+        the activations.  16-bit inference rows: both projections in one launch (``memory_gate_logits``) where they are
+        this file's Linears without hooks, whose calls it does not make."""
         wg, wb = self.w_gamma, self.w_beta
-        if not torch.is_grad_enabled() and x.dim() > 2 and memory_gate_logits_supported(x, wg.weight, wb.weight):
+        if not torch.is_grad_enabled() and x.dim() > 2 and plain_module(wg, Linear) and plain_module(wb, Linear) \
+                and memory_gate_logits_supported(x, wg.weight, wb.weight):
             return memory_gate_logits(x, wg.weight, wg.bias, wb.weight, wb.bias)
         return self.w_gamma(x).float(), self.w_beta(x).float()
 
@@ -258,6 +260,13 @@ class PolarAttention(nn.Module):
         layer-fusion kernels (``head_rms_norm``, ``global_gate``).  Not where the call is recorded (``_ops.watched``)."""
         return (not _ops.watched() and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and not torch.is_grad_enabled()
                 and self.head_dim in (64, 128) and self.mem is not None)
+
+    def _out_fusable(self, x):
+        """The output is formed from the weights (``_fused_out``, and the memory's readout alone): ``_glue_fusable``, and
+        the modules that are then not called are what this file makes of them, without hooks."""
+        m = self.mem
+        return (self._glue_fusable(x) and plain_module(m, TitansMemory)
+                and all(plain_module(l, Linear) for l in (self.proj, self.mu_proj, m.proj)))
 
     def _project(self, x):
         """q/gate, k, v projections and per-head RMSNorm of q, k (``model/reference.py:131-139``).
@@ -480,7 +489,7 @@ class PolarAttention(nn.Module):
         H, dk = self.num_heads, self.head_dim
         n_keys = torch.arange(1, T + 1, device=x.device, dtype=torch.float32)
         qh, kh, vh = (t.transpose(1, 2) for t in (q, k, v))   # (B, heads, T, dk) views
-        fused = self._glue_fusable(x)
+        fused = self._out_fusable(x)
 
         # under autograd the differentiable op (HIP forward with saved statistics, HIP
         # backward loops); otherwise the forward-only kernel
@@ -528,7 +537,7 @@ class PolarAttention(nn.Module):
         H, Hkv, dk = self.num_heads, self.num_kv_heads, self.head_dim
         q, gate, k, v = self._project_canon(x, 1, total, cache, slots, slot_mapping, token_maps=token_maps)
         c, mag = polar_attention_packed_fwd(q, k, v, *tile_maps, window=self.window, **self.polar_params())
-        fused = self._glue_fusable(x)
+        fused = self._out_fusable(x)
         if fused and gated_delta_prefill_supported(q, cache.mem_table):
             r = self.mem.readout_table(x, q, k, v, cache.mem_table, slots, seq_lens)
             res = self._fused_out(x, c.view(1, total, H, dk), mag, gate, r)
@@ -584,7 +593,7 @@ class PolarAttention(nn.Module):
                 ms.append(mag.transpose(1, 2))
             return (cs[0], ms[0]) if B == 1 else (torch.cat(cs), torch.cat(ms))
 
-        fused = self._glue_fusable(x)
+        fused = self._out_fusable(x)
         (c, mag), m = self._with_memory(attend,
                                         lambda signal: self._memory(x, q, k, v, fused, cache, slots, signal),
                                         (x, q, k, v))

@@ -33,12 +33,11 @@ def plain_module(m, cls):
 def train_glue_served(x, *params):
     """Whether rows ``x`` with these parameters (None allowed) take the fused training forms: eager autograd on 16-bit
     GPU rows, parameters in fp32 or the rows' type, nothing tracing, transforming or dispatching around it."""
-    if not (torch.is_grad_enabled() and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and x.numel() > 0
-            and type(x) in _PLAIN and not x.is_inference() and x.numel() // x.shape[-1] <= _MAX_ROWS):
+    # what records the call first: a compiler refuses some of the questions after it
+    if not torch.is_grad_enabled() or _ops.watched() or torch.is_autocast_enabled("cuda"):
         return False
-    if torch.compiler.is_compiling() or torch._C._are_functorch_transforms_active() \
-            or torch._C._len_torch_dispatch_stack() or torch.autograd.forward_ad._current_level >= 0 \
-            or torch.is_autocast_enabled("cuda"):
+    if not (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and x.numel() > 0 and type(x) in _PLAIN
+            and not x.is_inference() and x.numel() // x.shape[-1] <= _MAX_ROWS):
         return False
     return all(p is None or (type(p) in _PLAIN and not p.is_inference() and p.device == x.device and p.is_contiguous()
                              and p.dtype in (torch.float32, x.dtype) and p.shape[-1] % 8 == 0 and p.shape[0] % 8 == 0)

@@ -80,8 +80,18 @@ def _need_cuda(*ts):
 def _rows16(t: Tensor) -> Tensor:
     """Return t with unit innermost stride and 16-byte aligned rows/base."""
     es = t.element_size()
-    ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all((s * es) % 16 == 0 for s in t.stride()[:-1])
-    return t if ok else t.contiguous()
+    if t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all((s * es) % 16 == 0 for s in t.stride()[:-1]):
+        return t
+    t = _aligned16(t)
+    # (``contiguous`` keeps whatever stride a dimension of one has)
+    odd = any(n == 1 and (s * es) % 16 for n, s in zip(t.shape[:-1], t.stride()))
+    return t.clone(memory_format=torch.contiguous_format) if odd else t
+
+
+def _aligned16(t: Tensor) -> Tensor:
+    """Return t contiguous at a 16-byte aligned address (``contiguous`` hands a misaligned contiguous view back)."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
 
 
 # --------------------------------------------------------------------------- Polar fwd

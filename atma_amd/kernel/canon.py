@@ -25,10 +25,10 @@ def canon_supported(x, head_dim, kernel_size):
 
 
 def _taps(weights, dtype):
-    """Conv1d weights (C, 1, K) as contiguous taps, all in the rows' dtype or all in fp32."""
+    """Conv1d weights (C, 1, K) as contiguous aligned taps, all in the rows' dtype or all in fp32."""
     ws = [w.detach() for w in weights]
     dt = torch.float32 if all(w.dtype == torch.float32 for w in ws) else dtype
-    return [w.to(dt).contiguous() for w in ws], dt
+    return [_ops._aligned16(w.to(dt)) for w in ws], dt
 
 
 @torch.no_grad()
@@ -36,8 +36,8 @@ def canon_qkv(q, k, v, weights, eps, *, seq_len=0, token_maps=None, tails=None, 
               caches=None, slot_mapping=None):
     """``x + conv(x)`` of v and of the per-head RMS-normed (``eps``) q and k, one launch.
 
-    q: (rows, H, d), k, v: (rows, Hkv, d) views with unit inner stride and 16-byte aligned head-rows (q as the first
-    half of every head of the q|gate projection is read in place).  weights: the three depthwise conv weights.  Rows
+    q: (rows, H, d), k, v: (rows, Hkv, d) views with unit inner stride, read in place where head-rows are 16-byte aligned
+    (q as the first half of every head of the q|gate projection).  weights: the three depthwise conv weights.  Rows
     are sequences of ``seq_len``, or packed by ``token_maps`` (starts, ends, table rows; int32, one per token).
     ``tails``: the three conv state tables (rows, C, K - 1), written with each sequence's last K - 1 conv inputs in
     row ``slots[b]`` (or the token map's); ``continuing`` reads them first as the left context.  ``caches`` (k, v)
@@ -50,6 +50,7 @@ def canon_qkv(q, k, v, weights, eps, *, seq_len=0, token_maps=None, tails=None, 
     for t, h, w in zip(xs, heads, taps):
         if t.shape != (rows, h, d) or t.dtype != q.dtype or t.stride(2) != 1 or w.numel() != h * d * K:
             raise ValueError("canon_qkv: q, k, v (rows, heads, d) in one dtype and conv weights (heads d, 1, K)")
+    xs = [_ops._rows16(t) for t in xs]
     dev = q.device
     outs = [torch.empty((rows, h, d), device=dev, dtype=q.dtype) for h in heads]
     tp, ts, num_slots = (None,) * 3, (0,) * 3, 0

@@ -66,10 +66,14 @@ class PartialSums:
         return (not torch.is_grad_enabled() and not _ops.watched() and t.is_cuda and self.dtype in _DT and t.shape[-1] % 8 == 0
                 and 8 <= t.shape[-1] <= 4096 and len(self.biases) <= 3
                 and (t.dtype == torch.float32 and t.is_contiguous() and t.shape[0] <= 8 if self.base is None
-                     else t.dtype == self.dtype and t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0)
+                     else t.dtype == self.dtype and t.stride(1) == 1 and t.stride(0) % 8 == 0
+                     and t.stride(0) >= t.shape[1] and t.data_ptr() % 16 == 0)
                 and all(b.dtype == self.dtype and b.data_ptr() % 16 == 0 for b in self.biases)
                 and (self.mu_x is None or (self.mu_x.shape[1] in (4, 8, 16) and self.mu_x.dtype == self.dtype
-                                           and self.mu_w.dtype == self.dtype and self.mu_x.stride(1) == 1)))
+                                           and self.mu_w.dtype == self.dtype and self.mu_x.stride(1) == 1
+                                           and self.mu_x.stride(0) >= self.mu_x.shape[1]
+                                           and self.mu_x.stride(0) % 2 == 0 and self.mu_x.data_ptr() % 4 == 0
+                                           and (self.mu_w.data_ptr() % 16 == 0 or not self.mu_w.is_contiguous()))))
 
     def materialize(self):
         if self._summable():

@@ -156,7 +156,8 @@ def memory_gate_logits(x, wg, bg, wb, bb):
 def paged_kv_concat(k_cache, v_cache, pages, cached, k_new, v_new):
     """A continued sequence's keys and values, contiguous: its first ``cached`` rows from the paged caches (num_pages,
     page_size, Hkv, d), ``pages`` (1-D int32) naming the page of each page_size rows, then the chunk's k_new, v_new
-    (T, Hkv, d).  Returns two (cached + T, Hkv, d) tensors, one launch (torch ops where the call is recorded)."""
+    (T, Hkv, d).  Returns two (cached + T, Hkv, d) tensors, one launch (torch ops where the call is recorded
+    or rows are not 16-byte aligned)."""
     num_pages, page, Hkv, d = k_cache.shape
     T = k_new.shape[0]
     if k_cache.shape != v_cache.shape or not (k_cache.is_contiguous() and v_cache.is_contiguous()) \
@@ -164,7 +165,8 @@ def paged_kv_concat(k_cache, v_cache, pages, cached, k_new, v_new):
             or any(t.dtype != k_cache.dtype for t in (v_cache, k_new, v_new)) \
             or any(t.stride(2) != 1 or t.stride(1) != d for t in (k_new, v_new)):
         raise ValueError("paged_kv_concat: contiguous caches, chunk rows (T, Hkv, d) and pages for every cached row")
-    if _ops.watched():   # torch ops, which what records the call can see
+    if _ops.watched() or any(t.data_ptr() % 16 or t.stride(0) * t.element_size() % 16
+                             for t in (k_cache, v_cache, k_new, v_new)):   # torch ops: recorded, or not the kernel's rows
         rows = pages.long()
         return tuple(torch.cat([c[rows].reshape(-1, Hkv, d)[:cached], t], 0) for c, t in ((k_cache, k_new), (v_cache, v_new)))
     pages = pages.to(device=k_cache.device, dtype=torch.int32).contiguous()

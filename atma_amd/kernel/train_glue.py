@@ -32,7 +32,8 @@ def plain_module(m, cls):
 
 def train_glue_served(x, *params):
     """Whether rows ``x`` with these parameters (None allowed) take the fused training forms: eager autograd on 16-bit
-    GPU rows, parameters in fp32 or the rows' type, nothing tracing, transforming or dispatching around it."""
+    GPU rows, parameters in fp32 or the rows' type at 16-byte aligned addresses (the kernels' loads; a view behind an odd
+    offset of a flat buffer is not), nothing tracing, transforming or dispatching around it."""
     # what records the call first: a compiler refuses some of the questions after it
     if not torch.is_grad_enabled() or _ops.watched() or torch.is_autocast_enabled("cuda"):
         return False
@@ -40,7 +41,8 @@ def train_glue_served(x, *params):
             and not x.is_inference() and x.numel() // x.shape[-1] <= _MAX_ROWS):
         return False
     return all(p is None or (type(p) in _PLAIN and not p.is_inference() and p.device == x.device and p.is_contiguous()
-                             and p.dtype in (torch.float32, x.dtype) and p.shape[-1] % 8 == 0 and p.shape[0] % 8 == 0)
+                             and p.dtype in (torch.float32, x.dtype) and p.shape[-1] % 8 == 0 and p.shape[0] % 8 == 0
+                             and p.data_ptr() % 16 == 0)
                for p in params)
 
 
@@ -58,8 +60,7 @@ def _cast_blocks(blocks):
 
 def _rows2d(t, rows):
     """(rows, width) with unit inner stride and 16-byte aligned rows, by a copy if need be."""
-    t = t.reshape(rows, -1)
-    return t if t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 else t.contiguous()
+    return _ops._rows16(t.reshape(rows, -1))
 
 
 class _LinearsFn(torch.autograd.Function):
@@ -218,7 +219,7 @@ class _HeadNormFn(torch.autograd.Function):
             ys = [F.rms_norm(x, (x.shape[-1],), eps=ctx.eps) for x in xs]
             return (*(torch.autograd.grad(y, x, g, create_graph=True)[0] for y, x, g in zip(ys, xs, (dq, dk))), None)
         rows, d = xs[0].shape[0], xs[0].shape[2]
-        dn = [g.contiguous() for g in (dq, dk)]
+        dn = [_ops._aligned16(g) for g in (dq, dk)]
         dx = [torch.empty_like(g) for g in dn]
         rc = _lib.load().atma_head_norm_bwd(
             _P(*[x.data_ptr() for x in xs]), _L(*[x.stride(0) for x in xs]), _L(*[x.stride(1) for x in xs]),
@@ -251,7 +252,7 @@ class _GateFn(torch.autograd.Function):
             xa = (c * torch.sigmoid(gate.view_as(c))).reshape(rows, H * d)
             xm = F.rms_norm(r, (d,), eps=ctx.eps).reshape(rows, H * d) * torch.sigmoid(mgate)
             return (*torch.autograd.grad(torch.cat((xa, xm), 1), (c, gate, r, mgate), dx, create_graph=True), None)
-        dx = dx.contiguous()
+        dx = _ops._aligned16(dx)
         dc, dgate, dr, dmg = (c.new_empty((rows, H, d)) for _ in range(4))
         rc = _lib.load().atma_global_gate_bwd(
             c.data_ptr(), c.stride(0), c.stride(1), c.stride(2), c.shape[1], gate.data_ptr(), gate.stride(0),

@@ -294,7 +294,8 @@ class PolarAttention(nn.Module):
         tables = None if cache is None else (cache.conv_q, cache.conv_k, cache.conv_v)
         if cache is not None:
             served = served and all(t.dtype == x.dtype and t.is_contiguous()
-                                    for t in (*tables, cache.k_cache, cache.v_cache))
+                                    for t in (*tables, cache.k_cache, cache.v_cache)) \
+                and (cache.k_cache.data_ptr() | cache.v_cache.data_ptr()) % 16 == 0
         served = served and (torch.is_grad_enabled() or not _ops.watched())   # (canon_conv is a registered op)
         if served and not torch.is_grad_enabled():
             qg = self.q(x).view(rows, H, 2 * dk)

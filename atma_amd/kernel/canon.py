@@ -13,6 +13,7 @@ import torch
 import torch.nn.functional as F
 
 from .. import _lib, _ops  # noqa: F401  (_ops registers torch.ops.atma_hip.*)
+from .train_glue import eager_grads
 
 _DT = (torch.float32, torch.bfloat16, torch.float16)
 _P3, _L3, _I3 = ctypes.c_void_p * 3, ctypes.c_int64 * 3, ctypes.c_int * 3
@@ -105,10 +106,7 @@ class _CanonConvFn(torch.autograd.Function):
     def backward(ctx, *gy):
         saved = ctx.saved_tensors
         if torch.is_grad_enabled():   # create_graph: differentiable ops
-            grads = []
-            for x, w, g in zip(saved[:3], saved[3:], gy):
-                grads.append(torch.autograd.grad(_conv_torch(x, w), (x, w), g, create_graph=True))
-            return tuple(g[0] for g in grads) + tuple(g[1] for g in grads)
+            return tuple(eager_grads([_conv_torch(x, w) for x, w in zip(saved[:3], saved[3:])], saved, gy))
         return tuple(_ops.run.canon_conv_bwd([g.contiguous() for g in gy], list(saved[:3]), list(saved[3:])))
 
 

@@ -63,6 +63,20 @@ def _rows2d(t, rows):
     return _ops._rows16(t.reshape(rows, -1))
 
 
+def eager_grads(outs, ins, gs):
+    """The gradients of eager outs with respect to ins, differentiable themselves; None where an input is None or takes no
+    gradient (frozen parameters, rows that nothing trained leads to) or an output's gradient is None."""
+    live = [(o, g) for o, g in zip(outs, gs) if g is not None and o.requires_grad]
+    idx = [i for i, t in enumerate(ins) if t is not None and t.requires_grad]
+    res = [None] * len(ins)
+    if live and idx:
+        got = torch.autograd.grad([o for o, _ in live], [ins[i] for i in idx], [g for _, g in live], create_graph=True,
+                                  allow_unused=True)
+        for i, g in zip(idx, got):
+            res[i] = g
+    return res
+
+
 class _LinearsFn(torch.autograd.Function):
     """Several Linears as one GEMM.  ``cols`` False: of one input x (rows, K), outputs side by side; with ``inter`` the
     first is split by heads into two of that width, (rows, H, inter) each.  ``cols`` True: of inputs side by side in x,
@@ -125,7 +139,7 @@ class _LinearsFn(torch.autograd.Function):
         if torch.is_grad_enabled():   # create_graph: the eager form
             if ctx.versions != [None if p is None else p._version for p in params]:
                 raise RuntimeError("a parameter needed for the double backward has been modified by an inplace operation")
-            return _linears_double(x, inter, ctx.cols, ws, bs, gs, need)
+            return _linears_double(x, inter, ctx.cols, ws, bs, gs)
         widths = ([inter * (ws[0].shape[0] // (2 * inter))] * 2 if inter else []) + \
             [w.shape[0] for w in (ws[:1] if ctx.cols else ws[1 if inter else 0:])]
         parts = [None if g is None else _rows2d(g, rows) for g in gs]
@@ -166,7 +180,7 @@ class _LinearsFn(torch.autograd.Function):
         return (dx, None, None, *grads)
 
 
-def _linears_double(x, inter, cols, ws, bs, gs, need):
+def _linears_double(x, inter, cols, ws, bs, gs):
     ws16, bs16 = [w.type_as(x) for w in ws], [None if b is None else b.type_as(x) for b in bs]
     if cols:
         ks = [w.shape[1] for w in ws]
@@ -176,14 +190,7 @@ def _linears_double(x, inter, cols, ws, bs, gs, need):
         if inter:
             o = outs[0].view(x.shape[0], -1, 2, inter)
             outs = [o[:, :, 0], o[:, :, 1]] + outs[1:]
-    ins = [x, *ws, *bs]
-    idx = [i for i, t in enumerate(ins) if t is not None and t.requires_grad and need[i and i + 2]]
-    live = [(o, g) for o, g in zip(outs, gs) if g is not None]
-    got = torch.autograd.grad([o for o, _ in live], [ins[i] for i in idx], [g for _, g in live], create_graph=True,
-                              allow_unused=True)
-    res = [None] * len(ins)
-    for i, g in zip(idx, got):
-        res[i] = g
+    res = eager_grads(outs, [x, *ws, *bs], gs)
     return (res[0], None, None, *res[1:])
 
 
@@ -217,7 +224,7 @@ class _HeadNormFn(torch.autograd.Function):
         xs = ctx.saved_tensors
         if torch.is_grad_enabled():
             ys = [F.rms_norm(x, (x.shape[-1],), eps=ctx.eps) for x in xs]
-            return (*(torch.autograd.grad(y, x, g, create_graph=True)[0] for y, x, g in zip(ys, xs, (dq, dk))), None)
+            return (*eager_grads(ys, xs, (dq, dk)), None)
         rows, d = xs[0].shape[0], xs[0].shape[2]
         dn = [_ops._aligned16(g) for g in (dq, dk)]
         dx = [torch.empty_like(g) for g in dn]
@@ -251,7 +258,7 @@ class _GateFn(torch.autograd.Function):
         if torch.is_grad_enabled():
             xa = (c * torch.sigmoid(gate.view_as(c))).reshape(rows, H * d)
             xm = F.rms_norm(r, (d,), eps=ctx.eps).reshape(rows, H * d) * torch.sigmoid(mgate)
-            return (*torch.autograd.grad(torch.cat((xa, xm), 1), (c, gate, r, mgate), dx, create_graph=True), None)
+            return (*eager_grads([torch.cat((xa, xm), 1)], (c, gate, r, mgate), [dx]), None)
         dx = _ops._aligned16(dx)
         dc, dgate, dr, dmg = (c.new_empty((rows, H, d)) for _ in range(4))
         rc = _lib.load().atma_global_gate_bwd(
@@ -282,7 +289,7 @@ class _SquaredReluGateFn(torch.autograd.Function):
         W = y.shape[1] // 2
         if torch.is_grad_enabled():
             a, gate = y.chunk(2, 1)
-            return torch.autograd.grad(gate * a.relu().square(), y, dh, create_graph=True)[0]
+            return eager_grads([gate * a.relu().square()], [y], [dh])[0]
         dh = _rows2d(dh, y.shape[0])
         dy = torch.empty_like(y)
         rc = _lib.load().atma_squared_relu_gate_bwd(y.data_ptr(), y.stride(0), dh.data_ptr(), dh.stride(0), dy.data_ptr(),

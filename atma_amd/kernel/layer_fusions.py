@@ -14,6 +14,7 @@ import torch
 from .. import _lib, _ops
 
 _DT = (torch.bfloat16, torch.float16)
+GATE_HEADS = 64   # global_gate's most heads
 
 
 def _gpu16(*ts):
@@ -46,7 +47,7 @@ def global_gate(c, gate, r, mem_gate, mem_eps, out=None):
     ``xm = (rms_norm(r).to(dtype) * sigmoid(mem_gate.view(rows, H, d))).reshape(rows, H d)``.
     c: (B, T, H, d) view (Polar's head-major output transposed, or (1, tokens, H, d));
     gate: (rows, H, d) view; r: (rows, H, d) fp32 or c's dtype (heads contiguous) or None; mem_gate:
-    (rows, H d).  ``out`` (rows, 2 H d): both side by side there.  Returns (xa, xm or None)."""
+    (rows, H d); H at most ``GATE_HEADS``.  ``out`` (rows, 2 H d): both side by side there.  Returns (xa, xm or None)."""
     _gpu16(c, gate, mem_gate)
     B, T, H, d = c.shape
     rows = B * T

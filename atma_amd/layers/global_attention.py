@@ -55,7 +55,7 @@ from ..kernel.inference_ops import (linear_tokens, linear_tokens_supported, pack
                                      squared_relu_gate)
 from ..kernel.train_glue import (gate_train, head_norm_train, linear_train, out_train, plain_module, project_train,
                                  squared_relu_gate_train, train_glue_served)
-from ..kernel.layer_fusions import (global_gate, head_rms_norm, linear_gated, linear_gated_supported,
+from ..kernel.layer_fusions import (GATE_HEADS, global_gate, head_rms_norm, linear_gated, linear_gated_supported,
                                     memory_gate_logits, memory_gate_logits_supported, paged_kv_concat)
 from ..kernel.polar import global_decode_step_supported_shape
 from .attention import store_kvcache
@@ -262,10 +262,11 @@ class PolarAttention(nn.Module):
                 and self.head_dim in (64, 128) and self.mem is not None)
 
     def _out_fusable(self, x):
-        """The output is formed from the weights (``_fused_out``, and the memory's readout alone): ``_glue_fusable``, and
-        the modules that are then not called are what this file makes of them, without hooks."""
+        """The output is formed from the weights (``_fused_out``, and the memory's readout alone): ``_glue_fusable``, heads
+        that ``global_gate`` serves, and the modules that are then not called are what this file makes of them, without
+        hooks."""
         m = self.mem
-        return (self._glue_fusable(x) and plain_module(m, TitansMemory)
+        return (self._glue_fusable(x) and self.num_heads <= GATE_HEADS and plain_module(m, TitansMemory)
                 and all(plain_module(l, Linear) for l in (self.proj, self.mu_proj, m.proj)))
 
     def _project(self, x):
@@ -443,8 +444,8 @@ class PolarAttention(nn.Module):
         """Whether a training forward takes ``_forward_train``: shapes its launches serve, and submodules that are
         what this file makes of them, without hooks (their calls are not made there)."""
         m = self.mem
-        if m is None or x.dim() != 3 or not torch.is_grad_enabled() or not canon_supported(x, self.head_dim,
-                                                                                           self.kernel_size):
+        if m is None or x.dim() != 3 or not torch.is_grad_enabled() or self.num_heads > GATE_HEADS \
+                or not canon_supported(x, self.head_dim, self.kernel_size):
             return False
         lin = (self.q, self.k, self.v, m.gate, m.w_gamma, m.w_beta, self.proj, m.proj, self.mu_proj)
         return (plain_module(m, TitansMemory) and all(plain_module(l, Linear) for l in lin)

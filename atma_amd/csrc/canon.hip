@@ -154,7 +154,10 @@ __global__ void __launch_bounds__(256) canon_fwd_kernel(CanonArgs a) {
   float win[K][8];
   const bool first = dense && t_beg == seq_beg;
   int64_t slot = -1;
-  if (first && tails && a.slots) slot = a.slots[seq];
+  if (first && tails && a.slots) {
+    slot = a.slots[seq];
+    if (a.continuing && slot < 0) slot += a.num_slots;  // a row counted from the end, as the memory's state beside it
+  }
   if (slot >= a.num_slots) slot = -1;
   if (first) {
 #pragma unroll

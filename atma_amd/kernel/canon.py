@@ -41,7 +41,8 @@ def canon_qkv(q, k, v, weights, eps, *, seq_len=0, token_maps=None, tails=None, 
     (q as the first half of every head of the q|gate projection).  weights: the three depthwise conv weights.  Rows
     are sequences of ``seq_len``, or packed by ``token_maps`` (starts, ends, table rows; int32, one per token).
     ``tails``: the three conv state tables (rows, C, K - 1), written with each sequence's last K - 1 conv inputs in
-    row ``slots[b]`` (or the token map's); ``continuing`` reads them first as the left context.  ``caches`` (k, v)
+    row ``slots[b]`` (or the token map's); ``continuing`` reads them first as the left context, and counts negative rows
+    from the table's end as indexing does (a fresh sequence without a row, negative, keeps no tail).  ``caches`` (k, v)
     with ``slot_mapping`` int32: the k / v rows also go to the paged caches, slots < 0 skipped.
     Returns contiguous (rows, H, d), (rows, Hkv, d), (rows, Hkv, d)."""
     rows, H, d = q.shape

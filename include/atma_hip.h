@@ -682,7 +682,8 @@ int atma_lfm2_conv_packed(const void* bcx, int64_t ld, const void* weight, int64
  * within the row's sequence.  T > 0: rows / T sequences of T rows; T 0: packed rows with the token maps of
  * atma_packed_causal_conv1d.  tails (or tails[i]) non-NULL: (num_slots, heads d, K - 1), row stride tails_ss[i]; the
  * sequence's last K - 1 xn go to row slots[b] (T > 0) or the map's; continuing (T > 0): that row is read first as
- * the left context instead of zeros.  cache[i] non-NULL: out row r is also stored to row slot_mapping[r] of the
+ * the left context instead of zeros, and a negative slots[b] counts from the table's end.  Other rows outside the table
+ * are not written and read as zeros.  cache[i] non-NULL: out row r is also stored to row slot_mapping[r] of the
  * contiguous (total_slots, heads d) cache, negative and out-of-range slots skipped.  K 2..4, d 64 or 128, head-rows
  * 16-byte aligned; w_dtype is dtype or ATMA_F32.
  */

@@ -88,6 +88,9 @@ def canon_qkv(q, k, v, weights, eps, *, seq_len=0, token_maps=None, tails=None, 
         _lib.ptr(slot_mapping if caches is not None else None), total_slots, K, d, float(eps), _lib.dtype_code(wdt),
         _lib.dtype_code(q.dtype), _lib.stream_handle(dev))
     _lib.check(rc, "canon_qkv")
+    written = [t for ts_ in (tails, caches) if ts_ is not None for t in ts_]
+    if written:   # as the dispatcher does for ops that write their arguments
+        torch.autograd.graph.increment_version(written)
     return outs
 
 

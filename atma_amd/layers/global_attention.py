@@ -407,8 +407,10 @@ class PolarAttention(nn.Module):
             B, self.num_heads, self.head_dim, dtype, device))
 
     def _with_memory(self, polar_fn, mem_fn, inputs):
-        """Run the Polar part on the current stream and the memory branch (``mem_fn(signal)``)
-        in the layer's schedule; return (polar result, memory result)."""
+        """Run Polar attention (``polar_fn``) on the current stream and the memory branch (``mem_fn(signal)``) in the
+        layer's schedule; return (attention result, memory result).  ``polar_fn`` makes no library product: the memory
+        branch makes some, and products of two streams at once can be kernels whose workgroups wait for each other
+        (stream-K forms), with neither grid whole on the device."""
         if self.mem is None:
             return polar_fn(), None
         x = inputs[0]
@@ -497,19 +499,15 @@ class PolarAttention(nn.Module):
         # backward loops); otherwise the forward-only kernel
         attend = polar_attention if self._training(x, q, k, v) else polar_attention_fwd
 
-        def polar():
-            c, mag = attend(qh, kh, vh, n_keys, is_causal=True, window=self.window, **self.polar_params())
-            if fused:
-                return c, mag
-            return self._combine(c.transpose(1, 2), mag.transpose(1, 2), gate)
-
-        out, m = self._with_memory(polar, lambda signal: self._memory(x, q, k, v, fused, cache, slots, signal),
-                                   (x, q, k, v))
+        (c, mag), m = self._with_memory(
+            lambda: attend(qh, kh, vh, n_keys, is_causal=True, window=self.window, **self.polar_params()),
+            lambda signal: self._memory(x, q, k, v, fused, cache, slots, signal), (x, q, k, v))
+        c, mag = c.transpose(1, 2), mag.transpose(1, 2)
         if fused:
-            c, mag = out
-            res = self._fused_out(x.reshape(B * T, -1), c.transpose(1, 2), mag.transpose(1, 2).reshape(B * T, H),
-                                  gate.reshape(B * T, H, dk), m.reshape(B * T, H, dk))
+            res = self._fused_out(x.reshape(B * T, -1), c, mag.reshape(B * T, H), gate.reshape(B * T, H, dk),
+                                  m.reshape(B * T, H, dk))
             return res if defer else res.materialize().view(B, T, -1)
+        out = self._combine(c, mag, gate)
         return out if m is None else out + m
 
     def prefill(self, x, cache: GlobalLayerCache, slots, slot_mapping, defer=False):

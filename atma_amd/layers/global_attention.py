@@ -22,8 +22,8 @@ latency-bound with one workgroup per CU, so this pays only when its grid is smal
 quarter of the CUs or less: long sequences, small batches), and only if its workgroups
 start before Polar's fill the GPU; Polar's launch therefore waits on the recurrence's
 start signal (``StartSignal``).  ``overlap="auto"`` (default) takes the overlapped
-schedule for sequences of ``OVERLAP_TOKENS`` or more when ``recurrence_pays_to_overlap``
-says so, ``True`` always, ``False`` never.  Results agree in every schedule: bitwise where the
+schedule for sequences of ``OVERLAP_TOKENS`` or more (fp32 also ``OVERLAP_TOKENS_FP32``) when
+``recurrence_pays_to_overlap`` says so, ``True`` always, ``False`` never.  Results agree in every schedule: bitwise where the
 recurrence is not split along tokens, else to rounding.
 Training: when autograd must see the call (grad mode on and an input or parameter
 requiring grad), the full-sequence route runs the differentiable ops -- ``polar_attention``
@@ -72,8 +72,10 @@ def decode_rows(x):
             and x.is_contiguous() and not torch.is_grad_enabled())
 
 
-# overlap="auto": sequences from this length on run the memory branch beside Polar (PolarAttention._overlapped)
+# overlap="auto": sequences from this length on run the memory branch beside Polar, and in fp32, whose recurrence is not
+# split into segments, those of the second range too (PolarAttention._overlapped)
 OVERLAP_TOKENS = 8192
+OVERLAP_TOKENS_FP32 = (2304, 6000)
 
 # Polar structural priors (model/reference.py:17-20)
 LEN_GAIN_INIT = -1.0
@@ -399,11 +401,19 @@ class PolarAttention(nn.Module):
     def _overlapped(self, B, T, dtype, device, training=False):
         """Whether the memory branch runs beside Polar.  Short sequences do not (``OVERLAP_TOKENS``): their layer is
         bound by its launches, and the second stream's events cost the host about 190 us, more than the recurrence
-        it hides (2,999 tokens: 0.69 ms overlapped, 0.51 ms on one stream; 2,048 behind 12,000: 0.71 and 0.53 ms)."""
+        they hide.  Overlapped against one stream, 8 / 2 heads of 128: in bf16 one sequence of 8,192 tokens takes 0.56
+        to 0.61 against 0.46 to 0.50 ms, of 10,240 0.59 to 0.62 / 0.63, of 12,288 0.69 / 0.75; two of 6,144 0.64 / 0.58, of
+        7,168 0.61 / 0.63; a chunk of 8,192 behind 12,000 0.85 / 0.89, of 4,096 behind 12,000 0.76 / 0.49: the line lies
+        between the crossings of one sequence and of two.  In fp32 the recurrence costs more (``OVERLAP_TOKENS_FP32``):
+        2,048 tokens 0.65 / 0.57 ms, 2,304 0.67 to 0.71 / 0.72, 3,072 0.84 / 0.92, 4,096 1.06 / 1.26, 6,000 1.78 / 2.24, 8,192
+        2.54 / 2.76, 12,000 4.99 / 6.13.  Between 6,000 and 8,192 tokens nothing is measured (a run at 6,500 with both
+        schedules in turn, products of the two branches still at once, stopped answering; why is not known)."""
         if self.mem is None or self.overlap is False or device.type != "cuda" or training \
                 or torch.cuda.is_current_stream_capturing():
             return False
-        return self.overlap is True or (T >= OVERLAP_TOKENS and recurrence_pays_to_overlap(
+        lo, hi = OVERLAP_TOKENS_FP32
+        long = T >= OVERLAP_TOKENS or (dtype == torch.float32 and lo <= T <= hi)
+        return self.overlap is True or (long and recurrence_pays_to_overlap(
             B, self.num_heads, self.head_dim, dtype, device))
 
     def _with_memory(self, polar_fn, mem_fn, inputs):

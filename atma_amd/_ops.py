@@ -23,15 +23,16 @@ from . import _lib
 # of host time a call, a third of a small decode step (two sequences: 47 us dispatched)
 run = SimpleNamespace()
 _PLAIN = (Tensor, torch.nn.Parameter)
+_is_tracing, _dispatch_modes = torch._C._is_tracing, torch._C._len_torch_dispatch_stack
+_transforms, _forward_ad = torch._C._are_functorch_transforms_active, torch.autograd.forward_ad
 
 
 def watched():
     """Whether something records or transforms the calls made now: a compiler, the JIT tracer, a dispatch mode, functorch,
     forward-mode AD.  It sees torch ops and registered ops only: a launch made past them is missing from its record, whose
     replay then reads memory that nobody wrote."""
-    return (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
-            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._are_functorch_transforms_active()
-            or torch.autograd.forward_ad._current_level >= 0)
+    return (torch.compiler.is_compiling() or _is_tracing() or _dispatch_modes() > 0 or _transforms()
+            or _forward_ad._current_level >= 0)
 
 
 def _undispatched(args):

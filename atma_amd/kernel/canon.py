@@ -27,9 +27,13 @@ def canon_supported(x, head_dim, kernel_size):
 
 def _taps(weights, dtype):
     """Conv1d weights (C, 1, K) as contiguous aligned taps, all in the rows' dtype or all in fp32."""
-    ws = [w.detach() for w in weights]
-    dt = torch.float32 if all(w.dtype == torch.float32 for w in ws) else dtype
-    return [_ops._aligned16(w.to(dt)) for w in ws], dt
+    dt = torch.float32 if all(w.dtype == torch.float32 for w in weights) else dtype
+    return [w if w.dtype == dt and w.is_contiguous() and w.data_ptr() % 16 == 0 else _ops._aligned16(w.detach().to(dt))
+            for w in weights], dt
+
+
+def _layout(xs):
+    return [t.data_ptr() for t in xs], [t.stride(0) for t in xs], [t.stride(1) for t in xs]
 
 
 @torch.no_grad()
@@ -52,7 +56,10 @@ def canon_qkv(q, k, v, weights, eps, *, seq_len=0, token_maps=None, tails=None, 
     for t, h, w in zip(xs, heads, taps):
         if t.shape != (rows, h, d) or t.dtype != q.dtype or t.stride(2) != 1 or w.numel() != h * d * K:
             raise ValueError("canon_qkv: q, k, v (rows, heads, d) in one dtype and conv weights (heads d, 1, K)")
-    xs = [_ops._rows16(t) for t in xs]
+    ptrs, ldr, ldh = _layout(xs)
+    if (ptrs[0] | ptrs[1] | ptrs[2] | (ldr[0] | ldr[1] | ldr[2] | ldh[0] | ldh[1] | ldh[2]) * q.element_size()) % 16:
+        xs = [_ops._rows16(t) for t in xs]
+        ptrs, ldr, ldh = _layout(xs)
     dev = q.device
     outs = [torch.empty((rows, h, d), device=dev, dtype=q.dtype) for h in heads]
     tp, ts, num_slots = (None,) * 3, (0,) * 3, 0
@@ -81,7 +88,7 @@ def canon_qkv(q, k, v, weights, eps, *, seq_len=0, token_maps=None, tails=None, 
     if rows == 0:
         return outs
     rc = _lib.load().atma_canon_qkv(
-        _P3(*[t.data_ptr() for t in xs]), _L3(*[t.stride(0) for t in xs]), _L3(*[t.stride(1) for t in xs]), _L3(*heads),
+        _P3(*ptrs), _L3(*ldr), _L3(*ldh), _L3(*heads),
         _I3(1, 1, 0), _P3(*[w.data_ptr() for w in taps]), _P3(*[o.data_ptr() for o in outs]), _P3(*tp), _L3(*ts),
         _P3(*cp), 3, rows, 0 if token_maps is not None else int(seq_len), *[_lib.ptr(m) for m in maps],
         _lib.ptr(slots if token_maps is None else None), num_slots, 1 if continuing else 0,

@@ -18,16 +18,17 @@ _MAX = 16
 _MAX_ROWS = 65535 * 128   # gather_colsum's grid
 _P, _L, _I = ctypes.c_void_p * _MAX, ctypes.c_int64 * _MAX, ctypes.c_int32 * _MAX
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
-_HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks", "forward")
+_any_global_hook = torch.nn.modules.module._has_any_global_hook
 
 
 def plain_module(m, cls):
     """``m`` is a ``cls`` itself (no subclass, no parametrisation, no ``forward`` of its own) and nothing hooks into its
     calls, or into every module's: a fused call may stand in for it."""
-    if type(m) is not cls or torch.nn.modules.module._has_any_global_hook():
+    if type(m) is not cls:
         return False
     own = m.__dict__
-    return not any(own.get(h) for h in _HOOKS)
+    return not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
+                or "forward" in own or _any_global_hook())
 
 
 def train_glue_served(x, *params):

@@ -260,8 +260,8 @@ class PolarAttention(nn.Module):
     def _glue_fusable(self, x):
         """16-bit GPU inference with the memory branch: the per-head glue runs as the
         layer-fusion kernels (``head_rms_norm``, ``global_gate``).  Not where the call is recorded (``_ops.watched``)."""
-        return (not _ops.watched() and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and not torch.is_grad_enabled()
-                and self.head_dim in (64, 128) and self.mem is not None)
+        return (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and not torch.is_grad_enabled()
+                and self.head_dim in (64, 128) and self.mem is not None and not _ops.watched())
 
     def _out_fusable(self, x):
         """The output is formed from the weights (``_fused_out``, and the memory's readout alone): ``_glue_fusable``, heads
@@ -269,7 +269,7 @@ class PolarAttention(nn.Module):
         hooks."""
         m = self.mem
         return (self._glue_fusable(x) and self.num_heads <= GATE_HEADS and plain_module(m, TitansMemory)
-                and all(plain_module(l, Linear) for l in (self.proj, self.mu_proj, m.proj)))
+                and plain_module(self.proj, Linear) and plain_module(self.mu_proj, Linear) and plain_module(m.proj, Linear))
 
     def _project(self, x):
         """q/gate, k, v projections and per-head RMSNorm of q, k (``model/reference.py:131-139``).
@@ -456,7 +456,7 @@ class PolarAttention(nn.Module):
         """Whether a training forward takes ``_forward_train``: shapes its launches serve, and submodules that are
         what this file makes of them, without hooks (their calls are not made there)."""
         m = self.mem
-        if m is None or x.dim() != 3 or not torch.is_grad_enabled() or self.num_heads > GATE_HEADS \
+        if m is None or x.dim() != 3 or not torch.is_grad_enabled() or _ops.watched() or self.num_heads > GATE_HEADS \
                 or not canon_supported(x, self.head_dim, self.kernel_size):
             return False
         lin = (self.q, self.k, self.v, m.gate, m.w_gamma, m.w_beta, self.proj, m.proj, self.mu_proj)

@@ -1,5 +1,5 @@
-// Shared declarations of the chunked gated-delta prefill (fp32 VALU path and the
-// 16-bit MFMA path).
+// Shared declarations of the chunked gated-delta prefill (the fp32 path on v_mfma_f32_16x16x4f32 and the 16-bit path on
+// v_mfma_f32_16x16x32).
 #pragma once
 
 #include "common.h"
@@ -83,9 +83,11 @@ __device__ __forceinline__ SeqView gdn_seq(const GdnArgs& a, const VarSeqs& v, i
 
 // Segments of the 16-bit recurrence for B*H sequence-heads of NC chunks at head dim D on a device with `cus` compute
 // units; `states` = the D x D states of scratch per sequence-head.  The summaries and the replays cost the same per chunk
-// (1.4 and 1.2 us at D = 128), so a split into n takes 2 / n of the plain scan, and n is as large as keeps both on one workgroup
-// per CU, with at least 8 chunks a segment; 1 (the plain scan) below 3 segments, where nothing is gained, or when the
-// heads alone fill half of the device.  One summary of n - 1 takes two states, the first entry state one.
+// (1.4 and 1.2 us at D = 128), so a split into n takes 2 / n of the plain scan.  n has at least 8 chunks a segment, at most
+// one replay workgroup per CU and what the scratch holds: three states for each of 1 + cus / (2 per) segments (or NC / 8),
+// of which n - 1 summaries take two each and the first entry state one.  At D = 128 that is at most 50, 26, 14 and 8 segments
+// for 1, 2, 4 and 8 sequence-heads, 98, 50, 26 and 14 at D = 64.  1 (the plain scan) below 3 segments, where nothing is
+// gained, or when the plain scan's own grid is over a quarter of the device (more than 16 sequence-heads at D = 128).
 inline int gdn16_segments(int64_t BH, int64_t NC, int D, int cus, int64_t& states) {
   const int64_t per = BH * (D / 32);  // workgroups of one segment: summaries (64 of 2D columns each), replays (32 of D)
   states = 0;

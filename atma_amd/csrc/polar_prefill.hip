@@ -1558,7 +1558,10 @@ struct SplitPlan {
 
 static SplitPlan fwd_split_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t Tq, int64_t Tk, bool f32, bool causal,
                                 int64_t window) {
-  // causal 16-bit: 224 of 256 CUs, since the memory's recurrence runs beside a single prompt's attention on 32 of them
+  // causal 16-bit: 224 of the 256 CUs, the other 32 being the memory recurrence's where a caller runs the two beside each
+  // other (by itself the layer does from lengths on whose tiles stay whole at 8 heads).  Alone, 224 / 256 slots: 8 / 2 heads of 128, 2,048
+  // tokens 35 / 35 us, 2,999 45 / 53, 4,096 62 / 60, 5,000 91 / 80, 6,000 115 / 110, 8,000 171 / 169; 16 / 4 heads of 64,
+  // 2,048 36 / 37, 2,999 to 8,000 within 1%: neither is better throughout.
   const int64_t kSlots = f32 || !causal ? 256 : 224, kMinBlocks = f32 ? 4 : 8;
   const int64_t nt = (Tq + 127) / 128;
   const int64_t per = f32 ? B * Hq : B * Hq / 2;  // workgroups of a rank: a tile of one head, or of two

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("d", [64, 128])
-@pytest.mark.parametrize("T", [1024, 1536, 2500, 9000])   # 1, 3, 4 and 16 segments of 8 chunks of 64 or more, ragged
+@pytest.mark.parametrize("T", [1024, 1536, 2500, 9000])   # 1, 3, 5 and 16 (d 64) or 13 segments, ragged
 @pytest.mark.parametrize("state", [False, True])
 def test_entry_states_carry_through_segments(dev, d, T, state):
     from atma_amd.kernel import chunk_gated_delta_rule

@@ -731,7 +731,8 @@ class MLP(nn.Module):
                 w = self.proj.weight
                 parts = linear_tokens_chunks(h, [w[:, c * ck:(c + 1) * ck] for c in range(hidden // ck)], ck)
                 return PartialSums(parts, [self.proj.bias], dtype=x.dtype)
-        if x.is_cuda and not torch.is_grad_enabled() and x.is_contiguous() and self.fc.weight.dtype == x.dtype:
+        if x.is_cuda and not torch.is_grad_enabled() and x.is_contiguous() and self.fc.weight.dtype == x.dtype \
+                and not _ops.watched():
             rows, K = x.numel() // x.shape[-1], x.shape[-1]
             if linear_gated_supported(rows, K, self.fc.weight.shape[0], x.dtype):
                 # many rows (a prefill): the projection and its activation in one MFMA kernel

@@ -92,3 +92,18 @@ def test_traced_polar_reads_its_parameters(dev):
     traced = torch.jit.trace(call, tuple(p[0]), check_trace=False)
     for got, want in zip(traced(*p[1]), call(*p[1])):
         assert torch.equal(got, want)
+
+
+@torch.no_grad()
+def test_traced_mlp(dev):
+    """Rows enough for the projection and its activation as one kernel (4,096) outside a trace."""
+    from atma_amd.layers.global_attention import MLP
+    torch.manual_seed(6)
+    mlp = MLP(128).to(dev, torch.bfloat16).requires_grad_(False)
+    x, y = (torch.randn(4096, 128, generator=torch.Generator().manual_seed(s)).to(dev).bfloat16() for s in (1, 2))
+    traced = torch.jit.trace(lambda t: mlp(t), (x,), check_trace=False)
+    got = traced(y)   # (before the eager call, whose freed buffers would hold the answer)
+    with Listen():
+        want = mlp(y)
+    assert torch.equal(got, want)
+    assert rel_err(want, mlp(y)) <= BOUND[torch.bfloat16]
